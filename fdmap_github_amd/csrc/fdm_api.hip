@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -12,133 +13,17 @@
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
-#include "fdm_bulk.hpp"
+#include "fdm_stage.hpp"
 #include "../../include/fdmap_ensemble.h"
-
-namespace fdm {
-
-// mms_sin (mms.f90:52-234) on the device; same expression order as the
-// reference.  field: 0 vx,1 vy,2 sxx,3 sxy,4 syy,5 szz, 6..11 sources.
-__device__ double mms_sin(double x, double y, double t, int side, int field) {
-  const double G = 32.0, cs = 3.0, cp = 5.0;
-  double rho = G / (cs * cs);
-  double lambda = rho * (cp * cp) - 2.0 * G;
-  double Zs = rho * cs;
-  double pi = 4.0 * atan(1.0);
-  double kx = 2.0 * pi, ky = 2.0 * pi, mv = 2.0;
-  double w = (4.0 / 0.46) * pi;
-  double ft = cos(w * t);
-  double ft_t = -w * sin(w * t);
-  double mf = 0.1, kf = 1.0 * pi;
-  double ftpp = mf * kf * cos(kf * x);
-  double ftpp_x = -mf * (kf * kf) * sin(kf * x);
-  double nx = ftpp / sqrt(1.0 + ftpp * ftpp);
-  double ny = -1.0 / sqrt(1.0 + ftpp * ftpp);
-  double mx = ny, my = -nx;
-  double q = 1.0 + ftpp * ftpp;
-  double q3 = q * q * q;
-  double nx_x = ftpp_x / sqrt(q3);
-  double ny_x = ftpp * ftpp_x / sqrt(q3);
-  double mx_x = ny_x, my_x = -nx_x;
-  double nx_y = 0.0, ny_y = 0.0;
-  double mx_y = ny_y, my_y = -nx_y;
-  double sd = (double)side;
-  double amp = 2.0 * 12.6 / Zs;
-  double ckx = cos(kx * x), sky = sin(ky * y), cky = cos(ky * y), skx = sin(kx * x);
-  double vx = mv * (3.0 - 2.0 * sd) * amp * ckx * cky * ft;
-  double vx_t = mv * (3.0 - 2.0 * sd) * amp * ckx * cky * ft_t;
-  double vx_x = -mv * (3.0 - 2.0 * sd) * kx * amp * skx * cky * ft;
-  double vx_y = -mv * (3.0 - 2.0 * sd) * ky * amp * ckx * sky * ft;
-  double vy = amp * ckx * cky * ft;
-  double vy_t = amp * ckx * cky * ft_t;
-  double vy_x = -kx * amp * skx * cky * ft;
-  double vy_y = -ky * amp * ckx * sky * ft;
-  double syy = -63.0 * ckx * cky * ft - 126.0;
-  double syy_t = -63.0 * ckx * cky * ft_t;
-  double syy_x = kx * 63.0 * skx * cky * ft;
-  double syy_y = ky * 63.0 * ckx * sky * ft;
-  double sxy = 0.6 * 126.0 * ckx * cky * ft;
-  double sxy_t = 0.6 * 126.0 * ckx * cky * ft_t;
-  double sxy_x = -kx * 0.6 * 126.0 * skx * cky * ft;
-  double sxy_y = -ky * 0.6 * 126.0 * ckx * sky * ft;
-  double sxx = (2.0 * sd - 3.0) * 0.6 * 1260.0 * ckx * cky * ft;
-  double sxx_t = (2.0 * sd - 3.0) * 0.6 * 1260.0 * ckx * cky * ft_t;
-  double sxx_x = -(2.0 * sd - 3.0) * kx * 0.6 * 1260.0 * skx * cky * ft;
-  double sxx_y = -(2.0 * sd - 3.0) * ky * 0.6 * 1260.0 * ckx * sky * ft;
-  switch (field) {
-    case 5:
-      return 0.0;
-    case 0:
-      return ny * vx - my * vy;
-    case 1:
-      return mx * vy - nx * vx;
-    case 2:
-      return syy * (my * my) + sxx * (ny * ny) - 2.0 * sxy * my * ny;
-    case 4:
-      return syy * (mx * mx) + sxx * (nx * nx) - 2.0 * sxy * mx * nx;
-    case 3:
-      return -syy * my * mx - sxx * ny * nx + sxy * (ny * mx + nx * my);
-    case 6: {
-      double vxt = ny * vx_t - my * vy_t;
-      double sxxx = syy_x * (my * my) + sxx_x * (ny * ny) - 2.0 * sxy_x * my * ny +
-                    2.0 * syy * my * my_x + 2.0 * sxx * ny * ny_x -
-                    2.0 * sxy * (my_x * ny + my * ny_x);
-      double sxyy = -syy_y * my * mx - sxx_y * ny * nx + sxy_y * (ny * mx + nx * my) -
-                    syy * (my_y * mx + my * mx_y) - sxx * (ny_y * nx + ny * nx_y) +
-                    sxy * (ny_y * mx + ny * mx_y + nx_y * my + nx * my_y);
-      return vxt - (1.0 / rho) * (sxxx + sxyy);
-    }
-    case 7: {
-      double vyt = mx * vy_t - nx * vx_t;
-      double sxyx = -syy_x * my * mx - sxx_x * ny * nx + sxy_x * (ny * mx + nx * my) -
-                    syy * (my_x * mx + my * mx_x) - sxx * (ny_x * nx + ny * nx_x) +
-                    sxy * (ny_x * mx + ny * mx_x + nx_x * my + nx * my_x);
-      double syyy = syy_y * (mx * mx) + sxx_y * (nx * nx) - 2.0 * sxy_y * mx * nx +
-                    2.0 * syy * mx * mx_y + 2.0 * sxx * nx * nx_y -
-                    2.0 * sxy * (mx_y * nx + mx * nx_y);
-      return vyt - (1.0 / rho) * (sxyx + syyy);
-    }
-    case 8: {
-      double sxxt = syy_t * (my * my) + sxx_t * (ny * ny) - 2.0 * sxy_t * my * ny;
-      double vxx = ny_x * vx - my_x * vy + ny * vx_x - my * vy_x;
-      double vyy = mx_y * vy - nx_y * vx + mx * vy_y - nx * vx_y;
-      return sxxt - (lambda + 2.0 * G) * vxx - lambda * vyy;
-    }
-    case 10: {
-      double vxx = ny_x * vx - my_x * vy + ny * vx_x - my * vy_x;
-      double vyy = mx_y * vy - nx_y * vx + mx * vy_y - nx * vx_y;
-      double syyt = syy_t * (mx * mx) + sxx_t * (nx * nx) - 2.0 * sxy_t * mx * nx;
-      return syyt - lambda * vxx - (lambda + 2.0 * G) * vyy;
-    }
-    case 9: {
-      double vxy = ny_y * vx - my_y * vy + ny * vx_y - my * vy_y;
-      double vyx = mx_x * vy - nx_x * vx + mx * vy_x - nx * vx_x;
-      double sxyt = -syy_t * my * mx - sxx_t * ny * nx + sxy_t * (ny * mx + nx * my);
-      return sxyt - G * (vyx + vxy);
-    }
-    case 11: {
-      double szzt = 0.0;
-      double vxx = ny_x * vx - my_x * vy + ny * vx_x - my * vy_x;
-      double vyy = mx_y * vy - nx_y * vx + mx * vy_y - nx * vx_y;
-      return szzt - lambda * vxx - lambda * vyy;
-    }
-    default:
-      return 0.0;
-  }
-}
-
-}  // namespace fdm
 
 using namespace fdm;
 
 namespace {
 
 std::string g_create_error;
-
-// interior tile shapes (columns x rows) selectable with FDM_TILE
-const int kTileShape[3][2] = {{64, 4}, {64, 8}, {128, 4}};
 
 struct EventPair {
   hipEvent_t a, b;
@@ -206,12 +91,22 @@ struct fdm_ctx {
   // edge tasks
   int ntasks = 0;
   int2* tasks = nullptr;
+  EdgeNode* nodes = nullptr;  // the same tasks, resolved
+  // the stage launch (every context without a layer, with the tile kernels):
+  // rim groups, their nodes and points, and the inner band points
+  bool fused = false;
+  int nrim = 0, nib = 0;
+  int4* rim = nullptr;
+  EdgeNode* rimnodes = nullptr;
+  RimPt* rimpts = nullptr;
+  BandPt* ibpts = nullptr;
   // source
   fdm_source src{};
   SourcePlaceDev* dsrc = nullptr;
   // plasticity
   bool any_plastic = false;
-  bool any_mms = false;
+  bool any_mms = false;   // a block with the manufactured solution's source
+  bool mms_side = false;  // a side with its boundary data
   double* gammap = nullptr;
   double* lambda = nullptr;
   int* fail = nullptr;
@@ -263,7 +158,8 @@ struct fdm_ctx {
   int ntiles[3] = {0, 0, 0};
   int2* band = nullptr;
   int nband = 0;
-  // host copies of the tile, band and edge-task lists (ensembles merge them)
+  // host copies of the tile list (ensembles merge them), the band points and
+  // the edge tasks
   std::vector<int4> htiles[3];
   std::vector<int2> hband, htasks;
   // the latest interior launch was a lean one, which leaves DF6 unwritten at
@@ -274,25 +170,6 @@ struct fdm_ctx {
   bool graph_mode = false;
   double g_tinit = 0.0, g_dt = 0.0, g_rkc = 0.0;
   long long ninterior = 0;
-  // band split (plane strain, SBP4, uniform medium, with or without
-  // dissipation; FP64 by default): the band points on no block edge (iband) join the interior
-  // launch; the second stream's band kernel takes the edge points (eband)
-  bool band_split = false;
-  // lean plane-strain band points in a uniform medium: one lane per (point,
-  // field) (bulk_band_fl; FP64 by default, FDM_BAND_FL=0|1 overrides)
-  bool band_fl = true;
-  // antiplane band points without dissipation: one lane per (point, field)
-  // (bulk_band3_fl) when FDM_BAND_FL3=1; off by default, since it lengthened
-  // the C2-sized antiplane step (0.380 against 0.366 ms in FP64)
-  bool band_fl3 = false;
-  // plane strain in a medium or with dissipation: field lanes too
-  // (bulk_band_fl<..., EXT>): by default only in FP32-bulk in a medium
-  // without dissipation, the one case they shortened (FDM_BAND_FL_EXT
-  // overrides)
-  bool band_fl_ext = false;
-  int2* iband = nullptr;
-  int2* eband = nullptr;
-  int niband = 0, neband = 0;
   // adjoint forward passes: fault trajectories ([nstage][3][NI] per step,
   // step n at trace + (n - trace_n0) nstage 3 NI), the slot of the stage
   // being launched, and vx, vy at receivers after every step (step n at
@@ -468,8 +345,11 @@ EdgeArgs<T> edge_args(fdm_ctx* c, double t, double Bdt, double A, int do_scale, 
   a.F = (const T*)c->F[c->cur];
   a.ld = c->ld;
   a.ps = c->ps;
-  a.tasks = c->tasks;
+  a.nodes = c->nodes;
   a.ntasks = c->ntasks;
+  a.rim = c->rim;
+  a.rimnodes = c->rimnodes;
+  a.rimpts = c->rimpts;
   a.blocks = c->blocks;
   a.sd = SidesDev{c->sM, c->snormal, c->sF0, c->sx, c->sy, c->sFhat, c->NS};
   a.fi = IfacesDev{c->ifaces, c->inhat, c->irs, c->isw, c->iS0b, c->iN0b, c->ildS, c->ildN,
@@ -492,10 +372,8 @@ EdgeArgs<T> edge_args(fdm_ctx* c, double t, double Bdt, double A, int do_scale, 
 }
 
 template <typename T>
-int launch_edges(fdm_ctx* c, hipStream_t s, double t, double Bdt, double A, int do_scale,
-                 int do_update, int snapshot, double Bload) {
+int launch_edges(fdm_ctx* c, hipStream_t s, const EdgeArgs<T>& a) {
   if (c->ntasks == 0) return FDM_OK;
-  const EdgeArgs<T> a = edge_args<T>(c, t, Bdt, A, do_scale, do_update, snapshot, Bload);
   dim3 grid((c->ntasks + 63) / 64), block(64);
   EventPair* ep = prof_begin(c, 1, s);
   if (c->mode == 3 && c->any_force)
@@ -566,9 +444,9 @@ BulkArgs<T> bulk_args(fdm_ctx* c, double A, double Bdt, int do_update, double t,
   a.fxr = c->mfp[1];
   a.fyq = c->mfp[2];
   a.fyr = c->mfp[3];
-  a.ibpts = c->iband;
-  a.nib = c->niband;
-  a.nibwg = 0;  // set by the interior launch that carries them
+  a.ibpts = c->ibpts;
+  a.nib = c->nib;
+  a.nrimwg = a.nibwg = a.ib_lanes = 0;  // set by the launch that carries them
   a.rcc = nullptr;
   a.rout = nullptr;
   a.nrec = 0;
@@ -576,47 +454,29 @@ BulkArgs<T> bulk_args(fdm_ctx* c, double A, double Bdt, int do_update, double t,
   return a;
 }
 
-// the lean variants serve launches without sources, manufactured solutions
-// or a plastic update
+// the lean variants serve launches without manufactured solutions or a
+// plastic update
 template <typename T>
 bool full_variant(const fdm_ctx* c, const BulkArgs<T>& a) {
-  return c->src.nplace > 0 || c->any_mms || a.do_plastic;
+  return c->any_mms || c->mms_side || a.do_plastic;
 }
 
-template <typename T, int OP>
-void launch_band_op(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a, dim3 grid) {
-  // with the band split, the edge points only
-  const int2* pts = c->band_split ? c->eband : c->band;
-  const int n = c->band_split ? c->neband : c->nband;
-  if (c->mode == 3 && c->band_fl3 && !c->diss)
-    // one lane per (point, field), 21 points per wave
-    hipLaunchKernelGGL((bulk_band3_fl<T, OP>), dim3((n + 20) / 21), dim3(64), 0, s, a, pts, n);
-  else if (c->mode == 3)
-    hipLaunchKernelGGL((bulk_band3<T, OP>), grid, dim3(64), 0, s, a, pts, n);
-  else if (full_variant(c, a) && (c->het || c->diss))
-    hipLaunchKernelGGL((bulk_band<T, true, true, OP>), grid, dim3(64), 0, s, a, pts, n);
-  else if (full_variant(c, a))
-    hipLaunchKernelGGL((bulk_band<T, true, false, OP>), grid, dim3(64), 0, s, a, pts, n);
-  else if ((c->het || c->diss) && c->band_fl_ext)
-    hipLaunchKernelGGL((bulk_band_fl<T, OP, true>), dim3((n + 11) / 12), dim3(64), 0, s, a, pts, n);
-  else if (c->het || c->diss)
-    hipLaunchKernelGGL((bulk_band<T, false, true, OP>), grid, dim3(64), 0, s, a, pts, n);
-  else if (c->band_fl)
-    // one lane per (point, field), twelve points per wave
-    hipLaunchKernelGGL((bulk_band_fl<T, OP>), dim3((n + 11) / 12), dim3(64), 0, s, a, pts, n);
-  else
-    hipLaunchKernelGGL((bulk_band<T, false, false, OP>), grid, dim3(64), 0, s, a, pts, n);
-}
-
+// the band points of the blocks without a layer, in contexts with one
 template <typename T>
 void launch_band(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
-  const int n = c->band_split ? c->neband : c->nband;
+  const int n = c->nband;
   if (!n) return;
   EventPair* ep = prof_begin(c, 2, s);
-  dim3 grid((n + 63) / 64);
-  if (c->sbp == 2) launch_band_op<T, 2>(c, s, a, grid);
-  else if (c->sbp == 6) launch_band_op<T, 6>(c, s, a, grid);
-  else launch_band_op<T, 4>(c, s, a, grid);
+  dim3 grid((n + 63) / 64), block(64);
+  const bool ext = c->het || c->diss;
+  if (full_variant(c, a) && ext)
+    hipLaunchKernelGGL((bulk_band<T, true, true>), grid, block, 0, s, a, c->band, n);
+  else if (full_variant(c, a))
+    hipLaunchKernelGGL((bulk_band<T, true, false>), grid, block, 0, s, a, c->band, n);
+  else if (ext)
+    hipLaunchKernelGGL((bulk_band<T, false, true>), grid, block, 0, s, a, c->band, n);
+  else
+    hipLaunchKernelGGL((bulk_band<T, false, false>), grid, block, 0, s, a, c->band, n);
   prof_end(c, ep, 2, s);
 }
 
@@ -642,135 +502,67 @@ void launch_layer(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
   if (c->nlpts[1]) launch_layer_list<T, false>(c, s, a, 1);
 }
 
-template <typename T, int OP, bool HET, bool DISS>
-void launch_interior3_v(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a, dim3 grid, dim3 block) {
-  const int4* tl = c->tiles[c->tile_shape];
-  if (c->nt_store)
-    hipLaunchKernelGGL((bulk_interior3<T, 64, 4, true, OP, HET, DISS>), grid, block, 0, s, a, tl);
-  else
-    hipLaunchKernelGGL((bulk_interior3<T, 64, 4, false, OP, HET, DISS>), grid, block, 0, s, a, tl);
+// Inner band points: one lane per (point, field), or one lane per point?
+// Five lanes a point finish sooner (5 us against 12) but hold five times the
+// workgroups.  They pay while the whole launch is resident at once (`others`
+// its other workgroups); beyond that, every workgroup ahead of the tiles
+// holds a tile's place: 2 x 801x401 FP64 26.0 against 28.0 us a stage, 2 x
+// 1601x801 99.7 against 96.5 (FP32-bulk 50.6 against 47.6).
+// FDM_BAND_LANES = 0|1 overrides.
+inline int band_lanes(int nib, int others, int nt, int mode) {
+  if (const char* e = getenv("FDM_BAND_LANES")) return atoi(e) != 0;
+  const int per = (mode == 3 ? BandLanes<3>::wave : BandLanes<2>::wave) * (nt / 64);
+  return (nib + per - 1) / per + others <= 3 * 1024 * 256 / nt;
+}
+inline int band_wgs(int nib, int nt, int mode, int lanes) {
+  const int per = lanes ? (mode == 3 ? BandLanes<3>::wave : BandLanes<2>::wave) * (nt / 64) : nt;
+  return (nib + per - 1) / per;
 }
 
-template <typename T, int OP>
-void launch_interior3(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a, dim3 grid, dim3 block) {
-  if constexpr (OP == 4) {
-    if (c->diss) {
-      if (c->het) launch_interior3_v<T, OP, true, true>(c, s, a, grid, block);
-      else launch_interior3_v<T, OP, false, true>(c, s, a, grid, block);
-      return;
-    }
-  }
-  if (c->het) launch_interior3_v<T, OP, true, false>(c, s, a, grid, block);
-  else launch_interior3_v<T, OP, false, false>(c, s, a, grid, block);
-}
-
-// one interior tile variant: FULL (sources, MMS, plasticity), or lean with
-// non-temporal or normal stores
-template <typename T, int TX, int TY, bool HET, bool DISS, int OP, bool JI, bool MC = false>
-void launch_interior_v(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a, dim3 grid, dim3 block,
-                       bool full) {
-  const int4* tl = c->tiles[c->tile_shape];
-  if (full)
-    hipLaunchKernelGGL((bulk_interior<T, TX, TY, true, false, HET, DISS, OP, JI, MC>), grid, block, 0, s, a, tl);
-  else if (c->nt_store)
-    hipLaunchKernelGGL((bulk_interior<T, TX, TY, false, true, HET, DISS, OP, JI, MC>), grid, block, 0, s, a, tl);
-  else
-    hipLaunchKernelGGL((bulk_interior<T, TX, TY, false, false, HET, DISS, OP, JI, MC>), grid, block, 0, s, a, tl);
-}
-
-// the JI variants (Ji formed in the kernel) exist for FP64 only: fdm_create
-// sets ji_calc in FP64 alone; so do the MC variants (FP32-delta metrics),
-// for the 64 x 4 and 64 x 8 tiles
-template <typename T, int TX, int TY, bool HET, bool DISS, int OP>
-void launch_interior_j(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a, dim3 grid, dim3 block,
-                       bool full) {
-  if constexpr (std::is_same<T, double>::value) {
-    if constexpr (TX == 64 && (TY == 4 || TY == 8)) {
-      if (c->mcomp) {
-        if (c->ji_calc) launch_interior_v<T, TX, TY, HET, DISS, OP, true, true>(c, s, a, grid, block, full);
-        else launch_interior_v<T, TX, TY, HET, DISS, OP, false, true>(c, s, a, grid, block, full);
-        return;
-      }
-    }
-    if (c->ji_calc) {
-      launch_interior_v<T, TX, TY, HET, DISS, OP, true>(c, s, a, grid, block, full);
-      return;
-    }
-  }
-  launch_interior_v<T, TX, TY, HET, DISS, OP, false>(c, s, a, grid, block, full);
-}
-
-// the interior tiles of SBP2 or SBP6 (no dissipation): 64 x 4, or 64 x 8
-// for SBP6 in a uniform medium (tile_shape 1: its halo of 3 rows then costs
-// 6 staged rows per 8 instead of per 4, at the same occupancy)
-template <typename T, int OP, bool HET>
-void launch_interior_op(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a, dim3 grid, dim3 block,
-                        bool full) {
-  if constexpr (OP == 6 && !HET) {
-    if (c->tile_shape == 1) {
-      launch_interior_j<T, 64, 8, false, false, 6>(c, s, a, grid, block, full);
-      return;
-    }
-  }
-  launch_interior_j<T, 64, 4, HET, false, OP>(c, s, a, grid, block, full);
-}
-
+// One stage: the rim groups, receivers and inner band points ahead of the
+// interior tiles (contexts with a layer: the tiles alone).
 template <typename T>
-void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
+void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const EdgeArgs<T>& e) {
   const int q = c->tile_shape;
-  if (!c->ntiles[q]) return;
+  BulkArgs<T> a = a0;
+  const int nt = kTileShape[q][0] * kTileShape[q][1];
+  if (c->fused) {
+    a.nrimwg = c->nrim;
+    a.nrecwg = (a.nrec + nt - 1) / nt;
+    a.ib_lanes = band_lanes(c->nib, c->nrim + c->ntiles[q], nt, c->mode);
+    a.nibwg = band_wgs(c->nib, nt, c->mode, a.ib_lanes);
+  }
+  dim3 grid(a.nrimwg + a.nrecwg + a.nibwg + c->ntiles[q]);
+  dim3 block(kTileShape[q][0], kTileShape[q][1]);
+  if (!grid.x) return;
   EventPair* ep = prof_begin(c, 0, s);
   const bool full = full_variant(c, a);
-  c->df6_stale = !full;
-  dim3 grid(c->ntiles[q]);
-  dim3 block(kTileShape[q][0], kTileShape[q][1]);
+  c->df6_stale = !full && c->mode == 2;
+  // (shapes: fdm_create and fdm_tune keep 64 x 4 for antiplane shear, SBP2, a
+  // heterogeneous medium and dissipation; SBP6 in a uniform medium runs 64 x
+  // 8 by default or 64 x 4)
+  const StageLaunch L{s, grid, block, c->tiles[q], q, full, c->nt_store, c->ji_calc, c->mcomp};
   if (c->mode == 3) {
-    // antiplane shear runs the 64 x 4 tiles (fdm_create keeps tile_shape 0)
-    c->df6_stale = false;
-    if (c->sbp == 2) launch_interior3<T, 2>(c, s, a, grid, block);
-    else if (c->sbp == 6) launch_interior3<T, 6>(c, s, a, grid, block);
-    else if (c->band_split) {
-      // the inner band points ride ahead of the tiles (uniform medium, no
-      // dissipation)
-      BulkArgs<T> b = a;
-      b.nibwg = (c->niband + 255) / 256;
-      grid.x += b.nibwg;
-      launch_interior3<T, 4>(c, s, b, grid, block);
-    } else launch_interior3<T, 4>(c, s, a, grid, block);
-    prof_end(c, ep, 0, s);
-    return;
+    if (c->sbp == 2 && c->het) stage3<T, 2, true, false>(L, a, e);
+    else if (c->sbp == 2) stage3<T, 2, false, false>(L, a, e);
+    else if (c->sbp == 6 && c->het) stage3<T, 6, true, false>(L, a, e);
+    else if (c->sbp == 6) stage3<T, 6, false, false>(L, a, e);
+    else if (c->het && c->diss) stage3<T, 4, true, true>(L, a, e);
+    else if (c->diss) stage3<T, 4, false, true>(L, a, e);
+    else if (c->het) stage3<T, 4, true, false>(L, a, e);
+    else stage3<T, 4, false, false>(L, a, e);
   }
-  if (c->sbp != 4) {
-    // SBP2 and SBP6 run the 64 x 4 tiles, SBP6 in a uniform medium the
-    // 64 x 8 ones by default (fdm_create and fdm_tune keep tile_shape 0 or
-    // 1 there); neither has dissipation
-    if (c->sbp == 2) {
-      if (c->het) launch_interior_op<T, 2, true>(c, s, a, grid, block, full);
-      else launch_interior_op<T, 2, false>(c, s, a, grid, block, full);
-    } else {
-      if (c->het) launch_interior_op<T, 6, true>(c, s, a, grid, block, full);
-      else launch_interior_op<T, 6, false>(c, s, a, grid, block, full);
-    }
-    prof_end(c, ep, 0, s);
-    return;
-  }
-  // a heterogeneous medium and artificial dissipation run the 64 x 4 tiles
-  // only (fdm_create and fdm_tune keep tile_shape 0)
-  if (c->het && c->diss) launch_interior_j<T, 64, 4, true, true, 4>(c, s, a, grid, block, full);
-  else if (c->het) launch_interior_j<T, 64, 4, true, false, 4>(c, s, a, grid, block, full);
-  else {
-    // the inner band points ride ahead of the tiles (band split), one lane
-    // per point
-    BulkArgs<T> b = a;
-    const int nt = kTileShape[q][0] * kTileShape[q][1];
-    b.nibwg = c->band_split ? (c->niband + nt - 1) / nt : 0;
-    b.nrecwg = (a.nrec + nt - 1) / nt;
-    grid.x += b.nrecwg + b.nibwg;
-    if (c->diss) launch_interior_j<T, 64, 4, false, true, 4>(c, s, b, grid, block, full);
-    else if (q == 0) launch_interior_j<T, 64, 4, false, false, 4>(c, s, b, grid, block, full);
-    else if (q == 1) launch_interior_j<T, 64, 8, false, false, 4>(c, s, b, grid, block, full);
-    else launch_interior_j<T, 128, 4, false, false, 4>(c, s, b, grid, block, full);
-  }
+  else if (c->sbp == 2 && c->het) stage2<T, 2, true, false, 0>(L, a, e);
+  else if (c->sbp == 2) stage2<T, 2, false, false, 0>(L, a, e);
+  else if (c->sbp == 6 && c->het) stage2<T, 6, true, false, 0>(L, a, e);
+  else if (c->sbp == 6 && q == 1) stage2<T, 6, false, false, 1>(L, a, e);
+  else if (c->sbp == 6) stage2<T, 6, false, false, 0>(L, a, e);
+  else if (c->het && c->diss) stage2<T, 4, true, true, 0>(L, a, e);
+  else if (c->het) stage2<T, 4, true, false, 0>(L, a, e);
+  else if (c->diss) stage2<T, 4, false, true, 0>(L, a, e);
+  else if (q == 0) stage2<T, 4, false, false, 0>(L, a, e);
+  else if (q == 1) stage2<T, 4, false, false, 1>(L, a, e);
+  else stage2<T, 4, false, false, 2>(L, a, e);
   prof_end(c, ep, 0, s);
 }
 
@@ -842,48 +634,46 @@ int run_stage(fdm_ctx* c, int stage, double t0, double dt, int final_step, int s
   BulkArgs<T> a =
       bulk_args<T>(c, A, Bdt, final_step ? 0 : 1, t, srcA, (!final_step && last) ? 1 : 0, dt);
   a.skip_df = (skip_df && last && !final_step) ? 1 : 0;
-  // receivers of the previous step: in stage 1's interior launch where its
-  // kernel carries them (FP64 plane strain, SBP4, uniform medium), else a
+  // receivers of the previous step's fields (this stage's input): in the
+  // stage launch (adjoint contexts: FP64 plane strain, no layer), else a
   // launch of their own
   const bool rec_now = c->rec_out && stage == 1 && !final_step && c->cur_n > c->first_n;
-  const bool rec_fused = rec_now && std::is_same<T, double>::value && c->bulk_mode == 2 &&
-                         c->mode == 2 && c->sbp == 4 && !c->het && c->ntiles[c->tile_shape] > 0;
-  if (rec_fused) {
-    a.rcc = c->rec_cc;
-    a.rout = c->rec_out + (size_t)(c->cur_n - 1 - c->rec_n0) * c->nrec * 2;
-    a.nrec = c->nrec;
-  }
+  c->trace_cur = (c->trace && !final_step)
+                     ? c->trace + ((size_t)(c->cur_n - c->trace_n0) * c->nstage + (stage - 1)) * 3 * c->NI
+                     : nullptr;
+  const EdgeArgs<T> e = edge_args<T>(c, t, Bdt, A, 1, final_step ? 0 : 1, snapshot, Bload);
+  c->trace_cur = nullptr;
   int rc;
-  if (c->bulk_mode == 2) {
-    // Interior points need neither this stage's edge values nor this
-    // stage's band: only the band of the previous stage (halo values, and
-    // the buffer this launch overwrites is the one that band read).  The
-    // band needs this stage's edge values and the previous interior launch.
+  if (c->fused) {
+    const bool rec_fused = rec_now && std::is_same<T, double>::value && c->mode == 2;
+    if (rec_fused) {
+      a.rcc = c->rec_cc;
+      a.rout = c->rec_out + (size_t)(c->cur_n - 1 - c->rec_n0) * c->nrec * 2;
+      a.nrec = c->nrec;
+    } else if (rec_now) {
+      record_receivers(c, c->stream, c->cur_n - 1);
+    }
+    launch_interior<T>(c, c->stream, a, e);
+  } else if (c->bulk_mode == 2) {
+    // A context with a layer.  Interior points need neither this stage's
+    // edge values nor this stage's band: only the band of the previous stage
+    // (halo values, and the buffer this launch overwrites is the one that
+    // band read).  The band needs this stage's edge values and the previous
+    // interior launch.
     HIPCHK(c, hipStreamWaitEvent(c->stream, c->evB, 0));
-    launch_interior<T>(c, c->stream, a);
-    c->trace_cur = (c->trace && !final_step)
-                       ? c->trace + ((size_t)(c->cur_n - c->trace_n0) * c->nstage + (stage - 1)) * 3 * c->NI
-                       : nullptr;
-    rc = launch_edges<T>(c, c->side, t, Bdt, A, 1, final_step ? 0 : 1, snapshot, Bload);
-    c->trace_cur = nullptr;
+    launch_interior<T>(c, c->stream, a, e);
+    rc = launch_edges<T>(c, c->side, e);
     if (rc) return rc;
     HIPCHK(c, hipStreamWaitEvent(c->side, c->evI, 0));
     launch_band<T>(c, c->side, a);
     launch_layer<T>(c, c->side, a);
-    // the previous step's fields are this stage's input until stage 2
-    // writes them; both streams have finished them here
-    if (rec_now && !rec_fused) record_receivers(c, c->side, c->cur_n - 1);
     HIPCHK(c, hipEventRecord(c->evB, c->side));
     HIPCHK(c, hipEventRecord(c->evI, c->stream));
   } else {
-    c->trace_cur = (c->trace && !final_step)
-                       ? c->trace + ((size_t)(c->cur_n - c->trace_n0) * c->nstage + (stage - 1)) * 3 * c->NI
-                       : nullptr;
-    rc = launch_edges<T>(c, c->stream, t, Bdt, A, 1, final_step ? 0 : 1, snapshot, Bload);
-    c->trace_cur = nullptr;
+    rc = launch_edges<T>(c, c->stream, e);
     if (rc) return rc;
     launch_pointwise<T>(c, c->stream, a);
-    if (c->rec_out && stage == 1 && !final_step && c->cur_n > c->first_n) record_receivers(c, c->stream, c->cur_n - 1);
+    if (rec_now) record_receivers(c, c->stream, c->cur_n - 1);
   }
   HIPCHK(c, hipGetLastError());
   if (!final_step) c->cur = 1 - c->cur;
@@ -892,7 +682,7 @@ int run_stage(fdm_ctx* c, int stage, double t0, double dt, int final_step, int s
 
 template <typename T>
 int step_impl(fdm_ctx* c, double t, double dt, long long n_first, int nsteps) {
-  int rc = fork_side(c);
+  int rc = c->fused ? FDM_OK : fork_side(c);
   c->first_n = n_first;
   for (int k = 0; k < nsteps && !rc; k++) {
     long long n = n_first + k;
@@ -904,7 +694,7 @@ int step_impl(fdm_ctx* c, double t, double dt, long long n_first, int nsteps) {
     for (int stage = 1; stage <= c->nstage && !rc; stage++)
       rc = run_stage<T>(c, stage, t0, dt, 0, stage == 1, skip_df);
   }
-  int rj = join_side(c);
+  int rj = c->fused ? FDM_OK : join_side(c);
   if (!rc && !rj && c->rec_out && nsteps > 0) {
     record_receivers(c, c->stream, n_first + nsteps - 1);
     HIPCHK(c, hipGetLastError());
@@ -914,10 +704,19 @@ int step_impl(fdm_ctx* c, double t, double dt, long long n_first, int nsteps) {
 
 template <typename T>
 int stage1_impl(fdm_ctx* c, double t0, double dt) {
-  int rc = fork_side(c);
+  int rc = c->fused ? FDM_OK : fork_side(c);
   if (!rc) rc = run_stage<T>(c, 1, t0, dt, 1, 1);
-  int rj = join_side(c);
+  int rj = c->fused ? FDM_OK : join_side(c);
   return rc ? rc : rj;
+}
+
+// whether a point source's footprint holds point (i, j) of block b
+bool source_at(const fdm_ctx* c, int b, int i, int j) {
+  for (int p = 0; p < c->src.nplace; p++) {
+    const fdm_source_place& S = c->src.place[p];
+    if (S.block == b && std::abs(i - S.i0) <= 2 && std::abs(j - S.j0) <= 2) return true;
+  }
+  return false;
 }
 
 // DF6 = nu (DF3 + DF5) at the interior points of every block, in the
@@ -931,6 +730,7 @@ void restore_df6(const fdm_ctx* c, T* h) {
     for (int j = B.my + c->nbst; j <= B.py - c->nbst; j++)
       for (int i = B.mx + c->nbst; i <= B.px - c->nbst; i++) {
         const size_t k = (size_t)j * c->ld + i;
+        if (source_at(c, b, i, j)) continue;  // stored by its tile
         const T nu = c->het ? (T)c->hnu[(size_t)j * c->nx + i] : (T)B.nu;
         h[5 * pe + k] = nu * (h[2 * pe + k] + h[4 * pe + k]);
       }
@@ -1041,6 +841,165 @@ int check_fail(fdm_ctx* c) {
   HIPCHK(c, hipMemcpyAsync(&h, c->fail, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (h) return set_err(c, FDM_ENEWTON, "friction Newton solve failed (friction.f90:1012-1036)");
+  return FDM_OK;
+}
+
+}  // namespace
+
+namespace {
+
+// Work lists of the edges: the tasks resolved into EdgeNode records, and for
+// contexts without a layer the rim groups and inner band points of the stage
+// launch (see the band section of fdm_bulk.hpp).  A hat and the points it
+// enters belong to one group: tasks and points are joined where a task
+// writes a side node of the point (a corner joins its two or more tasks),
+// and whole joined sets are packed, interface nodes first (the fault solve
+// is the longest chain), until a group's first wave has no lane left for a
+// node or its other waves none for a point.
+int build_stage_lists(fdm_ctx* c) {
+  std::vector<EdgeNode> nodes(c->htasks.size());
+  // (block, side, node) -> edge point (i, j)
+  auto at = [&](int b, int s, int k) {
+    const BlockDev& B = c->hblocks[b];
+    return s < 2 ? make_int2(s == FDM_SIDE_L ? B.mx : B.px, B.my + k)
+                 : make_int2(B.mx + k, s == FDM_SIDE_B ? B.my : B.py);
+  };
+  auto cc = [&](int2 p) { return (unsigned)((long long)p.y * c->ld + p.x); };
+  struct Writes {
+    int n, blk[2], side[2], k[2];
+  };
+  std::vector<Writes> wr(c->htasks.size());
+  for (size_t t = 0; t < c->htasks.size(); t++) {
+    const int2 T = c->htasks[t];
+    EdgeNode& N = nodes[t];
+    Writes& W = wr[t];
+    if (T.x >= 0) {
+      const int b = T.x >> 2, s = T.x & 3;
+      const BlockDev& B = c->hblocks[b];
+      N = EdgeNode{-1, -1, cc(at(b, s, T.y)), 0u, B.side_off[s] + T.y, B.side_bc[s], b, B.id};
+      W = Writes{1, {b, 0}, {s, 0}, {T.y, 0}};
+    } else {
+      const IfaceDev& I = c->hifaces[-T.x - 1];
+      const BlockDev& Bm = c->hblocks[I.bm];
+      const BlockDev& Bp = c->hblocks[I.bp];
+      const int g = I.m + T.y, x = I.direction == 0;
+      const int sm = x ? FDM_SIDE_R : FDM_SIDE_T, sp = x ? FDM_SIDE_L : FDM_SIDE_B;
+      const int km = g - (x ? Bm.my : Bm.mx), kp = g - (x ? Bp.my : Bp.mx);
+      N = EdgeNode{-T.x - 1, I.node_off + T.y, cc(at(I.bm, sm, km)), cc(at(I.bp, sp, kp)),
+                   Bm.side_off[sm] + km, Bp.side_off[sp] + kp, I.bm, I.bp};
+      W = Writes{2, {I.bm, I.bp}, {sm, sp}, {km, kp}};
+    }
+  }
+  int rc;
+  if ((rc = dupload(c, &c->nodes, nodes.data(), std::max<size_t>(1, nodes.size()) * sizeof(EdgeNode)))) return rc;
+  c->fused = c->bulk_mode == 2 && !c->pml;
+  if (!c->fused) return FDM_OK;
+
+  auto band_pt = [&](int2 p) {
+    const int b = block_of(c, p.x, p.y);
+    const BlockDev& B = c->hblocks[b];
+    auto cap = [](int v) { return (unsigned)std::min(v, 255); };
+    return BandPt{p.x, p.y, b, cap(p.x - B.mx) | cap(B.px - p.x) << 8 | cap(p.y - B.my) << 16 | cap(B.py - p.y) << 24};
+  };
+  // edge points, their side nodes, and the set each belongs to
+  std::vector<BandPt> ib;
+  std::vector<RimPt> ep;
+  std::unordered_map<long long, int> id;
+  for (const int2& p : c->hband) {
+    const BandPt b = band_pt(p);
+    const BlockDev& B = c->hblocks[b.blk];
+    int so[4], n = 0;
+    if (p.x == B.mx) so[n++] = B.side_off[FDM_SIDE_L] + p.y - B.my;
+    if (p.x == B.px) so[n++] = B.side_off[FDM_SIDE_R] + p.y - B.my;
+    if (p.y == B.my) so[n++] = B.side_off[FDM_SIDE_B] + p.x - B.mx;
+    if (p.y == B.py) so[n++] = B.side_off[FDM_SIDE_T] + p.x - B.mx;
+    if (!n) {
+      ib.push_back(b);
+      continue;
+    }
+    id[(long long)p.y * c->nx + p.x] = (int)ep.size();
+    ep.push_back(RimPt{b, so[0], -1, n > 1 ? so[1] : -1, -1});
+  }
+  const int nt = (int)nodes.size(), np = (int)ep.size();
+  std::vector<int> par(nt + np);
+  for (int k = 0; k < nt + np; k++) par[k] = k;
+  auto root = [&](int k) {
+    while (par[k] != k) k = par[k] = par[par[k]];
+    return k;
+  };
+  std::vector<std::array<int, 2>> pt_of(nt, {-1, -1});
+  for (int t = 0; t < nt; t++)
+    for (int w = 0; w < wr[t].n; w++) {
+      const int2 p = at(wr[t].blk[w], wr[t].side[w], wr[t].k[w]);
+      pt_of[t][w] = id.at((long long)p.y * c->nx + p.x);
+      par[root(t)] = root(nt + pt_of[t][w]);
+    }
+  std::vector<std::vector<int>> mt(nt + np), mp(nt + np);
+  for (int t = 0; t < nt; t++) mt[root(t)].push_back(t);
+  for (int k = 0; k < np; k++) mp[root(nt + k)].push_back(k);
+  std::vector<int> order;
+  std::vector<char> seen(nt + np, 0);
+  auto visit = [&](int r) {
+    if (!seen[r]) order.push_back(r);
+    seen[r] = 1;
+  };
+  for (int t = 0; t < nt; t++)
+    if (nodes[t].iface >= 0) visit(root(t));
+  for (int t = 0; t < nt; t++) visit(root(t));
+  for (int k = 0; k < np; k++) visit(root(nt + k));
+  const int maxp = c->mode == 3 ? BandLanes<3>::group : BandLanes<2>::group;
+  static_assert(BandLanes<3>::group <= kRimPts && BandLanes<2>::group <= kRimPts, "points of a rim group");
+  std::vector<int4> groups;
+  std::vector<EdgeNode> rn;
+  std::vector<RimPt> rp;
+  std::vector<int> gt, gp;
+  bool gi = false;
+  auto has_iface = [&](const std::vector<int>& v) {
+    return std::any_of(v.begin(), v.end(), [&](int t) { return nodes[t].iface >= 0; });
+  };
+  auto flush = [&]() {
+    if (gt.empty() && gp.empty()) return;
+    const int stride = gi ? kRimIface : kRimNodes;
+    groups.push_back(make_int4((int)gt.size(), (int)gp.size(), gi ? 1 : 0, 0));
+    for (size_t q = 0; q < gt.size(); q++) {
+      const int t = gt[q];
+      rn.push_back(nodes[t]);
+      for (int w = 0; w < wr[t].n; w++) {
+        RimPt& P = ep[pt_of[t][w]];
+        const int so = w ? nodes[t].sop : nodes[t].som;
+        if (P.soA == so) P.slotA = (int)q + w * stride;
+        if (P.soB == so) P.slotB = (int)q + w * stride;
+      }
+    }
+    rn.resize(groups.size() * kRimNodes, EdgeNode{-1, 0, 0u, 0u, 0, 0, 0, 0});
+    std::stable_sort(gp.begin(), gp.end(), [&](int x, int y) { return ep[x].p.blk < ep[y].p.blk; });
+    for (int k : gp) rp.push_back(ep[k]);
+    rp.resize(groups.size() * kRimPts, RimPt{{0, 0, 0, 0u}, -1, -1, -1, -1});
+    gt.clear();
+    gp.clear();
+    gi = false;
+  };
+  for (int r : order) {
+    const bool ri = has_iface(mt[r]);
+    if (mt[r].size() > (size_t)(ri ? kRimIface : kRimNodes) || mp[r].size() > (size_t)maxp) {
+      // dozens of interfaces over the same nodes: the per-point kernels
+      c->fused = false;
+      c->bulk_mode = 0;
+      return FDM_OK;
+    }
+    const size_t most = gi || ri ? kRimIface : kRimNodes;
+    if (gt.size() + mt[r].size() > most || gp.size() + mp[r].size() > (size_t)maxp) flush();
+    gi = gi || ri;
+    gt.insert(gt.end(), mt[r].begin(), mt[r].end());
+    gp.insert(gp.end(), mp[r].begin(), mp[r].end());
+  }
+  flush();
+  c->nrim = (int)groups.size();
+  c->nib = (int)ib.size();
+  if (c->nrim && (rc = dupload(c, &c->rim, groups.data(), groups.size() * sizeof(int4)))) return rc;
+  if (!rn.empty() && (rc = dupload(c, &c->rimnodes, rn.data(), rn.size() * sizeof(EdgeNode)))) return rc;
+  if (!rp.empty() && (rc = dupload(c, &c->rimpts, rp.data(), rp.size() * sizeof(RimPt)))) return rc;
+  if (c->nib && (rc = dupload(c, &c->ibpts, ib.data(), ib.size() * sizeof(BandPt)))) return rc;
   return FDM_OK;
 }
 
@@ -1292,10 +1251,18 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
       const int ia = B.mx + nbst, ib = B.px - nbst, ja = B.my + nbst, jb = B.py - nbst;
       if (ia > ib || ja > jb) continue;
       c->ninterior += (long long)(ib - ia + 1) * (jb - ja + 1);
+      // .w: a point source's five-point footprint reaches the tile
+      auto reached = [&](int i0, int j0, int tx, int ty) {
+        for (int k = 0; k < P->source.nplace; k++) {
+          const fdm_source_place& S = P->source.place[k];
+          if (S.block == b && S.i0 + 2 >= i0 && S.i0 - 2 < i0 + tx && S.j0 + 2 >= j0 && S.j0 - 2 < j0 + ty) return 1;
+        }
+        return 0;
+      };
       for (int q = 0; q < 3; q++) {
         const int tx = kTileShape[q][0], ty = kTileShape[q][1];
         for (int j0 = ja; j0 <= jb; j0 += ty)
-          for (int i0 = ia; i0 <= ib; i0 += tx) tl[q].push_back(make_int4(b, i0, j0, 0));
+          for (int i0 = ia; i0 <= ib; i0 += tx) tl[q].push_back(make_int4(b, i0, j0, reached(i0, j0, tx, ty)));
       }
     }
     std::vector<int2> band, lpts[2];
@@ -1785,7 +1752,10 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
       c->mc_escapes = esc;
     }
   }
-  for (int b = 0; b < c->nb; b++) c->any_mms |= (P->blocks[b].mms != 0);
+  for (int b = 0; b < c->nb; b++) {
+    c->any_mms |= (P->blocks[b].mms != 0);
+    for (int s = 0; s < 4; s++) c->mms_side |= (P->blocks[b].side[s].bc == FDM_BC_MMS_SIN_W);
+  }
   bool graded = false;
   for (int b = 0; b < c->nb; b++) graded |= (c->hblocks[b].pmlx || c->hblocks[b].pmly) && c->hblocks[b].pml[0] > 0.0;
   if (c->any_mms || graded) {
@@ -1812,39 +1782,7 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     int z = 0;
     if ((rc = dupload(c, &c->fail, &z, sizeof(int)))) return fail(rc);
   }
-  // Both band forms pay off in FP64 with SBP4, where the interior launch is
-  // long enough to carry the inner band points and the field lanes shorten
-  // the second stream; in FP32-bulk (an interior launch half as long) and
-  // with SBP6 (whose field lanes took longer) the band kernel of one lane
-  // per point keeps the step shortest.
-  c->band_fl = c->precision == FDM_FP64 && c->sbp == 4;
-  if (const char* e = getenv("FDM_BAND_FL")) c->band_fl = atoi(e) != 0;
-  if (const char* e = getenv("FDM_BAND_FL3")) c->band_fl3 = atoi(e) != 0;
-  c->band_fl_ext = c->precision == FDM_FP32_BULK && c->het && !c->diss;
-  if (const char* e = getenv("FDM_BAND_FL_EXT")) c->band_fl_ext = atoi(e) != 0;
-  if (c->bulk_mode == 2 && c->sbp == 4 && !c->het && (c->mode == 2 || !c->diss) && c->nband) {
-    // band split: the band points on no block edge need no edge values of
-    // the stage and join the interior launch (bulk_interior); the second
-    // stream's band kernel takes the edge points (FDM_BAND_SPLIT=0|1
-    // overrides the default).  Antiplane shear splits only on request: its
-    // step took longer with the split (C2-size grid, 0.364 against 0.356
-    // ms in FP64, 0.239 against 0.215 in FP32-bulk).
-    bool use = c->precision == FDM_FP64 && c->mode == 2;
-    if (const char* e = getenv("FDM_BAND_SPLIT")) use = atoi(e) != 0;
-    if (use) {
-      std::vector<int2> ib, eb;
-      for (const int2& p : c->hband) {
-        const fdm_block& B = P->blocks[block_of(c, p.x, p.y)];
-        const bool edge = p.x == B.mx || p.x == B.px || p.y == B.my || p.y == B.py;
-        (edge ? eb : ib).push_back(p);
-      }
-      c->niband = (int)ib.size();
-      c->neband = (int)eb.size();
-      if (c->niband && (rc = dupload(c, &c->iband, ib.data(), ib.size() * sizeof(int2)))) return fail(rc);
-      if (c->neband && (rc = dupload(c, &c->eband, eb.data(), eb.size() * sizeof(int2)))) return fail(rc);
-      c->band_split = true;
-    }
-  }
+  if ((rc = build_stage_lists(c))) return fail(rc);
   {
     // frictional nodes and the reduction buffer of fdm_max_slip_velocity
     std::vector<int> fn;
@@ -2011,8 +1949,9 @@ int fdm_init_edges(fdm_ctx* c, double t) {
   if (!c) return FDM_EINVAL;
   // prepare_edges + enforce_edge_conditions(D,0d0) (domain.f90:346-356)
   double Bload = c->ld_T.empty() ? 1.0 : load_ramp(t, c->ld_T[0]);
-  int rc = c->precision == FDM_FP64 ? launch_edges<double>(c, c->stream, t, 0.0, 1.0, 0, 0, 0, Bload)
-                                    : launch_edges<float>(c, c->stream, t, 0.0, 1.0, 0, 0, 0, Bload);
+  int rc = c->precision == FDM_FP64
+               ? launch_edges<double>(c, c->stream, edge_args<double>(c, t, 0.0, 1.0, 0, 0, 0, Bload))
+               : launch_edges<float>(c, c->stream, edge_args<float>(c, t, 0.0, 1.0, 0, 0, 0, Bload));
   if (rc) return rc;
   return check_fail(c);
 }
@@ -2192,10 +2131,10 @@ int fdm_profile_read(fdm_ctx* c, fdm_profile_t* out) {
   out->edge_launches = c->kind_n[1];
   out->band_ms = c->kind_ms[2];
   out->band_launches = c->kind_n[2];
-  // the interior launch's points: tiles, inner layer points and, with the
-  // band split, the inner band points
-  out->bulk_points = c->bulk_mode == 2 ? (int64_t)c->ninterior + c->nlayer_inner + c->niband
-                                       : (int64_t)c->nx * c->ny;
+  // the points of one stage launch (all of them), in contexts with a layer
+  // the tiles' and the inner layer's
+  out->bulk_points = c->fused || c->bulk_mode != 2 ? (int64_t)c->nx * c->ny
+                                                   : (int64_t)c->ninterior + c->nlayer_inner;
   return FDM_OK;
 }
 
@@ -2230,28 +2169,25 @@ int fdm_tune(fdm_ctx* c, int32_t knob, int32_t value) {
 }  // extern "C"
 
 // An ensemble steps many contexts with batched launches: every RK stage is
-// one interior launch per tile shape in use, one edge launch and one band
-// launch over the merged work lists of all members, with the two-stream
-// ordering of a single context.  The per-member kernel arguments of each
+// one launch per tile shape in use over the merged work lists of all
+// members.  The per-member kernel arguments of each
 // (buffer parity, stage) sit in device tables; stage times come from one
 // device step counter.  A step is captured once per starting buffer parity
 // as a hipGraph (FDM_ENSEMBLE_GRAPH=0 launches the same kernels directly).
 struct fdm_ensemble {
   std::vector<fdm_ctx*> m;
-  int precision = FDM_FP64, nstage = 0, flip = 0, swz = 1;
-  bool any_plastic = false, use_graph = true, nt_store = false, any_force = false;
-  hipStream_t master = nullptr, side = nullptr;
-  hipEvent_t evJ = nullptr, evI = nullptr, evB = nullptr, done = nullptr;
+  int precision = FDM_FP64, nstage = 0, flip = 0, swz = 1, ib_lanes = 0;
+  bool any_plastic = false, mms_side = false, use_graph = true, nt_store = false;
+  hipStream_t master = nullptr;
+  hipEvent_t done = nullptr;
   std::vector<hipEvent_t> pre;  // each member's earlier work, before a step
-  // merged lists: tiles (block, i0, j0, member) per tile shape; band points
-  // (i, j, member, valid) and edge tasks (x, y, member, valid), each member's
-  // run padded to whole waves so that a wave serves one member
+  // merged lists per tile shape in use: tiles (block, i0, j0, member), and
+  // the workgroups ahead of them (member, its workgroup index): every rim
+  // group, then every inner band workgroup
   int4* tiles[3] = {nullptr, nullptr, nullptr};
   int ntiles[3] = {0, 0, 0};
-  int4* band = nullptr;
-  int nband = 0;
-  int4* tasks = nullptr;
-  int ntasks = 0;
+  int2* ahead[3] = {nullptr, nullptr, nullptr};
+  int nahead[3] = {0, 0, 0};
   void* btab = nullptr;  // BulkArgs<T>[2][nstage][members]
   void* etab = nullptr;  // EdgeArgs<T>[2][nstage][members]
   long long* nstep = nullptr;
@@ -2306,6 +2242,8 @@ int ens_tables(fdm_ensemble* e) {
         const int saved = c->cur;
         c->cur = cs;
         bt[o] = bulk_args<T>(c, A, Bdt, 1, ts, 0.0, s == ns ? 1 : 0, e->dt[k]);
+        bt[o].nrimwg = c->nrim;
+        bt[o].ib_lanes = e->ib_lanes;
         et[o] = edge_args<T>(c, ts, Bdt, A, 1, 1, s == 1 ? 1 : 0, 1.0);
         c->cur = saved;
         et[o].nstep = e->nstep;
@@ -2324,60 +2262,24 @@ int ens_tables(fdm_ensemble* e) {
   return FDM_OK;
 }
 
-template <typename T, bool FULL, bool NT>
-void ens_interior(fdm_ensemble* e, const BulkArgs<T>* tab) {
-  for (int q = 0; q < 3; q++) {
-    if (!e->ntiles[q]) continue;
-    const dim3 grid(e->ntiles[q]), block(kTileShape[q][0], kTileShape[q][1]);
-    if (q == 0)
-      hipLaunchKernelGGL((bulk_interior_batch<T, 64, 4, FULL, NT>), grid, block, 0, e->master, tab, e->tiles[q], e->swz);
-    else if (q == 1)
-      hipLaunchKernelGGL((bulk_interior_batch<T, 64, 8, FULL, NT>), grid, block, 0, e->master, tab, e->tiles[q], e->swz);
-    else
-      hipLaunchKernelGGL((bulk_interior_batch<T, 128, 4, FULL, NT>), grid, block, 0, e->master, tab, e->tiles[q], e->swz);
-  }
-}
-
-// One RK step of every member from buffer parity p: the stream DAG of
-// run_stage (interior on the master stream, edge and band on the side
-// stream), then the step counter.
+// One RK step of every member from buffer parity p: a stage launch per tile
+// shape in use, then the step counter.
 template <typename T>
 int ens_step_launches(fdm_ensemble* e, int p) {
   const size_t M = e->m.size(), ns = e->nstage;
-  ENSCHK(e, hipEventRecord(e->evJ, e->master));
-  ENSCHK(e, hipStreamWaitEvent(e->side, e->evJ, 0));
-  ENSCHK(e, hipEventRecord(e->evB, e->side));
-  ENSCHK(e, hipEventRecord(e->evI, e->master));
   for (size_t s = 1; s <= ns; s++) {
     const size_t o = ((size_t)p * ns + (s - 1)) * M;
     const BulkArgs<T>* bt = (const BulkArgs<T>*)e->btab + o;
     const EdgeArgs<T>* et = (const EdgeArgs<T>*)e->etab + o;
-    const bool full = e->any_plastic && s == ns;
-    ENSCHK(e, hipStreamWaitEvent(e->master, e->evB, 0));
-    if (full) ens_interior<T, true, false>(e, bt);
-    else if (e->nt_store) ens_interior<T, false, true>(e, bt);
-    else ens_interior<T, false, false>(e, bt);
-    if (e->ntasks && e->any_force)
-      hipLaunchKernelGGL((edge_kernel_batch<T, true>), dim3(e->ntasks / 64), dim3(64), 0, e->side, et,
-                         e->tasks, e->ntasks);
-    else if (e->ntasks)
-      hipLaunchKernelGGL((edge_kernel_batch<T, false>), dim3(e->ntasks / 64), dim3(64), 0, e->side, et,
-                         e->tasks, e->ntasks);
-    ENSCHK(e, hipStreamWaitEvent(e->side, e->evI, 0));
-    if (e->nband) {
-      if (full)
-        hipLaunchKernelGGL((bulk_band_batch<T, true>), dim3(e->nband / 64), dim3(64), 0, e->side, bt, e->band,
-                           e->nband);
-      else
-        hipLaunchKernelGGL((bulk_band_batch<T, false>), dim3(e->nband / 64), dim3(64), 0, e->side, bt,
-                           e->band, e->nband);
+    const bool full = e->mms_side || (e->any_plastic && s == ns);
+    for (int q = 0; q < 3; q++) {
+      const dim3 grid(e->nahead[q] + e->ntiles[q]), block(kTileShape[q][0], kTileShape[q][1]);
+      if (grid.x)
+        stage_batch<T>(StageLaunch{e->master, grid, block, e->tiles[q], q, full, e->nt_store, false, false}, bt, et,
+                       e->ahead[q], e->nahead[q], e->swz);
     }
-    ENSCHK(e, hipEventRecord(e->evB, e->side));
-    ENSCHK(e, hipEventRecord(e->evI, e->master));
   }
-  hipLaunchKernelGGL(step_counter_kernel, dim3(1), dim3(64), 0, e->side, e->nstep);
-  ENSCHK(e, hipEventRecord(e->evB, e->side));
-  ENSCHK(e, hipStreamWaitEvent(e->master, e->evB, 0));
+  hipLaunchKernelGGL(step_counter_kernel, dim3(1), dim3(64), 0, e->master, e->nstep);
   ENSCHK(e, hipGetLastError());
   return FDM_OK;
 }
@@ -2405,24 +2307,30 @@ int ens_capture(fdm_ensemble* e, int p) {
 // merged work lists of all members
 int ens_lists(fdm_ensemble* e) {
   const int M = (int)e->m.size();
-  std::vector<int4> tl[3], band, tasks;
+  std::vector<int4> tl[3];
+  std::vector<int2> ah[3];
+  int nib = 0, others = 0;
+  for (const fdm_ctx* c : e->m) {
+    nib += c->nib;
+    others += c->nrim + c->ntiles[c->tile_shape];
+  }
+  e->ib_lanes = band_lanes(nib, others, 256, 2);
+  for (int k = 0; k < M; k++)
+    for (int w = 0; w < e->m[k]->nrim; w++) ah[e->m[k]->tile_shape].push_back(make_int2(k, w));
   for (int k = 0; k < M; k++) {
     const fdm_ctx* c = e->m[k];
-    for (const int4& t : c->htiles[c->tile_shape]) tl[c->tile_shape].push_back(make_int4(t.x, t.y, t.z, k));
-    for (const int2& b : c->hband) band.push_back(make_int4(b.x, b.y, k, 1));
-    while (band.size() % 64) band.push_back(make_int4(0, 0, k, 0));
-    for (const int2& t : c->htasks) tasks.push_back(make_int4(t.x, t.y, k, 1));
-    while (tasks.size() % 64) tasks.push_back(make_int4(0, 0, k, 0));
+    const int q = c->tile_shape, nt = kTileShape[q][0] * kTileShape[q][1];
+    for (int w = 0; w < band_wgs(c->nib, nt, 2, e->ib_lanes); w++) ah[q].push_back(make_int2(k, c->nrim + w));
+    for (const int4& t : c->htiles[q]) tl[q].push_back(make_int4(t.x, t.y, t.z, k));
   }
   for (int q = 0; q < 3; q++) {
     e->ntiles[q] = (int)tl[q].size();
     if (e->ntiles[q] && ens_upload(e, &e->tiles[q], tl[q].data(), tl[q].size() * sizeof(int4)))
       return FDM_EDEVICE;
+    e->nahead[q] = (int)ah[q].size();
+    if (e->nahead[q] && ens_upload(e, &e->ahead[q], ah[q].data(), ah[q].size() * sizeof(int2)))
+      return FDM_EDEVICE;
   }
-  e->nband = (int)band.size();
-  if (e->nband && ens_upload(e, &e->band, band.data(), band.size() * sizeof(int4))) return FDM_EDEVICE;
-  e->ntasks = (int)tasks.size();
-  if (e->ntasks && ens_upload(e, &e->tasks, tasks.data(), tasks.size() * sizeof(int4))) return FDM_EDEVICE;
   return FDM_OK;
 }
 
@@ -2435,16 +2343,13 @@ const char* fdm_ensemble_last_error(const fdm_ensemble* e) { return e ? e->err.c
 void fdm_ensemble_destroy(fdm_ensemble* e) {
   if (!e) return;
   if (e->master) (void)hipStreamSynchronize(e->master);
-  if (e->side) (void)hipStreamSynchronize(e->side);
   for (int q = 0; q < 2; q++)
     if (e->exec[q]) (void)hipGraphExecDestroy(e->exec[q]);
   for (hipEvent_t ev : e->pre)
     if (ev) (void)hipEventDestroy(ev);
-  for (hipEvent_t ev : {e->evJ, e->evI, e->evB, e->done})
-    if (ev) (void)hipEventDestroy(ev);
+  if (e->done) (void)hipEventDestroy(e->done);
   for (void* p : e->allocs) (void)hipFree(p);
   if (e->master) (void)hipStreamDestroy(e->master);
-  if (e->side) (void)hipStreamDestroy(e->side);
   delete e;
 }
 
@@ -2483,16 +2388,14 @@ int fdm_ensemble_create(fdm_ctx* const* members, int32_t n, fdm_ensemble** out) 
   double ws = 0.0;
   for (fdm_ctx* c : e->m) {
     e->any_plastic = e->any_plastic || c->any_plastic;
-    e->any_force = e->any_force || c->any_force;
+    e->mms_side = e->mms_side || c->mms_side;
     ws += 23.0 * (double)c->ps * (double)c->esz;
   }
   e->nt_store = nt_store_choice(ws);
   if (const char* v = getenv("FDM_ENSEMBLE_GRAPH")) e->use_graph = atoi(v) != 0;
   e->pre.resize(n, nullptr);
   bool ok = hipStreamCreateWithFlags(&e->master, hipStreamNonBlocking) == hipSuccess &&
-            hipStreamCreateWithFlags(&e->side, hipStreamNonBlocking) == hipSuccess;
-  for (hipEvent_t* ev : {&e->evJ, &e->evI, &e->evB, &e->done})
-    ok = ok && hipEventCreateWithFlags(ev, hipEventDisableTiming) == hipSuccess;
+            hipEventCreateWithFlags(&e->done, hipEventDisableTiming) == hipSuccess;
   for (int k = 0; k < n && ok; k++) ok = hipEventCreateWithFlags(&e->pre[k], hipEventDisableTiming) == hipSuccess;
   int rc = ok ? FDM_OK : FDM_EDEVICE;
   if (!rc) rc = ens_lists(e);
@@ -2556,7 +2459,7 @@ int fdm_ensemble_step(fdm_ensemble* e, const double* t, const double* dt, int64_
   // interior points of a lean last-stage launch hold no DF6 (recomputed on
   // read); the full one (any plastic member) stores it, plastic corrections
   // included.  Members' own streams follow the ensemble's work.
-  for (fdm_ctx* c : e->m) c->df6_stale = !e->any_plastic;
+  for (fdm_ctx* c : e->m) c->df6_stale = !e->any_plastic && !e->mms_side;
   ENSCHK(e, hipEventRecord(e->done, e->master));
   for (fdm_ctx* c : e->m) ENSCHK(e, hipStreamWaitEvent(c->stream, e->done, 0));
   return FDM_OK;

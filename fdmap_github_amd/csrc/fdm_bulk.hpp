@@ -9,6 +9,22 @@
 
 namespace fdm {
 
+// A band point (within the closure depth of its block's edge): its index,
+// block and distances from the block's L, R, B, T sides (capped at 255, a
+// byte each).
+struct BandPt {
+  int i, j, blk;
+  unsigned d;
+};
+
+// A band point on its block's edge: up to two sides meet there (in the order
+// L, R, B, T); side node and hat slot of each (so < 0: no such side; slot <
+// 0: no task of the stage writes the hat).
+struct RimPt {
+  BandPt p;
+  int soA, slotA, soB, slotB;
+};
+
 template <typename T>
 struct BulkArgs {
   const T* Fin;
@@ -68,10 +84,13 @@ struct BulkArgs {
   const float* fyq;
   const float* fyr;
   // inner band points: the band points on no block edge (they need no edge
-  // values of the stage), updated by the first nibwg workgroups of the
-  // interior launch, one lane per point (nib points; none: nibwg = 0)
-  const int2* ibpts;
-  int nib, nibwg;
+  // values of the stage), nib of them, updated by nibwg workgroups of the
+  // stage launch ahead of its tiles: one lane per (point, field) with
+  // ib_lanes, else one lane per point
+  const BandPt* ibpts;
+  int nib, nibwg, ib_lanes;
+  // rim groups: the first nrimwg workgroups of the stage launch (fdm_rim.hpp)
+  int nrimwg;
   // receivers: vx, vy of Fin at the nrec points rcc into rout (FP64
   // plane-strain contexts), by nrecwg workgroups ahead of the inner band
   // points in stage 1 of a step; none: nrecwg = 0
@@ -337,14 +356,9 @@ struct GlobalAcc {
   __device__ __forceinline__ T yq(int dj) const { return pyq[cc + (long long)dj * ld]; }
 };
 
+// SAT penalty of the hat Fh (as stored) at a side node
 template <typename T>
-__device__ __forceinline__ void sat_term(T* d, const T* Fe, const SidesDev& sd, int so) {
-  const int NS = sd.NS;
-  double Fh[6];
-#pragma unroll
-  for (int l = 0; l < 6; l++) Fh[l] = sd.Fhat[l * NS + so];
-  T n1 = (T)sd.normal[so], n2 = (T)sd.normal[NS + so];
-  T Ks = (T)sd.M[3 * NS + so], Kp = (T)sd.M[4 * NS + so];
+__device__ __forceinline__ void sat_hat(T* d, const T* Fe, const double (&Fh)[6], T n1, T n2, T Ks, T Kp) {
   T dd[6];
 #pragma unroll
   for (int l = 0; l < 6; l++) dd[l] = (T)Fh[l] - Fe[l];
@@ -374,6 +388,16 @@ __device__ __forceinline__ void sat_term(T* d, const T* Fe, const SidesDev& sd, 
   for (int l = 0; l < 6; l++) d[l] = d[l] + Ks * Fs[l];
 #pragma unroll
   for (int l = 0; l < 6; l++) d[l] = d[l] + Kp * Fp[l];
+}
+
+// the same from the side arrays
+template <typename T>
+__device__ __forceinline__ void sat_term(T* d, const T* Fe, const SidesDev& sd, int so) {
+  const int NS = sd.NS;
+  double Fh[6];
+#pragma unroll
+  for (int l = 0; l < 6; l++) Fh[l] = sd.Fhat[l * NS + so];
+  sat_hat<T>(d, Fe, Fh, (T)sd.normal[so], (T)sd.normal[NS + so], (T)sd.M[3 * NS + so], (T)sd.M[4 * NS + so]);
 }
 
 // plastic_flow (plastic.f90:62-192) in FP64
@@ -427,12 +451,31 @@ __device__ __forceinline__ void plastic_point(double G, double K, double mu, dou
   Ds[3] = Ds[3] - lam * W[5];
 }
 
+// singular source (source.f90:196-254): the places whose five-point
+// footprint holds the point
+template <typename T>
+__device__ __forceinline__ void point_sources(const BulkArgs<T>& a, const double rho, const int bi, const int i,
+                                              const int j, T (&d)[6]) {
+  for (int p = 0; p < a.nplace; p++) {
+    const SourcePlaceDev& P = a.src[p];
+    int di = i - P.i0 + 2, dj = j - P.j0 + 2;
+    if (P.block == bi && di >= 0 && di <= 4 && dj >= 0 && dj <= 4) {
+      double dx = P.dx[di], dy = P.dy[dj];
+      d[0] = d[0] + (T)(a.srcA * a.Fx * dx * dy / rho);
+      d[1] = d[1] + (T)(a.srcA * a.Fy * dx * dy / rho);
+      d[2] = d[2] - (T)(a.srcA * a.Mxx * dx * dy);
+      d[3] = d[3] - (T)(a.srcA * a.Mxy * dx * dy);
+      d[4] = d[4] - (T)(a.srcA * a.Myy * dx * dy);
+    }
+  }
+}
+
 // szz overwrite, sources, RK update, plasticity and stores of one point
 // (rates.f90:920-936, source.f90:196-296, fields.f90:1225-1242,
 // plastic.f90:8-59).  Fc: the point's fields at the start of the stage.
-// FULL = false leaves out the singular source, the manufactured-solution
-// source and plasticity; the host selects it for launches that need none of
-// them.  NTS stores F and DF non-temporally.
+// FULL = false leaves out the manufactured-solution source and plasticity;
+// the host selects it for launches that need neither.  NTS stores F and DF
+// non-temporally.
 template <typename T, bool FULL, bool NTS = false>
 __device__ __forceinline__ void finish_point(const BulkArgs<T>& a, const BlockDev& B, const int bi,
                                              const int i, const int j, const long long cc,
@@ -441,19 +484,7 @@ __device__ __forceinline__ void finish_point(const BulkArgs<T>& a, const BlockDe
   // rates_szz (rates.f90:920-936): overwrite
   // (rates_h_szz, rates_heterogeneous.f90:901-917: the point's nu)
   d[5] = (a.mnu ? a.mnu[cc] : (T)B.nu) * (d[2] + d[4]);
-  // singular source (source.f90:196-254)
-  if constexpr (FULL) for (int p = 0; p < a.nplace; p++) {
-    const SourcePlaceDev& P = a.src[p];
-    int di = i - P.i0 + 2, dj = j - P.j0 + 2;
-    if (P.block == bi && di >= 0 && di <= 4 && dj >= 0 && dj <= 4) {
-      double dx = P.dx[di], dy = P.dy[dj];
-      d[0] = d[0] + (T)(a.srcA * a.Fx * dx * dy / B.rho);
-      d[1] = d[1] + (T)(a.srcA * a.Fy * dx * dy / B.rho);
-      d[2] = d[2] - (T)(a.srcA * a.Mxx * dx * dy);
-      d[3] = d[3] - (T)(a.srcA * a.Mxy * dx * dy);
-      d[4] = d[4] - (T)(a.srcA * a.Myy * dx * dy);
-    }
-  }
+  point_sources<T>(a, B.rho, bi, i, j, d);
   // manufactured-solution source (source.f90:256-269)
   if (FULL && B.mms) {
     double x = a.X[(long long)j * a.nx + i], y = a.Y[(long long)j * a.nx + i];
@@ -876,9 +907,15 @@ __device__ __forceinline__ void scaled_rates(const BulkArgs<T>& a, const long lo
 // neighbours straight from global memory: the per-point kernel, and the
 // closure points of the tile and marching kernels.  EXT as in closure_rates,
 // and also carries the perfectly matched layer.
-template <typename T, bool FULL, bool EXT, int OP = 4>
-__device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i, const int j) {
-  const int bi = a.blk[a.rowb[j] * a.nbx + a.colb[i]];
+template <typename T>
+__device__ __forceinline__ int block_at(const BulkArgs<T>& a, const int i, const int j) {
+  return a.blk[a.rowb[j] * a.nbx + a.colb[i]];
+}
+
+// PML = false leaves the layer out (contexts without one), INNER = true the
+// closures (interior points only).
+template <typename T, bool FULL, bool EXT, int OP = 4, bool PML = EXT, bool INNER = false>
+__device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i, const int j, const int bi) {
   const BlockDev& B = a.blocks[bi];
   const long long ps = a.ps;
   const int ld = a.ld;
@@ -890,7 +927,7 @@ __device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i,
   if constexpr (OP == 4) {
     // the perfectly matched layer and artificial dissipation are built for
     // SBP4 only (fdm_create refuses them with the other operators)
-    if (EXT && (B.pmlx | B.pmly)) {
+    if (PML && (B.pmlx | B.pmly)) {
       pml_rates<T>(a, B, i, j, cc, d);
       done = true;
     } else if (EXT && B.Cdiss > 0.0 && i - B.mx >= 4 && B.px - i >= 4 && j - B.my >= 4 &&
@@ -906,7 +943,7 @@ __device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i,
     }
   }
   if (done) {
-  } else if (i - B.mx >= NB && B.px - i >= NB && j - B.my >= NB && B.py - j >= NB) {
+  } else if (INNER || (i - B.mx >= NB && B.px - i >= NB && j - B.my >= NB && B.py - j >= NB)) {
     const GlobalAcc<T> acc{a.Fin, a.xq, a.xr, a.yq, a.yr, ps, cc, ld, a.J};
     if (EXT && a.mrho) {
       interior_rates<T, GlobalAcc<T>, PointCoef<T, OP>, HW>(
@@ -915,7 +952,7 @@ __device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i,
       interior_rates<T, GlobalAcc<T>, BlockCoef<T, const BlockDev&>, HW>(
           d, acc, (T)B.gamma, BlockCoef<T, const BlockDev&>{B}, a.Ji[cc]);
     }
-  } else {
+  } else if constexpr (!INNER) {
     closure_rates<T, EXT, OP>(a, B, i, j, cc, d);
   }
   T Fc[6];
@@ -932,7 +969,7 @@ __global__ void __launch_bounds__(256) bulk_kernel(BulkArgs<T> a) {
   const int i = tx * blockDim.x + threadIdx.x;
   const int j = ty * blockDim.y + threadIdx.y;
   if (i >= a.nx || j >= a.ny) return;
-  point_generic<T, true, true, OP>(a, i, j);
+  point_generic<T, true, true, OP>(a, i, j, block_at(a, i, j));
 }
 
 // global load at a 32-bit byte offset from a wave-uniform base, so that the
@@ -1007,14 +1044,33 @@ typedef const __attribute__((address_space(4))) BlockDev ConstBlockDev;
 // F1..F5 with a halo of two points in q and r, xr/yr with the q halo and
 // xq/yq with the r halo go to LDS; the lane's own DF, F6 and Ji stay in
 // registers.  Halo indices are clamped into the grid; a clamped value never
-// reaches an active lane.  tiles[k] = (block, i0, j0, 0).
+// reaches an active lane.  tiles[k] = (block, i0, j0, a point source reaches it).
 // JI: form Ji from the staged metrics (a context with ji_calc set) rather
 // than read it; a compile-time switch, so that neither path holds the other's
 // registers.  MC: read xq, xr, yq, yr as FP32 deltas from their block's base
 // (FP64 only; the values staged in LDS are the FP64 metrics to the bit).
+// LDS bytes of an interior tile with NF staged fields, and of a launch whose
+// rim workgroups use the same buffer for their hats
+template <typename T, int TX, int TY, bool DISS, int OP, int NF>
+constexpr int tile_bytes() {
+  constexpr int H = Sbp<OP>::half, HX = TX + 2 * H, HY = TY + 2 * H;
+  return (int)sizeof(T) * ((NF + (DISS ? 1 : 0)) * HY * HX + 2 * TY * HX + 2 * HY * TX);
+}
+// where EdgeArgs follow BulkArgs in a stage kernel's argument segment
+template <typename T>
+constexpr int edge_args_at() {
+  return (sizeof(BulkArgs<T>) + alignof(EdgeArgs<T>) - 1) / alignof(EdgeArgs<T>) * alignof(EdgeArgs<T>);
+}
+
+// a rim group's LDS: the staged rows of its nodes, then their hats
+constexpr int kRimRowsMax =
+    kNodeRowsBnd * kRimNodes > kNodeRows * kRimIface ? kNodeRowsBnd * kRimNodes : kNodeRows * kRimIface;
+constexpr int kRimHats = 2 * kRimIface > kRimNodes ? 2 * kRimIface : kRimNodes;
+constexpr int kRimBytes = (kRimRowsMax + 6 * kRimHats) * (int)sizeof(double);
+
 template <typename T, int TX, int TY, bool FULL, bool NTS, bool HET, bool DISS, int OP = 4,
           bool JI = false, bool MC = false>
-__device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 td) {
+__device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 td, char* smem) {
   // H: the operator's interior half-width, the tile's halo; NB: the
   // closure's depth, how far the interior rectangle stays from block edges
   constexpr int H = Sbp<OP>::half, NB = Sbp<OP>::nbst;
@@ -1024,11 +1080,11 @@ __device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 t
   constexpr int NF = (HY * HX + NT - 1) / NT;  // staging passes, F1..F5
   constexpr int NR = (TY * HX + NT - 1) / NT;  // xr, yr
   constexpr int NQ = (HY * TX + NT - 1) / NT;  // xq, yq
-  __shared__ T sF[5][HY][HX];
-  __shared__ T sR[2][TY][HX];
-  __shared__ T sQ[2][HY][TX];
+  T (*sF)[HY][HX] = reinterpret_cast<T (*)[HY][HX]>(smem);
+  T (*sR)[TY][HX] = reinterpret_cast<T (*)[TY][HX]>(smem + 5 * HY * HX * sizeof(T));
+  T (*sQ)[HY][TX] = reinterpret_cast<T (*)[HY][TX]>(smem + (5 * HY + 2 * TY) * HX * sizeof(T));
   // the Jacobian with the same halo as F, for artificial dissipation
-  __shared__ T sJ[DISS ? HY : 1][DISS ? HX : 1];
+  T (*sJ)[HX] = reinterpret_cast<T (*)[HX]>(smem + ((5 * HY + 2 * TY) * HX + 2 * HY * TX) * sizeof(T));
   const int bu = td.x, i0 = td.y, j0 = td.z;
   ConstBlockDev* B4 = (ConstBlockDev*)a.blocks + bu;
   const int tid = threadIdx.y * TX + threadIdx.x;
@@ -1244,199 +1300,599 @@ __device__ __forceinline__ T bscale_rt(T t, T D, T rho, T G, T M, int mat) {
   return mat == 0 ? td / rho : (mat == 1 ? td * G : td * M);
 }
 
-// Band kernel with one lane per (point, field) for plane strain in a
-// uniform medium without dissipation, lean stages (no sources, MMS or
-// plastic update).  Twelve points share a wave, five lanes each (lanes 60-63
-// idle); the lane of field l evaluates DF(l) alone, with the terms of
-// closure_rates in their order, so that it holds a fifth of the stencil and
-// its loads are in flight together.  The field-2 lane also forms szz, DF(6)
-// = nu (DF(3) + DF(5)), from the field-4 lane two lanes up.  Every lane runs
-// to the shuffle (idle lanes on a clamped point) and only active ones store.
-template <typename T, int OP = 4, bool EXT = false>
-__device__ __forceinline__ void band_fl_wave(const BulkArgs<T>& a, const int2* __restrict__ pts, int npts,
-                                             int wave, int lane) {
-  constexpr int NB = Sbp<OP>::nbst, NS = Sbp<OP>::nbnd, HW = Sbp<OP>::half;
-  const int grp = lane / 5, l = min(lane - 5 * grp, 4);
-  const int k = wave * 12 + grp;
-  const bool active = lane < 60 && k < npts;
-  const int2 p = pts[min(k, npts - 1)];
-  const int i = p.x, j = p.y;
-  const int bi = a.blk[a.rowb[j] * a.nbx + a.colb[i]];
-  const BlockDev& B = a.blocks[bi];
-  const long long ps = a.ps;
-  const int ld = a.ld;
-  const long long cc = (long long)j * ld + i;
-  const T* __restrict__ F = a.Fin;
-  const FldRt fr = fld_rt(l);
-  T d = a.a_zero ? (T)0.0 : (T)a.A * a.DF[l * ps + cc];
-  const int dl = i - B.mx, dr = B.px - i, db = j - B.my, dtp = B.py - j;
-  if (dl == 0 || dr == 0 || db == 0 || dtp == 0) {
-    // SAT penalties (all six fields, this lane's kept), sides L, R, B, T
-    T Fe[6], dd[6];
-#pragma unroll
-    for (int m = 0; m < 6; m++) {
-      Fe[m] = F[m * ps + cc];
-      dd[m] = d;
+// ---------------------------------------------------------------------
+// The band in the stage launch, one lane per (point, field).
+//
+// A point on a block edge needs only the hats of its own node, and a hat
+// only the fields of that node (of both sides, across an interface): the
+// edge nodes and edge points that belong together form small groups with no
+// dependence on each other.  A rim group is one workgroup: its first wave
+// evaluates the group's edge nodes (the boundary hats, the fault solve)
+// into LDS, while the other waves load the stencils of its edge points and
+// reduce them to their closure terms; after a barrier they add the SAT
+// penalties and the terms in the reference's order, and store.  So a stage
+// is one launch on one stream.
+//
+// It is bound by latency: the fault solve is a chain of FP64 exp, log and
+// divisions, and the loads of a point depend on its record and nothing
+// else.  A lane evaluates one field's closure terms, five (antiplane: three)
+// lanes a point.
+// ---------------------------------------------------------------------
+
+// closure terms of one field at a band point, in two runs: t, the one-sided
+// direction (q where the point has both, else the one it has), and u, the
+// other (one-sided in a corner, else central).  e, g: their dissipation
+// terms, dg the strips' diagonal.  (Each run is written whole on every path:
+// stores that differ between the paths would put it in scratch memory.)
+template <typename T, int OP, bool EXT>
+struct BandTerms {
+  static constexpr int NS = Sbp<OP>::nbnd;
+  T t[NS], u[NS];
+  T e[EXT ? NS : 1], g[EXT ? NS : 1];
+  T dg;
+  bool corner;
+};
+
+// Loads of a batch stay ahead of it, and their uses behind: without it the
+// compiler walks the terms one by one, a memory latency each.
+__device__ __forceinline__ void load_fence() { asm volatile("" ::: "memory"); }
+
+// the products of field l at a neighbour, p1 = (y metric) F(UA), p2 = (x
+// metric) F(UB): plane strain multiplies one of them by gamma (Fld),
+// antiplane shear has both for vz, the first alone for sxz and the second
+// alone for syz (on vz)
+template <typename T, int MODE>
+struct BandField {
+  const T* __restrict__ Fa;
+  const T* __restrict__ Fb;
+  const T* __restrict__ Fl;
+  FldRt fr;
+  int l;
+  T gamma, div, mul;  // of the lane's point (band_terms)
+  __device__ __forceinline__ BandField(const T* F, long long ps, int l_) : l(l_) {
+    Fl = F + l * ps;
+    if constexpr (MODE == 3) {
+      fr = FldRt{0, 0, l == 0 ? 0 : 1, false, false};
+      Fa = F + (l == 0 ? ps : 0);
+      Fb = F + (l == 0 ? 2 * ps : 0);
+    } else {
+      fr = fld_rt(l);
+      Fa = F + fr.ua * ps;
+      Fb = F + fr.ub * ps;
     }
-    if (dl == 0) sat_term<T>(dd, Fe, a.sd, B.side_off[FDM_SIDE_L] + db);
-    if (dr == 0) sat_term<T>(dd, Fe, a.sd, B.side_off[FDM_SIDE_R] + db);
-    if (db == 0) sat_term<T>(dd, Fe, a.sd, B.side_off[FDM_SIDE_B] + dl);
-    if (dtp == 0) sat_term<T>(dd, Fe, a.sd, B.side_off[FDM_SIDE_T] + dl);
-    d = l == 0 ? dd[0] : (l == 1 ? dd[1] : (l == 2 ? dd[2] : (l == 3 ? dd[3] : dd[4])));
   }
-  const T* __restrict__ xq = a.xq;
-  const T* __restrict__ xr = a.xr;
-  const T* __restrict__ yq = a.yq;
-  const T* __restrict__ yr = a.yr;
-  const T Ji = a.Ji[cc];
-  // EXT: a heterogeneous medium (the point's material) and artificial
-  // dissipation (SBP4 only), as in closure_rates
-  const bool het = EXT && a.mrho != nullptr;
-  const T gamma = het ? a.mgam[cc] : (T)B.gamma, rho = het ? a.mrho[cc] : (T)B.rho;
-  const T G = het ? a.mG[cc] : (T)B.G, M = het ? a.mM[cc] : (T)B.M;
-  const bool diss = EXT && OP == 4 && B.Cdiss > 0.0;
-  const T Cd = (T)B.Cdiss;
-  const T* __restrict__ Jp = a.J;
-  const T* __restrict__ Fl = F + l * ps;
-  const T* __restrict__ Fa = F + fr.ua * ps;
-  const T* __restrict__ Fb = F + fr.ub * ps;
-  const bool qone = (dl < NB) || (dr < NB);
-  const bool rone = (db < NB) || (dtp < NB);
-  const long long row = (long long)j * ld;
-  const long long colm = (long long)B.my * ld + i, colp = (long long)B.py * ld + i;
-  // q1: ay F(UA) - ax F(UB); r1: -by F(UA) + bx F(UB) (closure_rates)
-  if (qone) {
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      const long long kq = (dl < NB) ? row + B.mx + s : row + B.px - s;
-      const T Dq = (dl < NB) ? (T)sbp_dl<OP>(dl, s) : (T)(-sbp_dl<OP>(dr, s));
-      const T ay = (T)0.5 * (yr[kq] + yr[cc]), ax = (T)0.5 * (xr[kq] + xr[cc]);
-      const T tq = prod_rt(ay, Fa[kq], gamma, fr.ga) - prod_rt(ax, Fb[kq], gamma, fr.gb);
-      d = d + bscale_rt(tq, Dq, rho, G, M, fr.mat) * Ji;
-      if constexpr (EXT && OP == 4)
-        if (diss) d = d + Jp[kq] * Fl[kq] * (T)((dl < 4) ? kAL[dl][s] : kAL[dr][s]) * Ji * Cd;
-      if (rone) {
-        const long long kr = (db < NB) ? colm + (long long)s * ld : colp - (long long)s * ld;
-        const T Dr = (db < NB) ? (T)sbp_dl<OP>(db, s) : (T)(-sbp_dl<OP>(dtp, s));
-        const T by = (T)0.5 * (yq[kr] + yq[cc]), bx = (T)0.5 * (xq[kr] + xq[cc]);
-        const T tr = -prod_rt(by, Fa[kr], gamma, fr.ga) + prod_rt(bx, Fb[kr], gamma, fr.gb);
-        d = d + bscale_rt(tr, Dr, rho, G, M, fr.mat) * Ji;
-        if constexpr (EXT && OP == 4)
-          if (diss) d = d + Jp[kr] * Fl[kr] * (T)((db < 4) ? kAL[db][s] : kAL[dtp][s]) * Ji * Cd;
-      }
+  __device__ __forceinline__ void products(T my, T mx, T fa, T fb, T& p1, T& p2) const {
+    if constexpr (MODE == 3) {
+      p1 = my * fa;
+      p2 = mx * fb;
+    } else {
+      p1 = prod_rt(my, fa, gamma, fr.ga);
+      p2 = prod_rt(mx, fb, gamma, fr.gb);
     }
-    if (!rone) {
-      // L or R strip: central r (rc)
-      if constexpr (EXT && OP == 4)
-        if (diss) d = d + Fl[cc] * (T)FDM_AI0 * Cd;
-#pragma unroll
-      for (int s = 1; s <= HW; s++) {
-        const T D = (T)sbp_di<OP>(s);
-        const long long kp = cc + (long long)s * ld, km = cc - (long long)s * ld;
-        const T byp = (T)0.5 * (yq[kp] + yq[cc]), bxp = (T)0.5 * (xq[kp] + xq[cc]);
-        const T bym = (T)0.5 * (yq[km] + yq[cc]), bxm = (T)0.5 * (xq[km] + xq[cc]);
-        const T t = -prod_rt(byp, Fa[kp], gamma, fr.ga) + prod_rt(bxp, Fb[kp], gamma, fr.gb) +
-                    prod_rt(bym, Fa[km], gamma, fr.ga) - prod_rt(bxm, Fb[km], gamma, fr.gb);
-        d = d + bscale_rt(t, D, rho, G, M, fr.mat) * Ji;
-        if constexpr (EXT && OP == 4)
-          if (diss) d = d + (Jp[kp] * Fl[kp] + Jp[km] * Fl[km]) * ((s == 1) ? (T)FDM_AI1 : (T)FDM_AI2) * Ji * Cd;
-      }
+  }
+  // q: p1 - p2, r: -p1 + p2 (q1, r1; q1_3, r1_3)
+  __device__ __forceinline__ T one(bool q, T p1, T p2) const {
+    const T v = q ? p1 - p2 : p2 - p1;
+    if constexpr (MODE == 3) {
+      const T v1 = q ? p1 : -p1, v2 = q ? -p2 : p2;
+      return l == 0 ? v : (l == 1 ? v1 : v2);
     }
-  } else {
-    // B or T strip: one-sided r, then central q (qc)
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      const long long kr = (db < NB) ? colm + (long long)s * ld : colp - (long long)s * ld;
-      const T Dr = (db < NB) ? (T)sbp_dl<OP>(db, s) : (T)(-sbp_dl<OP>(dtp, s));
-      const T by = (T)0.5 * (yq[kr] + yq[cc]), bx = (T)0.5 * (xq[kr] + xq[cc]);
-      const T tr = -prod_rt(by, Fa[kr], gamma, fr.ga) + prod_rt(bx, Fb[kr], gamma, fr.gb);
-      d = d + bscale_rt(tr, Dr, rho, G, M, fr.mat) * Ji;
-      if constexpr (EXT && OP == 4)
-        if (diss) d = d + Jp[kr] * Fl[kr] * (T)((db < 4) ? kAL[db][s] : kAL[dtp][s]) * Ji * Cd;
+    return v;
+  }
+  // q: p1 - p2 - p3 + p4, r: -p1 + p2 + p3 - p4 (qc, rc; qc_3, rc_3), p1, p2
+  // at the plus neighbour, p3, p4 at the minus one
+  __device__ __forceinline__ T two(bool q, T p1, T p2, T p3, T p4) const {
+    const T v = q ? p1 - p2 - p3 + p4 : p2 - p1 + p3 - p4;
+    if constexpr (MODE == 3) {
+      const T v1 = q ? p1 - p3 : -p1 + p3, v2 = q ? -p2 + p4 : p2 - p4;
+      return l == 0 ? v : (l == 1 ? v1 : v2);
     }
-    if constexpr (EXT && OP == 4)
-      if (diss) d = d + Fl[cc] * (T)FDM_AI0 * Cd;
+    return v;
+  }
+  // ")*D/rho", ")*D*G", ")*D*M" (bscale, bscale3), both arms evaluated in
+  // every lane: as a branch, the lanes of vx and vy would run their
+  // divisions term by term
+  __device__ __forceinline__ T scale(T t, T D) const {
+    const T td = t * D;
+    T r = td / div;
+    asm volatile("" : "+v"(r));
+    return fr.mat == 0 ? r : td * mul;
+  }
+};
+
+// A one-sided sum's loads, neighbours base + s st for s = S0..S1-1, with the
+// coefficients of closure row `row`, and its terms (the coefficients negated
+// at the far side)
+template <typename T, int OP, int S0, int S1>
+struct OneSided {
+  static constexpr int N = S1 - S0, NS = Sbp<OP>::nbnd;
+  T my[N], mx[N], fa[N], fb[N], D[N], yc, xc;
+  template <typename F>
+  __device__ __forceinline__ void load(const F& f, const T* __restrict__ mY, const T* __restrict__ mX,
+                                       const long long cc, const long long base, const long long st,
+                                       const int row) {
+    yc = mY[cc];
+    xc = mX[cc];
+#pragma unroll
+    for (int s = 0; s < N; s++) {
+      const long long k = base + (S0 + s) * st;
+      my[s] = mY[k];
+      mx[s] = mX[k];
+      fa[s] = f.Fa[k];
+      fb[s] = f.Fb[k];
+      D[s] = (T)sbp_dl<OP>(row, S0 + s);
+    }
+  }
+  template <typename F>
+  __device__ __forceinline__ void terms(const F& f, const bool neg, const bool q, const T Ji, T (&t)[NS]) const {
+#pragma unroll
+    for (int s = 0; s < N; s++) {
+      T p1, p2;
+      f.products((T)0.5 * (my[s] + yc), (T)0.5 * (mx[s] + xc), fa[s], fb[s], p1, p2);
+      t[S0 + s] = f.scale(f.one(q, p1, p2), neg ? -D[s] : D[s]) * Ji;
+    }
+  }
+};
+
+template <typename T, int MODE, int OP, bool EXT>
+__device__ __forceinline__ void band_terms(const BulkArgs<T>& a, const BlockDev& B, const unsigned dist,
+                                           const long long cc, const int l, BandTerms<T, OP, EXT>& o) {
+  constexpr int NB = Sbp<OP>::nbst, NS = Sbp<OP>::nbnd, HW = Sbp<OP>::half;
+  const int dl = dist & 255, dr = (dist >> 8) & 255, db = (dist >> 16) & 255, dt = dist >> 24;
+  const int ld = a.ld;
+  const bool qone = dl < NB || dr < NB, rone = db < NB || dt < NB;
+  o.corner = qone && rone;
+  BandField<T, MODE> f(a.Fin, a.ps, l);
+  // base and stride of each direction's one-sided stencil, its row, its sign
+  const bool ql = dl < NB, rb = db < NB;
+  const long long bq = ql ? cc - dl : cc + dr, br = rb ? cc - (long long)db * ld : cc + (long long)dt * ld;
+  const long long sq = ql ? 1 : -1, sr = rb ? ld : -ld;
+  const int rq = ql ? dl : dr, rr = rb ? db : dt;
+  // the metric planes follow each other in the arena: xq, xr, yq, yr (a
+  // select between the argument's pointers would copy them to scratch)
+  const T* __restrict__ m1 = a.xq + (qone ? a.ps : 0);
+  const T* __restrict__ mX = a.xq + (qone ? 0 : a.ps);
+  const T* __restrict__ mY = mX + 2 * a.ps;
+  // SBP6's nine neighbours in FP64 in two batches (of up to 50 registers)
+  constexpr int SA = sizeof(T) == 8 && NS > 6 ? 5 : NS;
+  OneSided<T, OP, 0, SA> w;
+  w.load(f, m1 + 2 * a.ps, m1, cc, qone ? bq : br, qone ? sq : sr, qone ? rq : rr);
+  // the other direction's central neighbours (a corner has none: its own
+  // point, unused)
+  const long long sc = o.corner ? 0 : (qone ? ld : 1);
+  T my[2 * HW], mx[2 * HW], fa[2 * HW], fb[2 * HW], yc, xc;
+  auto load_central = [&]() {
+    yc = mY[cc];
+    xc = mX[cc];
 #pragma unroll
     for (int s = 1; s <= HW; s++) {
-      const T D = (T)sbp_di<OP>(s);
-      const long long kp = cc + s, km = cc - s;
-      const T ayp = (T)0.5 * (yr[kp] + yr[cc]), axp = (T)0.5 * (xr[kp] + xr[cc]);
-      const T aym = (T)0.5 * (yr[km] + yr[cc]), axm = (T)0.5 * (xr[km] + xr[cc]);
-      const T t = prod_rt(ayp, Fa[kp], gamma, fr.ga) - prod_rt(axp, Fb[kp], gamma, fr.gb) -
-                  prod_rt(aym, Fa[km], gamma, fr.ga) + prod_rt(axm, Fb[km], gamma, fr.gb);
-      d = d + bscale_rt(t, D, rho, G, M, fr.mat) * Ji;
-      if constexpr (EXT && OP == 4)
-        if (diss) d = d + (Jp[kp] * Fl[kp] + Jp[km] * Fl[km]) * ((s == 1) ? (T)FDM_AI1 : (T)FDM_AI2) * Ji * Cd;
+      const long long kp = cc + s * sc, km = cc - s * sc;
+      my[2 * s - 2] = mY[kp];
+      my[2 * s - 1] = mY[km];
+      mx[2 * s - 2] = mX[kp];
+      mx[2 * s - 1] = mX[km];
+      fa[2 * s - 2] = f.Fa[kp];
+      fa[2 * s - 1] = f.Fa[km];
+      fb[2 * s - 2] = f.Fb[kp];
+      fb[2 * s - 1] = f.Fb[km];
+    }
+  };
+  // in FP32 both directions' loads fit in flight together, in FP64 one's
+  constexpr bool kTogether = sizeof(T) == 4;
+  if constexpr (kTogether) load_central();
+  const T Ji = a.Ji[cc];
+  // the point's material in a heterogeneous medium (rates_h_boundary_mode2,
+  // rates_heterogeneous.f90:435-898; mode 3: 51-372)
+  const bool het = EXT && a.mrho != nullptr;
+  f.gamma = MODE == 3 ? (T)0 : (het ? a.mgam[cc] : (T)B.gamma);
+  f.div = het ? a.mrho[cc] : (T)B.rho;
+  const T G = het ? a.mG[cc] : (T)B.G;
+  f.mul = MODE == 3 || f.fr.mat == 1 ? G : (het ? a.mM[cc] : (T)B.M);
+  load_fence();
+  w.terms(f, qone ? !ql : !rb, qone, Ji, o.t);
+  if constexpr (SA < NS) {
+    OneSided<T, OP, SA, NS> v;
+    v.load(f, m1 + 2 * a.ps, m1, cc, qone ? bq : br, qone ? sq : sr, qone ? rq : rr);
+    load_fence();
+    v.terms(f, qone ? !ql : !rb, qone, Ji, o.t);
+  }
+  if constexpr (!kTogether) {
+    load_central();
+    load_fence();
+  }
+#pragma unroll
+  for (int s = 1; s <= HW; s++) {
+    const int u = 2 * s - 2;
+    T p1, p2, p3, p4;
+    f.products((T)0.5 * (my[u] + yc), (T)0.5 * (mx[u] + xc), fa[u], fb[u], p1, p2);
+    f.products((T)0.5 * (my[u + 1] + yc), (T)0.5 * (mx[u + 1] + xc), fa[u + 1], fb[u + 1], p3, p4);
+    o.u[s - 1] = f.scale(f.two(!qone, p1, p2, p3, p4), (T)sbp_di<OP>(s)) * Ji;
+  }
+#pragma unroll
+  for (int s = HW; s < NS; s++) o.u[s] = (T)0.0;
+  if (o.corner) {
+    w.load(f, mY, mX, cc, br, sr, rr);
+    load_fence();
+    w.terms(f, !rb, false, Ji, o.u);
+    if constexpr (SA < NS) {
+      OneSided<T, OP, SA, NS> v;
+      v.load(f, mY, mX, cc, br, sr, rr);
+      load_fence();
+      v.terms(f, !rb, false, Ji, o.u);
     }
   }
-  // finish_point (lean): szz, the field update, the rates
-  const T d4 = __shfl(d, (lane + 2) & 63, 64);
-  if (!active) return;
-  const T Bdt = (T)a.Bdt;
-  if (a.do_update) a.Fout[l * ps + cc] = F[l * ps + cc] + Bdt * d;
-  a.DF[l * ps + cc] = d;
-  if (l == 2) {
-    const T d5 = (a.mnu ? a.mnu[cc] : (T)B.nu) * (d + d4);
-    if (a.do_update) a.Fout[5 * ps + cc] = F[5 * ps + cc] + Bdt * d5;
-    a.DF[5 * ps + cc] = d5;
+  if constexpr (EXT && OP == 4) {
+    // dissipation terms beside each (closure_rates)
+    if (B.Cdiss > 0.0) {
+      const T Cd = (T)B.Cdiss;
+      const T* __restrict__ J = a.J;
+      const long long base = qone ? bq : br, st = qone ? sq : sr;
+      const int row = qone ? rq : rr;
+#pragma unroll
+      for (int s = 0; s < NS; s++) {
+        const long long k = base + s * st;
+        o.e[s] = J[k] * f.Fl[k] * (T)kAL[row][s] * Ji * Cd;
+      }
+      if (o.corner) {
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          const long long k = br + s * sr;
+          o.g[s] = J[k] * f.Fl[k] * (T)kAL[rr][s] * Ji * Cd;
+        }
+        o.dg = (T)0.0;
+      } else {
+#pragma unroll
+        for (int s = 1; s <= HW; s++) {
+          const long long kp = cc + s * sc, km = cc - s * sc;
+          o.g[s - 1] =
+              (J[kp] * f.Fl[kp] + J[km] * f.Fl[km]) * ((s == 1) ? (T)FDM_AI1 : (T)FDM_AI2) * Ji * Cd;
+        }
+#pragma unroll
+        for (int s = HW; s < NS; s++) o.g[s] = (T)0.0;
+        o.dg = f.Fl[cc] * (T)FDM_AI0 * Cd;
+      }
+    }
   }
 }
 
-template <typename T, int OP = 4, bool EXT = false>
-__global__ void __launch_bounds__(64) bulk_band_fl(BulkArgs<T> a, const int2* __restrict__ pts, int npts) {
-  band_fl_wave<T, OP, EXT>(a, pts, npts, blockIdx.x, threadIdx.x);
+// the terms added to d in the order of closure_rates: a corner interleaves
+// its two one-sided sums, a strip takes the one-sided one, then (with
+// dissipation) the diagonal, then the central one
+template <typename T, int OP, bool EXT>
+__device__ __forceinline__ T band_sum(T d, const BandTerms<T, OP, EXT>& o, const bool diss) {
+  constexpr int NS = Sbp<OP>::nbnd, HW = Sbp<OP>::half;
+  if (o.corner) {
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      d = d + o.t[s];
+      if (EXT && diss) d = d + o.e[s];
+      d = d + o.u[s];
+      if (EXT && diss) d = d + o.g[s];
+    }
+    return d;
+  }
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    d = d + o.t[s];
+    if (EXT && diss) d = d + o.e[s];
+  }
+  if (EXT && diss) d = d + o.dg;
+#pragma unroll
+  for (int s = 0; s < HW; s++) {
+    d = d + o.u[s];
+    if (EXT && diss) d = d + o.g[s];
+  }
+  return d;
 }
 
-// a heterogeneous medium holds five more values per lane, dissipation the
-// Jacobian's staging: three waves per SIMD keep them in registers
+// finish_point of a band point whose fields' rates sit in consecutive lanes.
+// Lean launches: each lane updates its own field, and field 2's lane forms
+// szz, DF(6) = nu (DF(3) + DF(5)), from field 4's rate two lanes up.  FULL:
+// the lane of field 0 gathers the rates and finishes the point.  Every lane
+// runs to the shuffles (idle ones on a clamped point).
+template <typename T, int MODE, bool FULL>
+__device__ __forceinline__ void band_finish(const BulkArgs<T>& a, const BlockDev& B, const BandPt& p,
+                                            const long long cc, const int l, const int lane, const bool active,
+                                            const T d, const T Fown, const T F6) {
+  const long long ps = a.ps;
+  if constexpr (MODE == 3) {
+    if (!active) return;
+    if (a.do_update) a.Fout[l * ps + cc] = Fown + (T)a.Bdt * d;
+    a.DF[l * ps + cc] = d;
+  } else if constexpr (FULL) {
+    T dd[6], Fc[6];
+#pragma unroll
+    for (int k = 0; k < 5; k++) dd[k] = __shfl(d, (lane - l + k) & 63, 64);
+    dd[5] = (T)0.0;
+    if (!active || l != 0) return;
+#pragma unroll
+    for (int k = 0; k < 6; k++) Fc[k] = a.Fin[k * ps + cc];
+    finish_point<T, true>(a, B, p.blk, p.i, p.j, cc, dd, Fc);
+  } else {
+    const T d4 = __shfl(d, (lane + 2) & 63, 64);
+    if (!active) return;
+    const T nu = a.mnu ? a.mnu[cc] : (T)B.nu;
+    const T Bdt = (T)a.Bdt;
+    const T d5 = nu * (d + d4);
+    T ds = d;
+    if (a.nplace) {
+      T v[6] = {d, d, d, d, d, d};
+      point_sources<T>(a, B.rho, p.blk, p.i, p.j, v);
+      ds = l == 0 ? v[0] : (l == 1 ? v[1] : (l == 2 ? v[2] : (l == 3 ? v[3] : v[4])));
+    }
+    if (a.do_update) a.Fout[l * ps + cc] = Fown + Bdt * ds;
+    a.DF[l * ps + cc] = ds;
+    if (l == 2) {
+      if (a.do_update) a.Fout[5 * ps + cc] = F6 + Bdt * d5;
+      a.DF[5 * ps + cc] = d5;
+    }
+  }
+}
+
+// lanes a point, points a wave and points a rim group (three waves)
+template <int MODE>
+struct BandLanes {
+  static constexpr int per = MODE == 3 ? 3 : 5, wave = 64 / per, group = 3 * wave;
+};
+
+// a wave of inner band points
+template <typename T, int MODE, bool FULL, bool EXT, int OP>
+__device__ __forceinline__ void inner_band_wave(const BulkArgs<T>& a, const int first, const int lane) {
+  using L = BandLanes<MODE>;
+  const int grp = lane / L::per, l = min(lane - L::per * grp, L::per - 1);
+  const bool active = grp < L::wave && first + grp < a.nib;
+  const BandPt p = a.ibpts[min(first + min(grp, L::wave - 1), a.nib - 1)];
+  const BlockDev& B = a.blocks[p.blk];
+  const long long cc = (long long)p.j * a.ld + p.i;
+  const T d0 = a.a_zero ? (T)0.0 : a.DF[l * a.ps + cc];
+  const T Fown = a.Fin[l * a.ps + cc], F6 = MODE == 3 ? (T)0 : a.Fin[5 * a.ps + cc];
+  BandTerms<T, OP, EXT> o;
+  band_terms<T, MODE, OP, EXT>(a, B, p.d, cc, l, o);
+  T d = a.a_zero ? (T)0.0 : (T)a.A * d0;
+  d = band_sum<T, OP, EXT>(d, o, B.Cdiss > 0.0);
+  band_finish<T, MODE, FULL>(a, B, p, cc, l, lane, active, d, Fown, F6);
+}
+
+// rows R..R+N-1 of a node into LDS, all loads before the first store
+template <typename T, int R, int N>
+__device__ __forceinline__ void stage_rows(const EdgeArgs<T>& e, const EdgeNode& nd, double* s, const int stride) {
+  double v[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) v[k] = node_row<T>(e, nd, R + k);
+  load_fence();
+#pragma unroll
+  for (int k = 0; k < N; k++) s[(R + k) * stride] = v[k];
+}
+
+// A kernel's arguments in memory (its own argument segment, or an ensemble's
+// table), read afresh through the constant address space: what one phase of
+// a rim group or the tiles loaded of them is not kept in scalar registers
+// for the next.
+template <typename P>
+__device__ __forceinline__ const P& memory_args(const void* p) {
+  typedef const __attribute__((address_space(4))) P ConstP;
+  unsigned long long u = (unsigned long long)p;
+  asm volatile("" : "+s"(u));
+  return *(const P*)(ConstP*)u;
+}
+
+// A rim group (see above).  First all four waves stage the values of its
+// edge nodes in LDS, a node a lane and a quarter of the rows a wave, so that
+// the node's whole input is in flight at once whatever registers the tiles
+// leave the kernel; then the first wave evaluates the nodes from LDS.
+template <typename T, int MODE, bool FULL, bool EXT, int OP>
+__device__ __forceinline__ void rim_group(const void* pa, const void* pe, const int wb, double* sN, const int wave,
+                                          const int lane) {
+  constexpr int NF = MODE == 3 ? 3 : 6;
+  using L = BandLanes<MODE>;
+  const EdgeArgs<T>& e = memory_args<EdgeArgs<T>>(pe);
+  const int4 g = e.rim[wb];
+  const int stride = g.z ? kRimIface : kRimNodes;
+  double (*sH)[6] = reinterpret_cast<double (*)[6]>(sN + kRimRowsMax);
+  const EdgeNode nd = e.rimnodes[wb * kRimNodes + lane];
+  // the point of this lane (the waves after the first)
+  const int first = max(wave - 1, 0) * L::wave;
+  const int grp = lane / L::per, l = min(lane - L::per * grp, L::per - 1);
+  const RimPt rp = e.rimpts[wb * kRimPts + max(min(first + min(grp, L::wave - 1), g.y - 1), 0)];
+  if (lane < g.x) {
+    double* s = sN + lane;
+    const bool itf = nd.iface >= 0;
+    if (wave == 0) {
+      stage_rows<T, kRowFm, NF>(e, nd, s, stride);
+      if (itf) stage_rows<T, kRowFp, NF>(e, nd, s, stride);
+    } else if (wave == 1) {
+      stage_rows<T, kRowF0m, NF>(e, nd, s, stride);
+      if (itf) stage_rows<T, kRowF0p, NF>(e, nd, s, stride);
+    } else if (wave == 2) {
+      stage_rows<T, kRowN, 5>(e, nd, s, stride);
+      if (itf) stage_rows<T, kRowRs, 7>(e, nd, s, stride);
+    } else if (wave == 3 && itf) {
+      stage_rows<T, kRowMp, 3>(e, nd, s, stride);
+      stage_rows<T, kRowS0, 3 + kNodeStRows>(e, nd, s, stride);
+    }
+  }
+  __syncthreads();
+  auto hats = [&](FaultSolved& f) {
+    const EdgeArgs<T>& en = memory_args<EdgeArgs<T>>(pe);
+    double hm[6], hp[6];
+    edge_node<T, MODE, true, FULL>(en, nd, NodeRows{sN + lane, stride}, hm, hp, f);
+#pragma unroll
+    for (int k = 0; k < NF; k++) sH[lane][k] = hm[k];
+    if (nd.iface >= 0) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) sH[stride + lane][k] = hp[k];
+    }
+  };
+  FaultSolved f;
+  // interface nodes on the first wave, boundary nodes of a group with both
+  // kinds (the corners) on the second, beside it
+  if (lane < g.x && wave == (g.z && nd.iface < 0 ? 1 : 0)) hats(f);
+  if (wave == 0) {
+    __syncthreads();
+    // the fault's own update, while the other waves finish the points
+    if (lane < g.x && nd.iface >= 0) edge_finish<T>(memory_args<EdgeArgs<T>>(pe), nd, NodeRows{sN + lane, stride}, f);
+    return;
+  }
+  const BulkArgs<T>& a = memory_args<BulkArgs<T>>(pa);
+  if (first >= g.y) {
+    __syncthreads();
+    return;
+  }
+  const bool active = grp < L::wave && first + grp < g.y;
+  const BandPt& p = rp.p;
+  const BlockDev& B = a.blocks[p.blk];
+  const long long ps = a.ps, cc = (long long)p.j * a.ld + p.i;
+  const int NS = a.sd.NS;
+  const T d0 = a.a_zero ? (T)0.0 : a.DF[l * ps + cc];
+  BandTerms<T, OP, EXT> o;
+  band_terms<T, MODE, OP, EXT>(a, B, p.d, cc, l, o);
+  T Fe[NF];
+#pragma unroll
+  for (int k = 0; k < NF; k++) Fe[k] = a.Fin[k * ps + cc];
+  // the side node's normal and penalty weights (a corner's second side: below)
+  T n1 = (T)0, n2 = (T)0, Ks = (T)0, Kp = (T)0;
+  auto side = [&](int so) {
+    Ks = (T)a.sd.M[3 * NS + so];
+    if constexpr (MODE == 2) {
+      n1 = (T)a.sd.normal[so];
+      n2 = (T)a.sd.normal[NS + so];
+      Kp = (T)a.sd.M[4 * NS + so];
+    }
+  };
+  side(rp.soA);
+  __syncthreads();
+  T d = a.a_zero ? (T)0.0 : (T)a.A * d0;
+  T Fown = Fe[0];
+#pragma unroll
+  for (int k = 1; k < L::per; k++) Fown = l == k ? Fe[k] : Fown;
+  // SAT penalties, sides in the order L, R, B, T
+#pragma unroll 1
+  for (int s = 0; s < 2; s++) {
+    const int so = s ? rp.soB : rp.soA, slot = s ? rp.slotB : rp.slotA;
+    if (so < 0) continue;
+    if (s) side(so);
+    if constexpr (MODE == 3) {
+      const double h = slot >= 0 ? sH[slot][l] : a.sd.Fhat[l * NS + so];
+      d = d + Ks * ((T)h - Fown);
+    } else {
+      double Fh[6];
+#pragma unroll
+      for (int k = 0; k < 6; k++) Fh[k] = slot >= 0 ? sH[slot][k] : a.sd.Fhat[k * NS + so];
+      // all fields' penalties, this lane's kept
+      T dd[6];
+#pragma unroll
+      for (int k = 0; k < 6; k++) dd[k] = d;
+      sat_hat<T>(dd, Fe, Fh, n1, n2, Ks, Kp);
+      d = l == 0 ? dd[0] : (l == 1 ? dd[1] : (l == 2 ? dd[2] : (l == 3 ? dd[3] : dd[4])));
+    }
+  }
+  d = band_sum<T, OP, EXT>(d, o, B.Cdiss > 0.0);
+  band_finish<T, MODE, FULL>(a, B, p, cc, l, lane, active, d, Fown, MODE == 3 ? (T)0 : Fe[NF - 1]);
+}
+
+template <typename T, int OP>
+__device__ __forceinline__ void point_generic3(const BulkArgs<T>& a, const int i, const int j, const int bi);
+
+// The workgroups of a stage launch ahead of its tiles: rim groups, then the
+// receivers of the previous step (nrecwg, plane strain), then the inner
+// band.  Dispatched first, their latency overlaps the tiles.  pa, pe: the
+// stage's BulkArgs (also a) and EdgeArgs in memory; wb: this workgroup's
+// index among them.
+template <typename T, int MODE, int TX, int TY, bool FULL, bool EXT, int OP>
+__device__ __forceinline__ void stage_ahead(const BulkArgs<T>& a, const void* pa, const void* pe, int wb,
+                                            char* smem) {
+  constexpr int NT = TX * TY;
+  const int tid = threadIdx.y * TX + threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  if (wb < a.nrimwg) {
+    rim_group<T, MODE, FULL, EXT, OP>(pa, pe, wb, reinterpret_cast<double*>(smem), wave, lane);
+    return;
+  }
+  wb -= a.nrimwg;
+  if constexpr (MODE == 2 && std::is_same<T, double>::value) {
+    if (wb < a.nrecwg) {
+      // the receivers of the previous step's fields (this stage's input,
+      // which the launch does not write)
+      const int r = wb * NT + tid;
+      if (r < a.nrec) {
+        const long long q = a.rcc[r];
+        a.rout[2 * r] = a.Fin[q];
+        a.rout[2 * r + 1] = a.Fin[a.ps + q];
+      }
+      return;
+    }
+    wb -= a.nrecwg;
+  }
+  if (a.ib_lanes) {
+    const int first = (wb * (NT / 64) + wave) * BandLanes<MODE>::wave;
+    if (first < a.nib) inner_band_wave<T, MODE, FULL, EXT, OP>(a, first, lane);
+    return;
+  }
+  const int k = wb * NT + tid;
+  if (k < a.nib) {
+    const BandPt p = a.ibpts[k];
+    if constexpr (MODE == 3) point_generic3<T, OP>(a, p.i, p.j, p.blk);
+    else point_generic<T, FULL, EXT, OP, false>(a, p.i, p.j, p.blk);
+  }
+}
+
+// The stage launch of plane strain: rim groups, receivers and inner band
+// (stage_ahead), then the interior tiles.  Large grids are bound by the
+// tiles' bytes, small ones by a rim group's chain (nodes' loads, Newton, SAT)
+// beside nearly empty tiles; the workgroups ahead start first so that the
+// chain runs under the tiles.  Against an edge, a band and an interior kernel
+// on two streams joined by events twice a stage, us a stage: 151^2 with a
+// point source 25.8 -> 10.4, 401^2 28.5 -> 13.5, 2 x 333x167 with a fault
+// 32.3 -> 15.4, 2 x 801x401 42.6 -> 26.1, 2 x 1601x801 106 -> 88.8 (FP32-bulk
+// 58.1 -> 47.6).  A heterogeneous medium holds five
+// more values per lane, dissipation the Jacobian's staging: three waves per
+// SIMD keep them in registers.
 template <typename T, int TX, int TY, bool FULL, bool NTS, bool HET, bool DISS, int OP = 4,
           bool JI = false, bool MC = false>
 __global__ void __launch_bounds__(TX * TY)
     __attribute__((amdgpu_waves_per_eu(FULL ? 2 : ((HET || DISS || OP == 6) ? 3 : 4))))
-bulk_interior(BulkArgs<T> a, const int4* __restrict__ tiles) {
-  if constexpr (!HET && OP == 4) {
-    // The first nibwg workgroups update the inner band points, one lane per
-    // point.  They need only what the tiles need (the previous stage's band
-    // and interior), so they ride in this launch rather than on the second
-    // stream after the edge values; dispatched first, their closures (bound
-    // by load latency) overlap the tiles.
-    if constexpr (std::is_same<T, double>::value) {
-      if ((int)blockIdx.x < a.nrecwg) {
-        // the receivers of the previous step's fields (this stage's input,
-        // which the launch does not write)
-        const int r = (int)blockIdx.x * (TX * TY) + (int)(threadIdx.y * TX + threadIdx.x);
-        if (r < a.nrec) {
-          const long long q = a.rcc[r];
-          a.rout[2 * r] = a.Fin[q];
-          a.rout[2 * r + 1] = a.Fin[a.ps + q];
-        }
-        return;
-      }
-    }
-    // receivers ride in FP64 launches only; the FP32 kernel keeps its offsets
-    const int wb = (int)blockIdx.x - (std::is_same<T, double>::value ? a.nrecwg : 0);
-    if (wb < a.nibwg) {
-      // one lane per point (five lanes per point, as in bulk_band_fl, made
-      // this launch slower: 600 workgroups ahead of the tiles instead of 112)
-      const int k = wb * (TX * TY) + (int)(threadIdx.y * TX + threadIdx.x);
-      if (k < a.nib) {
-        const int2 p = a.ibpts[k];
-        point_generic<T, FULL, DISS, OP>(a, p.x, p.y);
-      }
+bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
+  constexpr int kTile = tile_bytes<T, TX, TY, DISS, OP, 5>();
+  __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];
+  const int ahead = a.nrimwg + a.nrecwg + a.nibwg;
+  if ((int)blockIdx.x < ahead) {
+    const char* args = (const char*)__builtin_amdgcn_kernarg_segment_ptr();
+    stage_ahead<T, 2, TX, TY, FULL, HET || DISS, OP>(a, args, args + edge_args_at<T>(), blockIdx.x, smem);
+    return;
+  }
+  const int4 td = tiles[linear_tile(a.xcd_swizzle, ahead)];
+  if constexpr (!FULL) {
+    if (td.w) {
+      // The few tiles a point source reaches, a lane a point from global
+      // memory: in the tile's own path the source's terms took registers that
+      // it does not have (2 x 1601x801 FP64, tiles alone: 93.4 us a stage against
+      // 88.0).  DF6 is stored: the source makes it more than DF3 and DF5 tell.
+      const int bu = td.x, i = td.y + threadIdx.x, j = td.z + threadIdx.y;
+      const BlockDev& B = a.blocks[bu];
+      if (i <= B.px - Sbp<OP>::nbst && j <= B.py - Sbp<OP>::nbst)
+        point_generic<T, false, HET || DISS, OP, false, true>(a, i, j, bu);
       return;
     }
   }
-  interior_tile<T, TX, TY, FULL, NTS, HET, DISS, OP, JI, MC>(
-      a, tiles[linear_tile(a.xcd_swizzle, (std::is_same<T, double>::value ? a.nrecwg : 0) + a.nibwg)]);
+  interior_tile<T, TX, TY, FULL, NTS, HET, DISS, OP, JI, MC>(a, td, smem);
 }
 
-// Batched interior kernel: the tiles of many problems in one launch; tile
-// .w selects the problem's arguments in tab.
+// Batched stage launch: the rim groups, inner band points and tiles of many
+// problems.  ahead[k] = (problem, its workgroup index) of the nahead
+// workgroups ahead of the tiles; tile .w selects the problem's arguments.
 template <typename T, int TX, int TY, bool FULL, bool NTS>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(FULL ? 2 : 4)))
-bulk_interior_batch(const BulkArgs<T>* __restrict__ tab, const int4* __restrict__ tiles, int swz) {
-  const int4 td = tiles[linear_tile(swz)];
-  interior_tile<T, TX, TY, FULL, NTS, false, false>(tab[td.w], td);
+bulk_interior_batch(const BulkArgs<T>* __restrict__ tab, const EdgeArgs<T>* __restrict__ etab,
+                    const int2* __restrict__ ahead, int nahead, const int4* __restrict__ tiles, int swz) {
+  constexpr int kTile = tile_bytes<T, TX, TY, false, 4, 5>();
+  __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];
+  if ((int)blockIdx.x < nahead) {
+    const int2 w = ahead[blockIdx.x];
+    stage_ahead<T, 2, TX, TY, FULL, false, 4>(tab[w.x], tab + w.x, etab + w.x, w.y, smem);
+    return;
+  }
+  const int4 td = tiles[linear_tile(swz, nahead)];
+  interior_tile<T, TX, TY, FULL, NTS, false, false>(tab[td.w], td, smem);
 }
 
 
@@ -1447,7 +1903,7 @@ __global__ void __launch_bounds__(64) bulk_band(BulkArgs<T> a, const int2* __res
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= npts) return;
   const int2 p = pts[k];
-  point_generic<T, FULL, EXT, OP>(a, p.x, p.y);
+  point_generic<T, FULL, EXT, OP>(a, p.x, p.y, block_at(a, p.x, p.y));
 }
 
 // Layer kernel: the points of the perfectly matched layer blocks, one lane
@@ -1477,20 +1933,6 @@ __global__ void __launch_bounds__(256) bulk_pml(BulkArgs<T> a, const int2* __res
 #pragma unroll
   for (int l = 0; l < 6; l++) Fc[l] = a.Fin[l * a.ps + cc];
   finish_point<T, FULL, NTS>(a, B, bi, i, j, cc, d, Fc);
-}
-
-// Batched band kernel: pts[k] = (i, j, problem, valid), every wave's 64
-// entries of one problem (padding entries have valid = 0).
-template <typename T, bool FULL>
-__global__ void __launch_bounds__(64) bulk_band_batch(const BulkArgs<T>* __restrict__ tab,
-                                                      const int4* __restrict__ pts, int npts) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= npts) return;
-  const int4 p = pts[k];
-  const int m = __builtin_amdgcn_readfirstlane(p.z);
-  if (!p.w) return;
-  // ensemble members have neither a heterogeneous medium nor dissipation
-  point_generic<T, FULL, false>(tab[m], p.x, p.y);
 }
 
 // ---------------------------------------------------------------------
@@ -1720,9 +2162,8 @@ __device__ __forceinline__ void closure_rates3(const BulkArgs<T>& a, const Block
 // one grid point of one stage in antiplane shear, neighbours from global
 // memory: A*DF, SAT, rates, update (fields.f90:1117-1133, 1225-1242)
 template <typename T, int OP = 4>
-__device__ __forceinline__ void point_generic3(const BulkArgs<T>& a, const int i, const int j) {
+__device__ __forceinline__ void point_generic3(const BulkArgs<T>& a, const int i, const int j, const int bi) {
   constexpr int NB = Sbp<OP>::nbst, HW = Sbp<OP>::half;
-  const int bi = a.blk[a.rowb[j] * a.nbx + a.colb[i]];
   const BlockDev& B = a.blocks[bi];
   const long long ps = a.ps;
   const int ld = a.ld;
@@ -1783,124 +2224,7 @@ __global__ void __launch_bounds__(256) bulk_kernel3(BulkArgs<T> a) {
   const int i = tx * blockDim.x + threadIdx.x;
   const int j = ty * blockDim.y + threadIdx.y;
   if (i >= a.nx || j >= a.ny) return;
-  point_generic3<T, OP>(a, i, j);
-}
-
-// Antiplane band kernel with one lane per (point, field) for blocks
-// without dissipation: 21 points per wave, three lanes each (lane 63
-// idle).  The lane of field l evaluates DF(l) alone with closure_rates3's
-// terms in their order (a medium's rho and G per point as there); the three
-// fields are not coupled after the rates, so each lane finishes its own.
-// A point of a dissipative block is left to bulk_band3 (the host sends
-// only blocks without dissipation here).
-template <typename T, int OP = 4>
-__global__ void __launch_bounds__(64) bulk_band3_fl(BulkArgs<T> a, const int2* __restrict__ pts, int npts) {
-  constexpr int NB = Sbp<OP>::nbst, NS = Sbp<OP>::nbnd, HW = Sbp<OP>::half;
-  const int lane = threadIdx.x;
-  const int grp = lane / 3, l = lane - 3 * grp;
-  const int k = blockIdx.x * 21 + grp;
-  if (lane >= 63 || k >= npts) return;
-  const int2 p = pts[k];
-  const int i = p.x, j = p.y;
-  const int bi = a.blk[a.rowb[j] * a.nbx + a.colb[i]];
-  const BlockDev& B = a.blocks[bi];
-  const long long ps = a.ps;
-  const int ld = a.ld;
-  const long long cc = (long long)j * ld + i;
-  const T* __restrict__ F = a.Fin;
-  T d = a.a_zero ? (T)0.0 : (T)a.A * a.DF[l * ps + cc];
-  const int dl = i - B.mx, dr = B.px - i, db = j - B.my, dtp = B.py - j;
-  if (dl == 0 || dr == 0 || db == 0 || dtp == 0) {
-    const T Fe = F[l * ps + cc];
-    const int NSd = a.sd.NS;
-    const int sides[4] = {dl == 0 ? B.side_off[FDM_SIDE_L] + db : -1,
-                          dr == 0 ? B.side_off[FDM_SIDE_R] + db : -1,
-                          db == 0 ? B.side_off[FDM_SIDE_B] + dl : -1,
-                          dtp == 0 ? B.side_off[FDM_SIDE_T] + dl : -1};
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int so = sides[e];
-      if (so < 0) continue;
-      const T Ks = (T)a.sd.M[3 * NSd + so];
-      d = d + Ks * ((T)a.sd.Fhat[l * NSd + so] - Fe);
-    }
-  }
-  const T* __restrict__ xq = a.xq;
-  const T* __restrict__ xr = a.xr;
-  const T* __restrict__ yq = a.yq;
-  const T* __restrict__ yr = a.yr;
-  const T Ji = a.Ji[cc];
-  const T rho = a.mrho ? a.mrho[cc] : (T)B.rho, G = a.mrho ? a.mG[cc] : (T)B.G;
-  // field 0 (vz) pairs sxz with the y-metrics and syz with the x-metrics;
-  // fields 1 and 2 (sxz, syz) take vz alone
-  const T* __restrict__ Fa = F + (l == 0 ? ps : 0);
-  const T* __restrict__ Fb = F + 2 * ps;
-  const bool qone = (dl < NB) || (dr < NB);
-  const bool rone = (db < NB) || (dtp < NB);
-  const long long row = (long long)j * ld;
-  const long long colm = (long long)B.my * ld + i, colp = (long long)B.py * ld + i;
-  // q1_3, r1_3, qc_3, rc_3 and bscale3 of field l
-  auto q1 = [&](long long kk) {
-    const T ay = (T)0.5 * (yr[kk] + yr[cc]), ax = (T)0.5 * (xr[kk] + xr[cc]);
-    return l == 0 ? ay * Fa[kk] - ax * Fb[kk] : (l == 1 ? ay * Fa[kk] : -(ax * Fa[kk]));
-  };
-  auto r1 = [&](long long kk) {
-    const T by = (T)0.5 * (yq[kk] + yq[cc]), bx = (T)0.5 * (xq[kk] + xq[cc]);
-    return l == 0 ? -(by * Fa[kk]) + bx * Fb[kk] : (l == 1 ? -(by * Fa[kk]) : bx * Fa[kk]);
-  };
-  auto sc = [&](T t, T D) { return l == 0 ? t * D / rho : t * D * G; };
-  if (qone) {
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      const long long kq = (dl < NB) ? row + B.mx + s : row + B.px - s;
-      const T Dq = (dl < NB) ? (T)sbp_dl<OP>(dl, s) : (T)(-sbp_dl<OP>(dr, s));
-      d = d + sc(q1(kq), Dq) * Ji;
-      if (rone) {
-        const long long kr = (db < NB) ? colm + (long long)s * ld : colp - (long long)s * ld;
-        const T Dr = (db < NB) ? (T)sbp_dl<OP>(db, s) : (T)(-sbp_dl<OP>(dtp, s));
-        d = d + sc(r1(kr), Dr) * Ji;
-      }
-    }
-    if (!rone) {
-#pragma unroll
-      for (int s = 1; s <= HW; s++) {
-        const T D = (T)sbp_di<OP>(s);
-        const long long kp = cc + (long long)s * ld, km = cc - (long long)s * ld;
-        const T byp = (T)0.5 * (yq[kp] + yq[cc]), bxp = (T)0.5 * (xq[kp] + xq[cc]);
-        const T bym = (T)0.5 * (yq[km] + yq[cc]), bxm = (T)0.5 * (xq[km] + xq[cc]);
-        const T t = l == 0 ? -(byp * Fa[kp]) + bxp * Fb[kp] + bym * Fa[km] - bxm * Fb[km]
-                           : (l == 1 ? -(byp * Fa[kp]) + bym * Fa[km] : bxp * Fa[kp] - bxm * Fa[km]);
-        d = d + sc(t, D) * Ji;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      const long long kr = (db < NB) ? colm + (long long)s * ld : colp - (long long)s * ld;
-      const T Dr = (db < NB) ? (T)sbp_dl<OP>(db, s) : (T)(-sbp_dl<OP>(dtp, s));
-      d = d + sc(r1(kr), Dr) * Ji;
-    }
-#pragma unroll
-    for (int s = 1; s <= HW; s++) {
-      const T D = (T)sbp_di<OP>(s);
-      const long long kp = cc + s, km = cc - s;
-      const T ayp = (T)0.5 * (yr[kp] + yr[cc]), axp = (T)0.5 * (xr[kp] + xr[cc]);
-      const T aym = (T)0.5 * (yr[km] + yr[cc]), axm = (T)0.5 * (xr[km] + xr[cc]);
-      const T t = l == 0 ? ayp * Fa[kp] - axp * Fb[kp] - aym * Fa[km] + axm * Fb[km]
-                         : (l == 1 ? ayp * Fa[kp] - aym * Fa[km] : -(axp * Fa[kp]) + axm * Fa[km]);
-      d = d + sc(t, D) * Ji;
-    }
-  }
-  if (a.do_update) a.Fout[l * ps + cc] = F[l * ps + cc] + (T)a.Bdt * d;
-  a.DF[l * ps + cc] = d;
-}
-
-template <typename T, int OP = 4>
-__global__ void __launch_bounds__(64) bulk_band3(BulkArgs<T> a, const int2* __restrict__ pts, int npts) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= npts) return;
-  const int2 p = pts[k];
-  point_generic3<T, OP>(a, p.x, p.y);
+  point_generic3<T, OP>(a, i, j, block_at(a, i, j));
 }
 
 // interior tiles in antiplane shear: vz, sxz, syz with a halo of the
@@ -1910,34 +2234,25 @@ __global__ void __launch_bounds__(64) bulk_band3(BulkArgs<T> a, const int2* __re
 // halo of F; a block without it keeps the plain expression.
 template <typename T, int TX, int TY, bool NTS, int OP = 4, bool HET = false, bool DISS = false>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(DISS ? 3 : 4)))
-bulk_interior3(BulkArgs<T> a, const int4* __restrict__ tiles) {
+bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   static_assert(!DISS || OP == 4, "artificial dissipation is built for SBP4 only");
   constexpr int H = Sbp<OP>::half, NB = Sbp<OP>::nbst;
   constexpr int HX = TX + 2 * H, HY = TY + 2 * H, NT = TX * TY;
-  if constexpr (!HET && !DISS && OP == 4) {
-    // the inner band points ahead of the tiles, one lane per point, as in
-    // the plane-strain launch (band split, on request).  This path takes
-    // the FP64 kernel from 76 to 120 VGPRs (six waves per SIMD to four);
-    // with the split off, the four-wave kernel made the antiplane step
-    // shorter (0.356 against 0.366 ms on the C2-size grid, FP32-bulk 0.215
-    // against 0.221).
-    if ((int)blockIdx.x < a.nibwg) {
-      const int k = (int)blockIdx.x * NT + (int)(threadIdx.y * TX + threadIdx.x);
-      if (k < a.nib) {
-        const int2 p = a.ibpts[k];
-        point_generic3<T, OP>(a, p.x, p.y);
-      }
-      return;
-    }
+  constexpr int kTile = tile_bytes<T, TX, TY, DISS, OP, 3>();
+  __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];
+  if ((int)blockIdx.x < a.nrimwg + a.nibwg) {
+    const char* args = (const char*)__builtin_amdgcn_kernarg_segment_ptr();
+    stage_ahead<T, 3, TX, TY, false, HET || DISS, OP>(a, args, args + edge_args_at<T>(), blockIdx.x, smem);
+    return;
   }
   constexpr int NF = (HY * HX + NT - 1) / NT;
   constexpr int NR = (TY * HX + NT - 1) / NT;
   constexpr int NQ = (HY * TX + NT - 1) / NT;
-  __shared__ T sF[3][HY][HX];
-  __shared__ T sR[2][TY][HX];
-  __shared__ T sQ[2][HY][TX];
-  __shared__ T sJ[DISS ? HY : 1][DISS ? HX : 1];
-  const int4 td = tiles[linear_tile(a.xcd_swizzle, a.nibwg)];
+  T (*sF)[HY][HX] = reinterpret_cast<T (*)[HY][HX]>(smem);
+  T (*sR)[TY][HX] = reinterpret_cast<T (*)[TY][HX]>(smem + 3 * HY * HX * sizeof(T));
+  T (*sQ)[HY][TX] = reinterpret_cast<T (*)[HY][TX]>(smem + (3 * HY + 2 * TY) * HX * sizeof(T));
+  T (*sJ)[HX] = reinterpret_cast<T (*)[HX]>(smem + ((3 * HY + 2 * TY) * HX + 2 * HY * TX) * sizeof(T));
+  const int4 td = tiles[linear_tile(a.xcd_swizzle, a.nrimwg + a.nibwg)];
   const int bu = td.x, i0 = td.y, j0 = td.z;
   ConstBlockDev* B4 = (ConstBlockDev*)a.blocks + bu;
   const int tid = threadIdx.y * TX + threadIdx.x;

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/fdmap.h"
+#include "fdm_mms.hpp"
 
 namespace fdm {
 
@@ -143,10 +144,13 @@ __device__ __forceinline__ double pow8(double x) {
   return x4 * x4;
 }
 
-// mms_sin (mms.f90:52-234).  field: 0..5 fields, 6..11 sources s_*.
-__device__ double mms_sin(double x, double y, double t, int side, int field);
+// x**0.125 by three square roots, each correctly rounded: the error stays
+// below 0.9 ulp, and the chain is a few dozen instructions instead of pow's
+// hundreds (it lies on the stage's longest dependent chain)
+__device__ __forceinline__ double root8(double x) { return sqrt(sqrt(sqrt(x))); }
 
 // set_bc_mode2 (boundaries.f90:216-377)
+template <bool MMS>
 __device__ __forceinline__ void set_bc_mode2(double* Fhat, const double* F, const double* F0,
                                              double n1, double n2, int bc, double Zs, double Zp,
                                              double gamma, double x, double y, double t,
@@ -161,17 +165,18 @@ __device__ __forceinline__ void set_bc_mode2(double* Fhat, const double* F, cons
   NT fd = xy2nt(Fd, n1, n2);
   double vt = 0.0, vn = 0.0, snt = 0.0, snn = 0.0;
   switch (bc) {
-    case FDM_BC_MMS_SIN_W: {
-      double FEX[6];
-      for (int l = 0; l < 5; l++) FEX[l] = mms_sin(x, y, t, iblock, l);
-      FEX[5] = 0.0;
-      NT ex = xy2nt(FEX, n1, n2);
-      vt = 0.5 * (ex.vt + fd.vt + Zsi * (ex.snt - fd.snt));
-      snt = 0.5 * (ex.snt + fd.snt + Zs * (ex.vt - fd.vt));
-      vn = 0.5 * (ex.vn + fd.vn + Zpi * (ex.snn - fd.snn));
-      snn = 0.5 * (ex.snn + fd.snn + Zp * (ex.vn - fd.vn));
+    case FDM_BC_MMS_SIN_W:
+      if constexpr (MMS) {
+        double FEX[6];
+        for (int l = 0; l < 5; l++) FEX[l] = mms_sin(x, y, t, iblock, l);
+        FEX[5] = 0.0;
+        NT ex = xy2nt(FEX, n1, n2);
+        vt = 0.5 * (ex.vt + fd.vt + Zsi * (ex.snt - fd.snt));
+        snt = 0.5 * (ex.snt + fd.snt + Zs * (ex.vt - fd.vt));
+        vn = 0.5 * (ex.vn + fd.vn + Zpi * (ex.snn - fd.snn));
+        snn = 0.5 * (ex.snn + fd.snn + Zp * (ex.vn - fd.vn));
+      }
       break;
-    }
     case FDM_BC_ABSORBING:
     case FDM_BC_ABSORBING_0:
       vt = 0.5 * (fd.vt - Zsi * fd.snt);
@@ -400,7 +405,7 @@ __device__ __forceinline__ double state_rate(int law, const double* rs, double V
     case FDM_LAW_FL:
       frs = a * log(absV / V0) + Psi;
       fLV = f0 - (b - a) * log(absV / V0);
-      fss = fw + (fLV - fw) / pow(1.0 + pow8(V / Vw), 0.125);
+      fss = fw + (fLV - fw) / root8(1.0 + pow8(V / Vw));
       return -(absV / L) * (frs - fss);
     case FDM_LAW_RSL:
       fss = f0 - (b - a) * log(absV / V0);
@@ -408,12 +413,12 @@ __device__ __forceinline__ double state_rate(int law, const double* rs, double V
       return -(absV / L) * (frs - fss);
     case FDM_LAW_RFL:
       fLV = f0 - (b - a) * log(absV / V0);
-      fss = fw + (fLV - fw) / pow(1.0 + pow8(V / Vw), 0.125);
+      fss = fw + (fLV - fw) / root8(1.0 + pow8(V / Vw));
       frs = a * arcsinh_ref(0.5 * absV / V0 * E);
       return (absV / L) * (fss - frs);
     case FDM_LAW_RSF:
       fLV = f0 - (b - a) * log(absV / V0);
-      fss = fw + (fLV - fw) / pow(1.0 + pow8(V / Vw), 0.125);
+      fss = fw + (fLV - fw) / root8(1.0 + pow8(V / Vw));
       Psiss = a * log(2.0 * V0 / absV * sinh(fss / a));
       return (absV / L) * (Psiss - Psi);
     case FDM_LAW_RAL:
@@ -494,8 +499,10 @@ __device__ __forceinline__ bool solve_friction_core(int law, const double* rs, c
       return false;
     }
     default: {
-      bool fail = newton_solver(law, rs[0], rs[2], V, S, Slock, Nreg, eta, Psi, E);
-      if (fail) fail = newton_solver(law, rs[0], rs[2], V, S, Slock, Nreg, eta, Psi, E);
+      // a second try from where the first one stopped
+      bool fail = true;
+#pragma unroll 1
+      for (int k = 0; k < 2 && fail; k++) fail = newton_solver(law, rs[0], rs[2], V, S, Slock, Nreg, eta, Psi, E);
       if (force) {
         const double Sk = kc0 + Nreg * kf;
         if (Sk < fabs(S)) {

@@ -229,12 +229,13 @@ typedef struct fdm_problem {
 
 /* Kernel timing gathered with HIP events on the context's stream. */
 typedef struct fdm_profile_t {
-  double bulk_ms;        /* summed duration of the bulk (stencil+RK) launches
-                            that update the block interiors: the interior
-                            tiles and, in PML blocks, the layer points four
-                            or more from every block edge                  */
+  double bulk_ms;        /* summed duration of the bulk (stencil+RK) launches:
+                            whole stages, or in a problem with a PML the
+                            interior tiles and the layer points four or more
+                            from every block edge                          */
   int64_t bulk_launches;
-  double edge_ms;        /* summed duration of edge/interface launches      */
+  double edge_ms;        /* summed duration of edge/interface launches (0
+                            where the stage launch evaluates them)         */
   int64_t edge_launches;
   int64_t bulk_points;   /* grid points updated per stage by those launches */
   double band_ms;        /* summed duration of the launches that update the
