@@ -27,7 +27,7 @@ namespace fdm {
 
 // SBP4 first-derivative matrix entry (row r, column c) on n >= 12 points:
 // rows 0..3 the closure DL, the last four rows -DL mirrored, else DI.
-__device__ __forceinline__ double sbp_entry(int r, int c, int n) {
+__host__ __device__ constexpr double sbp_entry(int r, int c, int n) {
   if (r < 4) return (c >= 0 && c < 6) ? kDL[r][c] : 0.0;
   if (r > n - 5) {
     const int rr = n - 1 - r, cr = n - 1 - c;
@@ -39,6 +39,28 @@ __device__ __forceinline__ double sbp_entry(int r, int c, int n) {
   if (s == 2) return FDM_DI2;
   if (s == -2) return -FDM_DI2;
   return 0.0;
+}
+
+// The entries of column c in rows max(0, c-5) + t, t = 0..10, by the place of
+// c: its distance from the near side up to 5, inside (6), or 12 less its
+// distance from the far side (n >= 12: no column is near both).  A table: as
+// selects on r and c per row, the entries took 100 registers of the gathers.
+struct SbpColumns {
+  double d[13][11];
+};
+constexpr SbpColumns sbp_columns() {
+  SbpColumns T{};
+  const int n = 24;
+  for (int k = 0; k < 13; k++) {
+    const int c = k < 6 ? k : (k == 6 ? 11 : n - 1 - (12 - k));
+    const int r0 = c > 5 ? c - 5 : 0;
+    for (int t = 0; t < 11; t++) T.d[k][t] = r0 + t <= (c + 5 < n - 1 ? c + 5 : n - 1) ? sbp_entry(r0 + t, c, n) : 0.0;
+  }
+  return T;
+}
+__device__ constexpr SbpColumns kSbpColumns = sbp_columns();
+__device__ __forceinline__ const double* sbp_column(int c, int n) {
+  return kSbpColumns.d[min(c, 6) + 6 - min(n - 1 - c, 6)];
 }
 
 struct AdjBulkArgs {
@@ -126,12 +148,23 @@ __device__ __forceinline__ void adj_dir(const AdjBulkArgs& a, double (&g)[5], co
     row(c + 2, -FDM_DI2);
   } else {
     const int r0 = max(0, c - 5), r1 = min(n - 1, c + 5);
+    const double* __restrict__ col = sbp_column(c, n);
 #pragma unroll
     for (int t = 0; t < 11; t++) {
       const int r = min(r0 + t, r1);
-      const double D = (r0 + t <= r1) ? sbp_entry(r, c, n) : 0.0;
-      row(r, D);
+      row(r, col[t]);
     }
+  }
+}
+
+// the two recurrences
+__device__ __forceinline__ void adj_finish(const AdjBulkArgs& a, const long long cc, const double (&g)[5]) {
+  const long long ps = a.ps;
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    const double lo = a.lin[l * ps + cc] + g[l];
+    a.lout[l * ps + cc] = lo;
+    a.mout[l * ps + cc] = a.A * a.min[l * ps + cc] + a.Bdt_prev * lo;
   }
 }
 
@@ -161,12 +194,7 @@ __device__ __forceinline__ void adj_point(const AdjBulkArgs& a, const int i, con
   for (int k = 0; k < nso; k++)
 #pragma unroll
     for (int l = 0; l < 5; l++) g[l] += a.gE[l * NS + so[k]];
-#pragma unroll
-  for (int l = 0; l < 5; l++) {
-    const double lo = a.lin[l * ps + cc] + g[l];
-    a.lout[l * ps + cc] = lo;
-    a.mout[l * ps + cc] = a.A * a.min[l * ps + cc] + a.Bdt_prev * lo;
-  }
+  adj_finish(a, cc, g);
 }
 
 __global__ void __launch_bounds__(256) adj_bulk_kernel(AdjBulkArgs a) {
@@ -191,64 +219,55 @@ __device__ __forceinline__ void adj_dir_any(const AdjBulkArgs& a, double (&g)[5]
   const double y0 = m1[cc], x0 = m2[cc];
   const long long ps = a.ps;
   const int r0 = max(0, c - 5), r1 = min(n - 1, c + 5);
+  // a batch's loads are in flight together; all eleven rows at once would
+  // take registers that the stage kernel's tiles do not leave
+  const double* __restrict__ col = sbp_column(c, n);
+  constexpr int kBatch = 4;
 #pragma unroll
-  for (int t = 0; t < 11; t++) {
-    const int r = min(r0 + t, r1);
-    const double D = (r0 + t <= r1) ? sbp_entry(r, c, n) : 0.0;
-    const long long kk = base + (long long)r * step;
-    const double Jk = a.Ji[kk];
-    double w[5];
+  for (int t0 = 0; t0 < 11; t0 += kBatch) {
+    double v[kBatch][8], D[kBatch];
 #pragma unroll
-    for (int l = 0; l < 5; l++) w[l] = a.min[l * ps + kk] * Jk * cl[l];
-    const double ay = sg * (0.5 * (m1[kk] + y0) * D), ax = sg * (0.5 * (m2[kk] + x0) * D);
-    adj_row<true>(g, w, ay, ax, gam);
+    for (int u = 0; u < kBatch && t0 + u < 11; u++) {
+      const int t = t0 + u, r = min(r0 + t, r1);
+      D[u] = col[t];
+      // (32-bit byte offsets: the tiles' bound on a plane's size holds here)
+      unsigned o = (unsigned)(base + (long long)r * step) * 8u;
+      asm volatile("" : "+v"(o));
+#pragma unroll
+      for (int l = 0; l < 5; l++) v[u][l] = ld_off(a.min + l * ps, o);
+      v[u][5] = ld_off(a.Ji, o);
+      v[u][6] = ld_off(m1, o);
+      v[u][7] = ld_off(m2, o);
+    }
+    load_fence();
+#pragma unroll
+    for (int u = 0; u < kBatch && t0 + u < 11; u++) {
+      double w[5];
+#pragma unroll
+      for (int l = 0; l < 5; l++) w[l] = v[u][l] * v[u][5] * cl[l];
+      const double ay = sg * (0.5 * (v[u][6] + y0) * D[u]), ax = sg * (0.5 * (v[u][7] + x0) * D[u]);
+      adj_row<true>(g, w, ay, ax, gam);
+    }
   }
 }
 
-// points within six of their block's edge (closure rows reach them, or
-// SAT), two lanes per point: the even lane gathers the q-derivative rows,
-// the odd lane the r-derivative rows (so each lane's chain of dependent
-// loads is half as long, and twice the waves are in flight); the pair adds
-// its sums, and the even lane adds the edge contributions and finishes the
-// point as adj_point does
-__global__ void __launch_bounds__(64) adj_band_kernel(AdjBulkArgs a, const int2* __restrict__ pts,
-                                                      int npts) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = t >> 1;
-  if (k >= npts) return;  // both lanes of a pair leave together
-  const bool q = (t & 1) == 0;
-  const int2 p = pts[k];
-  const int i = p.x, j = p.y;
-  const int bi = a.blk[a.rowb[j] * a.nbx + a.colb[i]];
-  const BlockDev& B = a.blocks[bi];
+// A point within six of its block's edge (closure rows reach it, or SAT) on
+// two lanes: the even lane gathers the q-derivative rows, the odd lane the
+// r-derivative rows (so each lane's chain of dependent loads is half as long,
+// and twice the waves are in flight), and the pair adds its sums.  R^T mu at
+// the point, in both lanes.
+__device__ __forceinline__ void adj_pair(const AdjBulkArgs& a, const BlockDev& B, const int i, const int j,
+                                         const bool q, double (&g)[5]) {
   const int nq = B.px - B.mx + 1, nr = B.py - B.my + 1;
   const int il = i - B.mx, jl = j - B.my;
-  const long long ps = a.ps;
   const int ld = a.ld;
-  const long long cc = (long long)j * ld + i;
-  const double gam = B.gamma;
   const double cl[5] = {1.0 / B.rho, 1.0 / B.rho, B.M, B.G, B.M};
-  double g[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int l = 0; l < 5; l++) g[l] = 0.0;
   adj_dir_any(a, g, q ? il : jl, q ? nq : nr, q ? (long long)j * ld + B.mx : (long long)B.my * ld + i,
-              q ? 1 : ld, cc, cl, gam, q);
+              q ? 1 : ld, (long long)j * ld + i, cl, B.gamma, q);
 #pragma unroll
   for (int l = 0; l < 5; l++) g[l] = g[l] + __shfl_xor(g[l], 1);
-  if (!q) return;
-  const int NS = a.NS;
-  int so[4], nso = 0;
-  if (il == 0) so[nso++] = B.side_off[FDM_SIDE_L] + jl;
-  if (il == nq - 1) so[nso++] = B.side_off[FDM_SIDE_R] + jl;
-  if (jl == 0) so[nso++] = B.side_off[FDM_SIDE_B] + il;
-  if (jl == nr - 1) so[nso++] = B.side_off[FDM_SIDE_T] + il;
-  for (int m = 0; m < nso; m++)
-#pragma unroll
-    for (int l = 0; l < 5; l++) g[l] += a.gE[l * NS + so[m]];
-#pragma unroll
-  for (int l = 0; l < 5; l++) {
-    const double lo = a.lin[l * ps + cc] + g[l];
-    a.lout[l * ps + cc] = lo;
-    a.mout[l * ps + cc] = a.A * a.min[l * ps + cc] + a.Bdt_prev * lo;
-  }
 }
 
 // Interior adjoint kernel over TX x TY tiles of each block's rectangle
@@ -260,17 +279,19 @@ __global__ void __launch_bounds__(64) adj_band_kernel(AdjBulkArgs a, const int2*
 // q and r, xr/yr with the q halo and xq/yq with the r halo are staged in
 // LDS.  Halo indices are clamped into the grid; a clamped value never
 // reaches an active lane.  tiles[k] = (block, i0, j0, 0).
+template <int TX, int TY>
+constexpr int adj_tile_bytes() {
+  return 8 * (5 * (TY + 4) * (TX + 4) + 2 * TY * (TX + 4) + 2 * (TY + 4) * TX);
+}
 template <int TX, int TY, bool NTS>
-__global__ void __launch_bounds__(TX * TY) adj_interior_kernel(AdjBulkArgs a,
-                                                               const int4* __restrict__ tiles) {
+__device__ __forceinline__ void adj_tile(const AdjBulkArgs& a, const int4 td, char* smem) {
   constexpr int HX = TX + 4, HY = TY + 4, NT = TX * TY;
   constexpr int NF = (HY * HX + NT - 1) / NT;
   constexpr int NR = (TY * HX + NT - 1) / NT;
   constexpr int NQ = (HY * TX + NT - 1) / NT;
-  __shared__ double sW[5][HY][HX];
-  __shared__ double sR[2][TY][HX];
-  __shared__ double sQ[2][HY][TX];
-  const int4 td = tiles[linear_tile(1)];
+  double (*sW)[HY][HX] = reinterpret_cast<double (*)[HY][HX]>(smem);
+  double (*sR)[TY][HX] = reinterpret_cast<double (*)[TY][HX]>(smem + 8 * 5 * HY * HX);
+  double (*sQ)[HY][TX] = reinterpret_cast<double (*)[HY][TX]>(smem + 8 * (5 * HY + 2 * TY) * HX);
   const int bu = td.x, i0 = td.y, j0 = td.z;
   ConstBlockDev* B4 = (ConstBlockDev*)a.blocks + bu;
   const double rho = B4->rho, Gm = B4->G, Mm = B4->M, gam = B4->gamma;
@@ -543,7 +564,7 @@ struct AdjEdgeArgs {
   const double* mu;  // mu of this stage (5 planes)
   int ld;
   long long ps;
-  const int2* tasks;
+  const EdgeNode* nodes;
   int ntasks;
   const BlockDev* blocks;
   SidesDev sd;
@@ -562,29 +583,21 @@ __device__ __forceinline__ void load_mu(const AdjEdgeArgs& a, long long cc, doub
   mu[5] = 0.0;
 }
 
-__device__ __forceinline__ void store_gE(const AdjEdgeArgs& a, int so, const double* lF,
-                                         const double* ldd) {
-#pragma unroll
-  for (int l = 0; l < 5; l++) a.gE[l * a.sd.NS + so] = lF[l] - ldd[l];
-}
-
-__global__ void __launch_bounds__(64) adj_edge_kernel(AdjEdgeArgs a) {
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= a.ntasks) return;
-  const int2 task = a.tasks[tid];
+// gE of one edge node, Gm of its minus side (a boundary node's only one) and
+// Gp of its plus side, with the state variables and gradients of a
+// frictional node updated
+__device__ __forceinline__ void adj_edge_node(const AdjEdgeArgs& a, const EdgeNode& nd, double (&Gm)[5],
+                                              double (&Gp)[5]) {
   const int NS = a.sd.NS;
-  if (task.x >= 0) {
+  auto put = [](double (&G)[5], const double* lF, const double* ldd) {
+#pragma unroll
+    for (int l = 0; l < 5; l++) G[l] = lF[l] - ldd[l];
+  };
+  if (nd.iface < 0) {
     // boundary node: SAT and set_bc_mode2 transposed
-    const int b = task.x >> 2, s = task.x & 3, k = task.y;
-    const BlockDev& B = a.blocks[b];
-    int i, j;
-    if (s == FDM_SIDE_L) { i = B.mx; j = B.my + k; }
-    else if (s == FDM_SIDE_R) { i = B.px; j = B.my + k; }
-    else if (s == FDM_SIDE_B) { i = B.mx + k; j = B.my; }
-    else { i = B.mx + k; j = B.py; }
-    const int so = B.side_off[s] + k;
+    const int so = nd.som;
     double mu[6], ldd[6], lF[6];
-    load_mu(a, (long long)j * a.ld + i, mu);
+    load_mu(a, nd.ccm, mu);
     sat_T(mu, a.sd, so, ldd);
     const double n1 = a.sd.normal[so], n2 = a.sd.normal[NS + so];
     const double Zs = a.sd.M[so], Zp = a.sd.M[NS + so], gamma = a.sd.M[2 * NS + so];
@@ -595,35 +608,22 @@ __global__ void __launch_bounds__(64) adj_edge_kernel(AdjEdgeArgs a) {
     lf.szz = lh.szz;
     const double lsnn = lh.snn + gamma * (lh.stt + lh.szz);
     double cvv, cvs, csv, css;
-    bc_coef(B.side_bc[s], cvv, cvs, csv, css);
+    bc_coef(nd.sop, cvv, cvs, csv, css);
     lf.vt = cvv * lh.vt + csv * Zs * lh.snt;
     lf.snt = cvs * Zsi * lh.vt + css * lh.snt;
     lf.vn = cvv * lh.vn + csv * Zp * lsnn;
     lf.snn = cvs * Zpi * lh.vn + css * lsnn - gamma * (lh.stt + lh.szz);
     xy2nt_T(lf, n1, n2, lF);
-    store_gE(a, so, lF, ldd);
+    put(Gm, lF, ldd);
     return;
   }
   // interface node
-  const IfaceDev& I = a.fi.tab[-task.x - 1];
-  const int k = task.y, g = I.m + k, q = I.node_off + k;
+  const IfaceDev& I = a.fi.tab[nd.iface];
+  const int q = nd.q, som = nd.som, sop = nd.sop;
   const int NI = a.fi.NI;
-  const BlockDev& Bm = a.blocks[I.bm];
-  const BlockDev& Bp = a.blocks[I.bp];
-  int im, jm, ip, jp, km, kp, sm, sp;
-  if (I.direction == 0) {
-    sm = FDM_SIDE_R; sp = FDM_SIDE_L;
-    im = Bm.px; jm = g; ip = Bp.mx; jp = g;
-    km = g - Bm.my; kp = g - Bp.my;
-  } else {
-    sm = FDM_SIDE_T; sp = FDM_SIDE_B;
-    im = g; jm = Bm.py; ip = g; jp = Bp.my;
-    km = g - Bm.mx; kp = g - Bp.mx;
-  }
-  const int som = Bm.side_off[sm] + km, sop = Bp.side_off[sp] + kp;
   double mum[6], mup[6], lddm[6], lddp[6];
-  load_mu(a, (long long)jm * a.ld + im, mum);
-  load_mu(a, (long long)jp * a.ld + ip, mup);
+  load_mu(a, nd.ccm, mum);
+  load_mu(a, nd.ccp, mup);
   sat_T(mum, a.sd, som, lddm);
   sat_T(mup, a.sd, sop, lddp);
   const double n1 = a.fi.nhat[q], n2 = a.fi.nhat[NI + q];
@@ -699,8 +699,106 @@ __global__ void __launch_bounds__(64) adj_edge_kernel(AdjEdgeArgs a) {
   double lFp[6], lFm[6];
   xy2nt_T(lp, n1, n2, lFp);
   xy2nt_T(lm, n1, n2, lFm);
-  store_gE(a, sop, lFp, lddp);
-  store_gE(a, som, lFm, lddm);
+  put(Gp, lFp, lddp);
+  put(Gm, lFm, lddm);
+}
+
+// the edge nodes in a launch of their own, for the per-point kernel
+__global__ void __launch_bounds__(64) adj_edge_kernel(AdjEdgeArgs a) {
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+  if (tid >= a.ntasks) return;
+  const EdgeNode nd = a.nodes[tid];
+  double Gm[5], Gp[5];
+  adj_edge_node(a, nd, Gm, Gp);
+#pragma unroll
+  for (int l = 0; l < 5; l++) a.gE[l * a.sd.NS + nd.som] = Gm[l];
+  if (nd.iface >= 0) {
+#pragma unroll
+    for (int l = 0; l < 5; l++) a.gE[l * a.sd.NS + nd.sop] = Gp[l];
+  }
+}
+
+// A rim group (fdm_bulk.hpp): the first wave evaluates the group's edge nodes
+// into LDS while the others gather their points' stencil rows; after the
+// barrier these add the edge contributions and finish the points.
+__device__ __forceinline__ void adj_rim_group(const AdjBulkArgs& a, const AdjEdgeArgs& e, const int4 g,
+                                              const EdgeNode* __restrict__ nodes, const RimPt* __restrict__ pts,
+                                              const int tid, double (*sG)[5]) {
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  if (wave == 0) {
+    if (lane < g.x) {
+      const EdgeNode nd = nodes[lane];
+      const int stride = g.z ? kRimIface : kRimNodes;
+      double Gm[5], Gp[5];
+      adj_edge_node(e, nd, Gm, Gp);
+#pragma unroll
+      for (int l = 0; l < 5; l++) sG[lane][l] = Gm[l];
+      if (nd.iface >= 0) {
+#pragma unroll
+        for (int l = 0; l < 5; l++) sG[stride + lane][l] = Gp[l];
+      }
+    }
+    __syncthreads();
+    return;
+  }
+  const int k = (tid - 64) >> 1;  // both lanes of a pair go together
+  const bool q = (tid & 1) == 0, active = k < g.y;
+  const RimPt P = pts[active ? k : 0];
+  double w[5];
+  if (active) adj_pair(a, a.blocks[P.p.blk], P.p.i, P.p.j, q, w);
+  __syncthreads();
+  if (!active || !q) return;
+  if (P.soA >= 0 && P.slotA >= 0) {
+#pragma unroll
+    for (int l = 0; l < 5; l++) w[l] += sG[P.slotA][l];
+  }
+  if (P.soB >= 0 && P.slotB >= 0) {
+#pragma unroll
+    for (int l = 0; l < 5; l++) w[l] += sG[P.slotB][l];
+  }
+  adj_finish(a, (long long)P.p.j * a.ld + P.p.i, w);
+}
+
+// A backward stage in one launch: rim groups, the other points within six of
+// a block edge (128 a workgroup), then the interior tiles, under which the
+// latency of the first two passes.  Against an edge, a band and an interior
+// kernel on two streams joined by events twice a stage, 2 x 801x401 points:
+// 43 -> 33 us a stage, 29.5 of them the kernel.  Three waves per SIMD hold the
+// edge node's and the pair's registers; four spill them.
+struct AdjLists {
+  const int4* rim;
+  const EdgeNode* rimnodes;
+  const RimPt* rimpts;
+  int nrim;
+  const BandPt* band;
+  int nband, nbandwg;
+  const int4* tiles;
+};
+
+template <int TX, int TY, bool NTS>
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(3))) adj_stage_kernel(AdjBulkArgs a, AdjEdgeArgs e, AdjLists L) {
+  static_assert(2 * BandLanes<2>::group <= TX * TY - 64, "a rim group's points on the waves after the first");
+  static_assert(adj_tile_bytes<TX, TY>() >= 8 * 5 * kRimHats, "a rim group's hats in the tile's LDS");
+  __shared__ __attribute__((aligned(16))) char smem[adj_tile_bytes<TX, TY>()];
+  const int tid = threadIdx.y * TX + threadIdx.x;
+  int wb = blockIdx.x;
+  if (wb < L.nrim) {
+    adj_rim_group(a, e, L.rim[wb], L.rimnodes + wb * kRimNodes, L.rimpts + wb * kRimPts, tid,
+                  reinterpret_cast<double (*)[5]>(smem));
+    return;
+  }
+  wb -= L.nrim;
+  if (wb < L.nbandwg) {
+    const int t = wb * TX * TY + tid, k = t >> 1;
+    if (k >= L.nband) return;  // both lanes of a pair leave together
+    const BandPt p = L.band[k];
+    const bool q = (t & 1) == 0;
+    double g[5];
+    adj_pair(a, a.blocks[p.blk], p.i, p.j, q, g);
+    if (q) adj_finish(a, (long long)p.j * a.ld + p.i, g);
+    return;
+  }
+  adj_tile<TX, TY, NTS>(a, L.tiles[linear_tile(1, L.nrim + L.nbandwg)], smem);
 }
 
 // lambda_F += g and mu += b g at the receivers: one lane per distinct grid
@@ -748,14 +846,14 @@ struct fdm_adjoint {
   double* lpsi = nullptr;        // [NI]
   double* ldpsi = nullptr;       // [NI]
   double* grad = nullptr;        // [FDM_GRAD_NFIELDS][NI]
-  // bulk adjoint: interior tiles (64 x 4) of [mx+6, px-6] x [my+6, py-6]
-  // on the main stream, the other points on the side stream after the edge
-  // adjoint; or one per-point kernel (FDM_ADJ_BULK=generic)
+  // bulk adjoint: the stage launch (contexts whose forward stages are one),
+  // with interior tiles (64 x 4) of [mx+6, px-6] x [my+6, py-6]; or an edge and
+  // a per-point kernel (FDM_ADJ_BULK=generic)
   bool tiled = true;
   bool nt_store = false;  // adjoint planes and metrics beyond the last-level cache
   int4* tiles = nullptr;
   int ntiles = 0;
-  int2* band = nullptr;
+  BandPt* band = nullptr;
   int nband = 0;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   double ms_fwd = 0.0, ms_rec = 0.0, ms_sweep = 0.0;
@@ -843,24 +941,22 @@ int adj_stage(fdm_adjoint* a, int n, int s, int& cur) {
   const double A = c->rkA[s - 1], Bdt = c->rkB[s - 1] * a->dt;
   const double Bprev = (s > 1 ? c->rkB[s - 2] : c->rkB[ns - 1]) * a->dt;
   AdjEdgeArgs e;
-  if (c->ntasks) {
-    e.mu = a->mu[cur];
-    e.ld = c->ld;
-    e.ps = c->ps;
-    e.tasks = c->tasks;
-    e.ntasks = c->ntasks;
-    e.blocks = c->blocks;
-    e.sd = SidesDev{c->sM, c->snormal, c->sF0, c->sx, c->sy, c->sFhat, c->NS};
-    e.fi = IfacesDev{c->ifaces, c->inhat, c->irs, c->isw, c->iS0b, c->iN0b, c->ildS, c->ildN,
-                     c->iout, c->iknx, c->ist, c->ist1, c->NI};
-    e.trace = a->trace + ((size_t)((n - 1) % K) * ns + (s - 1)) * 3 * c->NI;
-    e.lpsi = a->lpsi;
-    e.ldpsi = a->ldpsi;
-    e.grad = a->grad;
-    e.gE = a->gE;
-    e.A = A;
-    e.Bdt = Bdt;
-  }
+  e.mu = a->mu[cur];
+  e.ld = c->ld;
+  e.ps = c->ps;
+  e.nodes = c->nodes;
+  e.ntasks = c->ntasks;
+  e.blocks = c->blocks;
+  e.sd = SidesDev{c->sM, c->snormal, c->sF0, c->sx, c->sy, c->sFhat, c->NS};
+  e.fi = IfacesDev{c->ifaces, c->inhat, c->irs, c->isw, c->iS0b, c->iN0b, c->ildS, c->ildN,
+                   c->iout, c->iknx, c->ist, c->ist1, c->NI};
+  e.trace = a->trace + ((size_t)((n - 1) % K) * ns + (s - 1)) * 3 * c->NI;
+  e.lpsi = a->lpsi;
+  e.ldpsi = a->ldpsi;
+  e.grad = a->grad;
+  e.gE = a->gE;
+  e.A = A;
+  e.Bdt = Bdt;
   AdjBulkArgs b;
   b.lin = a->lF[cur];
   b.lout = a->lF[1 - cur];
@@ -885,27 +981,10 @@ int adj_stage(fdm_adjoint* a, int n, int s, int& cur) {
   b.A = A;
   b.Bdt_prev = Bprev;
   if (a->tiled) {
-    // The interior points read mu of this stage within two points (the band
-    // of the later stage wrote it there) and overwrite the buffer the later
-    // stage's band read; the band reads mu within five points (the later
-    // interior launch) and needs this stage's edge adjoint.
-    ADJCHK(a, hipStreamWaitEvent(c->stream, c->evB, 0));
-    if (a->ntiles) {
-      if (a->nt_store)
-        hipLaunchKernelGGL((adj_interior_kernel<64, 4, true>), dim3(a->ntiles), dim3(64, 4), 0, c->stream,
-                           b, a->tiles);
-      else
-        hipLaunchKernelGGL((adj_interior_kernel<64, 4, false>), dim3(a->ntiles), dim3(64, 4), 0, c->stream,
-                           b, a->tiles);
-    }
-    if (c->ntasks)
-      hipLaunchKernelGGL(adj_edge_kernel, dim3((c->ntasks + 63) / 64), dim3(64), 0, c->side, e);
-    ADJCHK(a, hipStreamWaitEvent(c->side, c->evI, 0));
-    if (a->nband)
-      hipLaunchKernelGGL(adj_band_kernel, dim3((2 * a->nband + 63) / 64), dim3(64), 0, c->side, b,
-                         a->band, a->nband);
-    ADJCHK(a, hipEventRecord(c->evB, c->side));
-    ADJCHK(a, hipEventRecord(c->evI, c->stream));
+    const AdjLists L{c->rim, c->rimnodes, c->rimpts, c->nrim, a->band, a->nband, (2 * a->nband + 255) / 256, a->tiles};
+    const dim3 grid(L.nrim + L.nbandwg + a->ntiles), block(64, 4);
+    if (a->nt_store) hipLaunchKernelGGL((adj_stage_kernel<64, 4, true>), grid, block, 0, c->stream, b, e, L);
+    else hipLaunchKernelGGL((adj_stage_kernel<64, 4, false>), grid, block, 0, c->stream, b, e, L);
   } else {
     if (c->ntasks)
       hipLaunchKernelGGL(adj_edge_kernel, dim3((c->ntasks + 63) / 64), dim3(64), 0, c->stream, e);
@@ -1020,27 +1099,27 @@ int fdm_adjoint_create(fdm_ctx* c, int32_t nrec, const int32_t* rec_i, const int
   // 32-bit
   if (const char* v = getenv("FDM_ADJ_BULK")) a->tiled = strcmp(v, "generic") != 0;
   a->nt_store = nt_store_choice(25.0 * (double)c->ps * 8.0);
-  if ((size_t)c->ps * 8 >= ((size_t)1 << 31)) a->tiled = false;
+  if ((size_t)c->ps * 8 >= ((size_t)1 << 31) || !c->fused) a->tiled = false;
   if (a->tiled) {
     std::vector<int4> tl;
-    std::vector<int2> band;
+    std::vector<BandPt> band;  // the edge points themselves are in the rim groups
     for (int b = 0; b < c->nb; b++) {
       const BlockDev& B = c->hblocks[b];
       for (int j0 = B.my + 6; j0 <= B.py - 6; j0 += 4)
         for (int i0 = B.mx + 6; i0 <= B.px - 6; i0 += 64) tl.push_back(make_int4(b, i0, j0, 0));
-      for (int j = B.my; j <= B.py; j++)
-        for (int i = B.mx; i <= B.px; i++)
-          if (i - B.mx < 6 || B.px - i < 6 || j - B.my < 6 || B.py - j < 6) band.push_back(make_int2(i, j));
+      for (int j = B.my + 1; j < B.py; j++)
+        for (int i = B.mx + 1; i < B.px; i++)
+          if (i - B.mx < 6 || B.px - i < 6 || j - B.my < 6 || B.py - j < 6) band.push_back(BandPt{i, j, b, 0u});
     }
     a->ntiles = (int)tl.size();
     a->nband = (int)band.size();
     rc = adj_alloc(a, &a->tiles, tl.size() * sizeof(int4));
-    if (!rc) rc = adj_alloc(a, &a->band, band.size() * sizeof(int2));
+    if (!rc) rc = adj_alloc(a, &a->band, band.size() * sizeof(BandPt));
     if (!rc && a->ntiles &&
         hipMemcpy(a->tiles, tl.data(), tl.size() * sizeof(int4), hipMemcpyHostToDevice) != hipSuccess)
       rc = adj_err(a, FDM_EDEVICE, "fdm_adjoint_create: upload failed");
     if (!rc && a->nband &&
-        hipMemcpy(a->band, band.data(), band.size() * sizeof(int2), hipMemcpyHostToDevice) != hipSuccess)
+        hipMemcpy(a->band, band.data(), band.size() * sizeof(BandPt), hipMemcpyHostToDevice) != hipSuccess)
       rc = adj_err(a, FDM_EDEVICE, "fdm_adjoint_create: upload failed");
     if (rc) {
       g_create_error = a->err;
@@ -1129,33 +1208,17 @@ int fdm_adjoint_backward(fdm_adjoint* a, const double* rec_bar, double* grad, do
       if (rc) return rc;
     }
     ADJCHK(a, hipEventRecord(a->ev[1], c->stream));
-    if (a->tiled) {
-      const int rf = fork_side(c);
-      if (rf) return adj_err(a, rf, c->err);
-    }
     for (int n = n1; n >= n0; n--) {
       if (a->nrec) {
-        // after both streams' last writes of the later step, before either
-        // reads this step's last stage
-        hipStream_t sr = c->stream;
-        if (a->tiled) {
-          ADJCHK(a, hipStreamWaitEvent(c->side, c->evI, 0));
-          sr = c->side;
-        }
-        hipLaunchKernelGGL(adj_inject_kernel, dim3((a->nuniq + 63) / 64), dim3(64), 0, sr, a->lF[cur],
+        hipLaunchKernelGGL(adj_inject_kernel, dim3((a->nuniq + 63) / 64), dim3(64), 0, c->stream, a->lF[cur],
                            a->mu[cur], c->ps, a->rec_cc, a->rec_first, a->rec_order, a->nuniq,
                            a->rec_bar + (size_t)(n - 1) * a->nrec * 2, b_last);
         ADJCHK(a, hipGetLastError());
-        if (a->tiled) ADJCHK(a, hipEventRecord(c->evB, c->side));
       }
       for (int s = ns; s >= 1; s--) {
         int rc = adj_stage(a, n, s, cur);
         if (rc) return rc;
       }
-    }
-    if (a->tiled) {
-      const int rj = join_side(c);
-      if (rj) return adj_err(a, rj, c->err);
     }
     ADJCHK(a, hipEventRecord(a->ev[2], c->stream));
     ADJCHK(a, hipEventSynchronize(a->ev[2]));

@@ -90,8 +90,7 @@ struct fdm_ctx {
   std::vector<double> ld_T;  // per interface
   // edge tasks
   int ntasks = 0;
-  int2* tasks = nullptr;
-  EdgeNode* nodes = nullptr;  // the same tasks, resolved
+  EdgeNode* nodes = nullptr;
   // the stage launch (every context without a layer, with the tile kernels):
   // rim groups, their nodes and points, and the inner band points
   bool fused = false;
@@ -1580,8 +1579,6 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     if ((rc = dupload(c, &c->ist1, st.data(), st.size() * 8))) return fail(rc);
   }
   c->ntasks = (int)tasks.size();
-  if ((rc = dupload(c, &c->tasks, tasks.data(), std::max<size_t>(1, tasks.size()) * sizeof(int2))))
-    return fail(rc);
   c->htasks = tasks;
 
   // ---- source ----
