@@ -138,11 +138,16 @@ struct fdm_ctx {
   // Wy, DWx, DWy, 6 planes each (field precision, plane stride ps)
   bool pml = false, pml_wx = false, pml_wy = false;
   void* W = nullptr;
-  // the points of the layer blocks, row-major within each block: those four
-  // or more from every edge of their block (lpts[0]) and the rest (lpts[1])
-  int2* lpts[2] = {nullptr, nullptr};
-  int nlpts[2] = {0, 0};
-  long long nlayer_inner = 0;  // lpts[0] entries that are points (not padding)
+  // the points of the layer blocks within four of an edge of their block
+  // (lpts), and the tiles of the others (bulk_layer; hltiles: on the host,
+  // without padding)
+  int2* lpts = nullptr;
+  int nlpts = 0;
+  int4* ltiles = nullptr;
+  int nltiles = 0;
+  std::vector<int4> hltiles;
+  long long nlayer_inner = 0;  // points of the layer tiles
+  int layer_all = 0;           // BulkArgs::layer_all
   // 2: plane strain, 6 fields; 3: antiplane shear, 3 fields
   int mode = 2, nF = 6;
   // first-derivative operator SBP2/4/6 (fd_coeff.f90:41-248) and its
@@ -450,6 +455,7 @@ BulkArgs<T> bulk_args(fdm_ctx* c, double A, double Bdt, int do_update, double t,
   a.rout = nullptr;
   a.nrec = 0;
   a.nrecwg = 0;
+  a.layer_all = c->layer_all;
   return a;
 }
 
@@ -479,26 +485,30 @@ void launch_band(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
   prof_end(c, ep, 2, s);
 }
 
-template <typename T, bool INNER>
-void launch_layer_list(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a, int q) {
-  EventPair* ep = prof_begin(c, INNER ? 0 : 2, s);
-  dim3 grid((c->nlpts[q] + 255) / 256), block(256);
-  if (full_variant(c, a))
-    hipLaunchKernelGGL((bulk_pml<T, true, INNER, false>), grid, block, 0, s, a, c->lpts[q], c->nlpts[q]);
-  else if (c->nt_store)
-    hipLaunchKernelGGL((bulk_pml<T, false, INNER, true>), grid, block, 0, s, a, c->lpts[q], c->nlpts[q]);
-  else
-    hipLaunchKernelGGL((bulk_pml<T, false, INNER, false>), grid, block, 0, s, a, c->lpts[q], c->nlpts[q]);
-  prof_end(c, ep, INNER ? 0 : 2, s);
+// the layer points near block edges, after the band on the same stream (they
+// need this stage's edge values); timed with the band
+template <typename T>
+void launch_layer_edges(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
+  if (!c->nlpts) return;
+  EventPair* ep = prof_begin(c, 2, s);
+  dim3 grid((c->nlpts + 63) / 64), block(64);
+  if (full_variant(c, a)) hipLaunchKernelGGL((bulk_pml<T, true>), grid, block, 0, s, a, c->lpts, c->nlpts);
+  else hipLaunchKernelGGL((bulk_pml<T, false>), grid, block, 0, s, a, c->lpts, c->nlpts);
+  prof_end(c, ep, 2, s);
 }
 
-// the layer points, after the band on the same stream (their boundary
-// points need this stage's edge values); the inner points are timed with
-// the interior launches, the rest with the band
+// the other layer points, which need no edge value: timed with the interior
 template <typename T>
-void launch_layer(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
-  if (c->nlpts[0]) launch_layer_list<T, true>(c, s, a, 0);
-  if (c->nlpts[1]) launch_layer_list<T, false>(c, s, a, 1);
+void launch_layer_tiles(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
+  if (!c->nltiles) return;
+  const bool full = full_variant(c, a);
+  c->df6_stale = !full;
+  EventPair* ep = prof_begin(c, 0, s);
+  dim3 grid(c->nltiles), block(64, 4);
+  if (full) hipLaunchKernelGGL((bulk_layer<T, true, false>), grid, block, 0, s, a, c->ltiles);
+  else if (c->nt_store) hipLaunchKernelGGL((bulk_layer<T, false, true>), grid, block, 0, s, a, c->ltiles);
+  else hipLaunchKernelGGL((bulk_layer<T, false, false>), grid, block, 0, s, a, c->ltiles);
+  prof_end(c, ep, 0, s);
 }
 
 // Inner band points: one lane per (point, field), or one lane per point?
@@ -661,11 +671,12 @@ int run_stage(fdm_ctx* c, int stage, double t0, double dt, int final_step, int s
     // interior launch.
     HIPCHK(c, hipStreamWaitEvent(c->stream, c->evB, 0));
     launch_interior<T>(c, c->stream, a, e);
+    launch_layer_tiles<T>(c, c->stream, a);
     rc = launch_edges<T>(c, c->side, e);
     if (rc) return rc;
     HIPCHK(c, hipStreamWaitEvent(c->side, c->evI, 0));
     launch_band<T>(c, c->side, a);
-    launch_layer<T>(c, c->side, a);
+    launch_layer_edges<T>(c, c->side, a);
     HIPCHK(c, hipEventRecord(c->evB, c->side));
     HIPCHK(c, hipEventRecord(c->evI, c->stream));
   } else {
@@ -846,6 +857,72 @@ int check_fail(fdm_ctx* c) {
 }  // namespace
 
 namespace {
+
+// A block's layer in effect: all of its points go to the layer lists.
+bool layer_block(const fdm_block& B) { return (B.pmlx || B.pmly) && !(B.Cdiss > 0.0); }
+
+// Tiles of the layer blocks' points four or more from every edge of their
+// block (bulk_layer), each with the directions that damp some point of it.
+// The order puts a run of neighbours on each XCD (whose L2 then holds the rows
+// a stencil shares) and an equal share of each kind: tiles with auxiliary
+// fields move two or three times the bytes and lie together at the rims.
+int layer_tiles(fdm_ctx* c, const fdm_problem* P) {
+  std::vector<int4> kind[4];
+  for (int b = 0; b < c->nb; b++) {
+    const fdm_block& B = P->blocks[b];
+    if (!layer_block(B)) continue;
+    const int ia = B.mx + 4, ib = B.px - 4, ja = B.my + 4, jb = B.py - 4;
+    if (ia > ib || ja > jb) continue;
+    c->nlayer_inner += (long long)(ib - ia + 1) * (jb - ja + 1);
+    // a direction may be left out where its profile (pml_rates) is zero at
+    // every point, if zeros then stay zeros: finite factors, and a first
+    // stage that starts its rates afresh
+    const double* p = B.pml;
+    const bool graded = p[0] > 0.0 && P->x && P->y && std::isfinite(p[1]) && std::isfinite(p[2]) && P->rkA[0] == 0.0;
+    auto damped = [&](const double* at, double lo, double hi, int i0, int j0) {
+      if (!graded) return true;
+      for (int j = j0; j < j0 + 4 && j <= jb; j++)
+        for (int i = std::max(i0, ia); i < i0 + 64 && i <= ib; i++) {
+          const double v = at[(size_t)j * P->nx + i];
+          if (!(v >= lo && v <= hi)) return true;
+        }
+      return false;
+    };
+    for (int j0 = ja; j0 <= jb; j0 += 4)
+      for (int i0 = ia - (ia + c->coff) % 64; i0 <= ib; i0 += 64) {
+        const int w = (B.pmlx && damped(P->x, p[3], p[4], i0, j0) ? 1 : 0) |
+                      (B.pmly && damped(P->y, p[5], p[6], i0, j0) ? 2 : 0);
+        kind[w].push_back(make_int4(b, i0, j0, w));
+      }
+  }
+  std::vector<int4> seq[8], list;
+  for (int w = 3; w >= 0; w--) {
+    c->hltiles.insert(c->hltiles.end(), kind[w].begin(), kind[w].end());
+    const size_t n = kind[w].size();
+    for (size_t x = 0; x < 8; x++)
+      seq[x].insert(seq[x].end(), kind[w].begin() + x * n / 8, kind[w].begin() + (x + 1) * n / 8);
+  }
+  size_t most = 0;
+  for (auto& q : seq) most = std::max(most, q.size());
+  for (size_t k = 0; k < most; k++)
+    for (auto& q : seq) list.push_back(k < q.size() ? q[k] : make_int4(-1, 0, 0, 0));
+  c->nltiles = (int)list.size();
+  return c->nltiles ? dupload(c, &c->ltiles, list.data(), list.size() * sizeof(int4)) : FDM_OK;
+}
+
+// whether the caller's Wx (dir 0) or Wy (dir 1) is nonzero at a point of a
+// layer tile that leaves the direction out
+bool layer_needs(const fdm_ctx* c, int dir, const double* W) {
+  for (const int4& t : c->hltiles) {
+    const BlockDev& B = c->hblocks[t.x];
+    if ((t.w >> dir & 1) || !(dir ? B.pmly : B.pmlx)) continue;
+    for (int l = 0; l < 6; l++)
+      for (int j = t.z; j < t.z + 4 && j <= B.py - 4; j++)
+        for (int i = std::max(t.y, B.mx + 4); i < t.y + 64 && i <= B.px - 4; i++)
+          if (W[((size_t)l * c->ny + j) * c->nx + i] != 0.0) return true;
+  }
+  return false;
+}
 
 // Work lists of the edges: the tasks resolved into EdgeNode records, and for
 // contexts without a layer the rim groups and inner band points of the stage
@@ -1242,11 +1319,10 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     // covered from its corner, x fastest; band: every other point, row-major.
     // A block with a perfectly matched layer in effect has no tiles and no
     // band: all of its points go to the layer list.
-    auto layer = [&](const fdm_block& B) { return (B.pmlx || B.pmly) && !(B.Cdiss > 0.0); };
     std::vector<int4> tl[3];
     for (int b = 0; b < c->nb; b++) {
       const fdm_block& B = P->blocks[b];
-      if (layer(B)) continue;
+      if (layer_block(B)) continue;
       const int ia = B.mx + nbst, ib = B.px - nbst, ja = B.my + nbst, jb = B.py - nbst;
       if (ia > ib || ja > jb) continue;
       c->ninterior += (long long)(ib - ia + 1) * (jb - ja + 1);
@@ -1264,40 +1340,20 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
           for (int i0 = ia; i0 <= ib; i0 += tx) tl[q].push_back(make_int4(b, i0, j0, reached(i0, j0, tx, ty)));
       }
     }
-    std::vector<int2> band, lpts[2];
+    std::vector<int2> band, lpts;
     for (int j = 0; j < P->ny; j++)
       for (int i = 0; i < P->nx; i++) {
         const fdm_block& B = P->blocks[block_of(c, i, j)];
         const bool edge = i - B.mx < nbst || B.px - i < nbst || j - B.my < nbst || B.py - j < nbst;
-        if (c->mode == 2 && layer(B)) {
-          if (edge) lpts[1].push_back(make_int2(i, j));
+        if (c->mode == 2 && layer_block(B)) {
+          if (edge) lpts.push_back(make_int2(i, j));
         } else if (edge) {
           band.push_back(make_int2(i, j));
         }
       }
-    // inner layer points: each row of a layer block's interior in runs of
-    // 64 that start where the stored planes are 64-element aligned
-    // ((i + coff) % 64 == 0), padded with (-1, -1) entries that do nothing
-    for (int b = 0; b < c->nb; b++) {
-      const fdm_block& B = P->blocks[b];
-      if (c->mode != 2 || !layer(B)) continue;
-      const int ia = B.mx + 4, ib = B.px - 4;
-      if (ia > ib) continue;
-      const int i0 = ia - (ia + c->coff) % 64;
-      const int i1 = ib + 1 + (64 - (ib + 1 + c->coff) % 64) % 64;
-      // count the points as they are pushed: a block with fewer than
-      // nine rows has no inner rows at all
-      for (int j = B.my + 4; j <= B.py - 4; j++) {
-        for (int i = i0; i < i1; i++)
-          lpts[0].push_back(i >= ia && i <= ib ? make_int2(i, j) : make_int2(-1, -1));
-        c->nlayer_inner += ib - ia + 1;
-      }
-    }
-    for (int q = 0; q < 2; q++) {
-      c->nlpts[q] = (int)lpts[q].size();
-      if (c->nlpts[q] && (rc = dupload(c, &c->lpts[q], lpts[q].data(), lpts[q].size() * sizeof(int2))))
-        return fail(rc);
-    }
+    c->nlpts = (int)lpts.size();
+    if (c->nlpts && (rc = dupload(c, &c->lpts, lpts.data(), lpts.size() * sizeof(int2)))) return fail(rc);
+    if (c->mode == 2 && (rc = layer_tiles(c, P))) return fail(rc);
     for (int q = 0; q < 3; q++) {
       c->ntiles[q] = (int)tl[q].size();
       if (c->ntiles[q] && (rc = dupload(c, &c->tiles[q], tl[q].data(), tl[q].size() * sizeof(int4))))
@@ -2067,8 +2123,12 @@ int fdm_set_pml(fdm_ctx* c, const double* Wx, const double* Wy) {
     return set_err(c, FDM_EINVAL, "fdm_set_pml: no block has that PML direction");
   HIPCHK(c, hipStreamSynchronize(c->stream));
   int rc;
-  if (Wx && (rc = pml_copy(c, 0, nullptr, Wx))) return rc;
-  if (Wy && (rc = pml_copy(c, 6, nullptr, Wy))) return rc;
+  for (int dir = 0; dir < 2; dir++) {
+    const double* W = dir ? Wy : Wx;
+    if (!W) continue;
+    if ((rc = pml_copy(c, 6 * dir, nullptr, W))) return rc;
+    c->layer_all = (c->layer_all & ~(1 << dir)) | (layer_needs(c, dir, W) ? 1 << dir : 0);
+  }
   return FDM_OK;
 }
 

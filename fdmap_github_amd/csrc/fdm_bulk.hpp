@@ -97,6 +97,8 @@ struct BulkArgs {
   const long long* rcc;
   double* rout;
   int nrec, nrecwg;
+  // layer contexts: bit 0 (1) carries Wx (Wy) in every layer tile (bulk_layer)
+  int layer_all;
 };
 
 // Map the hardware workgroup id to a tile.  Workgroups are dispatched to the
@@ -726,10 +728,11 @@ __device__ __forceinline__ void pml_yterm(T (&d)[6], T (&dw)[6], const T (&v)[6]
 // rates are scaled by A and the fields updated in place (fields.f90:
 // 1074-1077, 1181-1184): each lane touches only its own point's W.
 // INNER = true compiles the interior form alone (points four or more from
-// every edge of their block, where no SAT applies).
-template <typename T, bool INNER = false>
-__device__ __forceinline__ void pml_rates(const BulkArgs<T>& a, const BlockDev& B, const int i, const int j,
-                                          const long long cc, T (&d)[6]) {
+// every edge of their block, where no SAT applies).  onx, ony: whether the
+// point has Wx, Wy; a direction left out adds nothing to d.
+template <typename T, bool INNER = false, typename BlockRef>
+__device__ __forceinline__ void pml_rates(const BulkArgs<T>& a, BlockRef& B, const int i, const int j,
+                                          const long long cc, T (&d)[6], const bool onx, const bool ony) {
   const long long ps = a.ps;
   const int ld = a.ld;
   const T* __restrict__ F = a.Fin;
@@ -750,13 +753,17 @@ __device__ __forceinline__ void pml_rates(const BulkArgs<T>& a, const BlockDev& 
   double sxd = B.pml[1], syd = B.pml[1];
   if (B.pml[0] > 0.0) {
     const long long pc = (long long)j * a.nx + i;
-    const double x = a.X[pc], y = a.Y[pc];
-    sxd = B.pml[1] * pow(fabs(fmax(0.0, fmax(B.pml[3] - x, x - B.pml[4]))), B.pml[0]);
-    syd = B.pml[1] * pow(fabs(fmax(0.0, fmax(B.pml[5] - y, y - B.pml[6]))), B.pml[0]);
+    if (onx) {
+      const double x = a.X[pc];
+      sxd = B.pml[1] * pow(fabs(fmax(0.0, fmax(B.pml[3] - x, x - B.pml[4]))), B.pml[0]);
+    }
+    if (ony) {
+      const double y = a.Y[pc];
+      syd = B.pml[1] * pow(fabs(fmax(0.0, fmax(B.pml[5] - y, y - B.pml[6]))), B.pml[0]);
+    }
   }
   const T sx = (T)sxd, sy = (T)syd, kap = (T)B.pml[2];
   const T rho = (T)B.rho, G = (T)B.G, M = (T)B.M, gamma = (T)B.gamma;
-  const bool onx = B.pmlx != 0, ony = B.pmly != 0;
   T* __restrict__ W = a.W;
   const T A = (T)a.A;
   T dwx[6], dwy[6];
@@ -928,7 +935,7 @@ __device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i,
     // the perfectly matched layer and artificial dissipation are built for
     // SBP4 only (fdm_create refuses them with the other operators)
     if (PML && (B.pmlx | B.pmly)) {
-      pml_rates<T>(a, B, i, j, cc, d);
+      pml_rates<T>(a, B, i, j, cc, d, B.pmlx != 0, B.pmly != 0);
       done = true;
     } else if (EXT && B.Cdiss > 0.0 && i - B.mx >= 4 && B.px - i >= 4 && j - B.my >= 4 &&
                B.py - j >= 4) {
@@ -1906,33 +1913,80 @@ __global__ void __launch_bounds__(64) bulk_band(BulkArgs<T> a, const int2* __res
   point_generic<T, FULL, EXT, OP>(a, p.x, p.y, block_at(a, p.x, p.y));
 }
 
-// Layer kernel: the points of the perfectly matched layer blocks, one lane
-// each, from a list that runs row by row through each block (consecutive
-// lanes read consecutive addresses; entries with x < 0 pad the inner list
-// to aligned runs of 64).  It carries only the layer's code;
-// INNER = true serves the points four or more from every block edge with
-// the interior form alone, which keeps more waves in flight.  NTS: F and
-// DF stored non-temporally (working set beyond the last-level cache).
-template <typename T, bool FULL, bool INNER, bool NTS>
+// The points of the perfectly matched layer blocks within four points of an
+// edge of their block, one lane each.
+template <typename T, bool FULL>
 __global__ void __launch_bounds__(256) bulk_pml(BulkArgs<T> a, const int2* __restrict__ pts, int npts) {
-  // the list runs row by row: with the XCD swizzle each XCD takes a
-  // contiguous run of it, so the rows a stencil shares are fetched into one
-  // L2 rather than into up to five
-  const int k = linear_tile(a.xcd_swizzle) * blockDim.x + threadIdx.x;
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= npts) return;
   const int2 p = pts[k];
-  if (p.x < 0) return;  // padding of an aligned run
   const int i = p.x, j = p.y;
   const int bi = a.blk[a.rowb[j] * a.nbx + a.colb[i]];
   const BlockDev& B = a.blocks[bi];
   const long long cc = (long long)j * a.ld + i;
   T d[6];
   scaled_rates<T>(a, cc, d);
-  pml_rates<T, INNER>(a, B, i, j, cc, d);
+  pml_rates<T>(a, B, i, j, cc, d, B.pmlx != 0, B.pmly != 0);
   T Fc[6];
 #pragma unroll
   for (int l = 0; l < 6; l++) Fc[l] = a.Fin[l * a.ps + cc];
-  finish_point<T, FULL, NTS>(a, B, bi, i, j, cc, d, Fc);
+  finish_point<T, FULL>(a, B, bi, i, j, cc, d, Fc);
+}
+
+// The other points of the layer blocks: 64 x 4 tiles (block, i0, j0, w),
+// columns aligned to 64 stored elements, listed in the order of dispatch
+// (block < 0: padding).  Bit 0 (1) of w: Wx (Wy) is carried in the tile.
+// Where a direction's damping is zero its auxiliary fields start at zero and
+// stay there (rates of a zero field without damping and a zero source), so
+// tiles without any damped point in a direction leave out its 24 reads and
+// writes a point; a graded layer damps the rim of its block only.  a.layer_all
+// carries them everywhere, for a caller that has set nonzero ones there.
+// Bound by bytes: 22 values a point a stage, 24 more per direction carried.
+// 2 x 1001x501 points, a fifth of them damped in each direction, with the
+// tiles on the main stream: 184 -> 93 us a stage.
+// NTS: F and DF stored non-temporally (working set beyond the last-level
+// cache).
+template <typename T, bool FULL, bool NTS>
+__global__ void __launch_bounds__(256) bulk_layer(BulkArgs<T> a, const int4* __restrict__ tiles) {
+  const int4 td = tiles[blockIdx.x];
+  if (td.x < 0) return;
+  ConstBlockDev& B = *((ConstBlockDev*)a.blocks + td.x);
+  const int i = td.y + threadIdx.x, j = td.z + threadIdx.y;
+  if (i < B.mx + 4 || i > B.px - 4 || j > B.py - 4) return;
+  const int w = td.w | a.layer_all;
+  const long long cc = (long long)j * a.ld + i, ps = a.ps;
+  T Fc[6];
+#pragma unroll
+  for (int l = 0; l < 6; l++) Fc[l] = a.Fin[l * ps + cc];
+  T d[6];
+  scaled_rates<T>(a, cc, d);
+  pml_rates<T, true>(a, B, i, j, cc, d, B.pmlx != 0 && (w & 1), B.pmly != 0 && (w & 2));
+  if constexpr (FULL) {
+    finish_point<T, true, NTS>(a, a.blocks[td.x], td.x, i, j, cc, d, Fc);
+  } else {
+    // as in the interior tiles, DF6 is stored only where a source adds to it
+    d[5] = (a.mnu ? a.mnu[cc] : (T)B.nu) * (d[2] + d[4]);
+    if (a.nplace) {
+      point_sources<T>(a, B.rho, td.x, i, j, d);
+      a.DF[5 * ps + cc] = d[5];
+    }
+    const T Bdt = (T)a.Bdt;
+    if (a.do_update) {
+#pragma unroll
+      for (int l = 0; l < 6; l++) {
+        const T f = Fc[l] + Bdt * d[l];
+        if constexpr (NTS) __builtin_nontemporal_store(f, &a.Fout[l * ps + cc]);
+        else a.Fout[l * ps + cc] = f;
+      }
+    }
+    if (!a.skip_df) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) {
+        if constexpr (NTS) __builtin_nontemporal_store(d[l], &a.DF[l * ps + cc]);
+        else a.DF[l * ps + cc] = d[l];
+      }
+    }
+  }
 }
 
 // ---------------------------------------------------------------------
