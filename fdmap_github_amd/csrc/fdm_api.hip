@@ -1774,15 +1774,24 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     // stage).  This file is compiled without contraction, as the kernel.
     bool exact = c->precision == FDM_FP64;
     const size_t np = (size_t)c->nx * c->ny;
-    for (size_t k = 0; k < np && exact; k++) {
-      const double J = P->xq[k] * P->yr[k] - P->xr[k] * P->yq[k];
-      const double ji = 1.0 / J;
-      exact = std::memcmp(&ji, &P->Ji[k], sizeof(double)) == 0;
-    }
+    std::atomic<bool> same{exact};
+    if (exact)
+      parallel_parts(np * 40, [&](int part, int nt) {
+        const size_t k1 = np * (part + 1) / nt;
+        for (size_t k = np * part / nt; k < k1; k++) {
+          const double J = P->xq[k] * P->yr[k] - P->xr[k] * P->yq[k];
+          const double ji = 1.0 / J;
+          if (std::memcmp(&ji, &P->Ji[k], sizeof(double)) != 0) {
+            same = false;
+            return;
+          }
+        }
+      });
+    exact = same;
     if (const char* v = getenv("FDM_JI_CALC")) exact = exact && atoi(v) != 0;
     c->ji_calc = exact;
   }
-  if (c->precision == FDM_FP64 && c->mode == 2 && c->bulk_mode == 2) {
+  if (c->precision == FDM_FP64 && c->bulk_mode == 2 && (c->mode == 2 || c->ji_calc)) {
     // FP32-delta metrics: xq, xr, yq, yr of a point stored as d = m - base
     // in FP32, base = the metric at the first interior point of its block,
     // kept where base + (double)d reproduces m to the bit and marked NaN
@@ -1798,21 +1807,27 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     }
     const float qnan = std::numeric_limits<float>::quiet_NaN();
     std::vector<float> h[4];
-    long long esc = 0;
+    std::atomic<long long> escapes{0};
     for (int q = 0; q < 4; q++) h[q].assign((size_t)c->ps, 0.0f);
-    for (int j = 0; j < c->ny; j++)
-      for (int i = 0; i < c->nx; i++) {
-        const BlockDev& D = c->hblocks[block_of(c, i, j)];
-        for (int q = 0; q < 4; q++) {
-          const double m = mets[q][(size_t)j * c->nx + i];
-          const double d = m - D.mbase[q];
-          const float f = (float)d;
-          const double back = D.mbase[q] + (double)f;
-          const bool ok = std::isfinite(d) && (double)f == d && std::memcmp(&back, &m, sizeof(double)) == 0;
-          h[q][(size_t)j * c->ld + i] = ok ? f : qnan;
-          esc += ok ? 0 : 1;
+    parallel_parts((size_t)c->nx * c->ny * 32, [&](int part, int nt) {
+      const int j1 = (int)((long long)c->ny * (part + 1) / nt);
+      long long n = 0;
+      for (int j = (int)((long long)c->ny * part / nt); j < j1; j++)
+        for (int i = 0; i < c->nx; i++) {
+          const BlockDev& D = c->hblocks[block_of(c, i, j)];
+          for (int q = 0; q < 4; q++) {
+            const double m = mets[q][(size_t)j * c->nx + i];
+            const double d = m - D.mbase[q];
+            const float f = (float)d;
+            const double back = D.mbase[q] + (double)f;
+            const bool ok = std::isfinite(d) && (double)f == d && std::memcmp(&back, &m, sizeof(double)) == 0;
+            h[q][(size_t)j * c->ld + i] = ok ? f : qnan;
+            n += ok ? 0 : 1;
+          }
         }
-      }
+      escapes += n;
+    });
+    const long long esc = escapes;
     bool use = esc * 64 <= 4LL * c->nx * c->ny;
     if (const char* v = getenv("FDM_METRIC_F32")) use = use && atoi(v) != 0;
     if (use) {

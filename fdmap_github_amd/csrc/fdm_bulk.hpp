@@ -2285,8 +2285,12 @@ __global__ void __launch_bounds__(256) bulk_kernel3(BulkArgs<T> a) {
 // operator's half-width, the metrics as in the plane-strain kernel, one
 // barrier.  HET: a heterogeneous medium, the lane's own rho and G.  DISS:
 // artificial dissipation in some block (SBP4), the Jacobian staged with the
-// halo of F; a block without it keeps the plain expression.
-template <typename T, int TX, int TY, bool NTS, int OP = 4, bool HET = false, bool DISS = false>
+// halo of F; a block without it keeps the plain expression.  JI, MC: as in the
+// plane-strain tile.  2 x 701x1401 points, FP64 SBP6, us a stage: 52.0 with
+// Ji and the metrics read as FP64, DF stored every stage and the loads under
+// their lane conditions, 49.5 now.
+template <typename T, int TX, int TY, bool NTS, int OP = 4, bool HET = false, bool DISS = false, bool JI = false,
+          bool MC = false>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(DISS ? 3 : 4)))
 bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   static_assert(!DISS || OP == 4, "artificial dissipation is built for SBP4 only");
@@ -2313,44 +2317,45 @@ bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   const int ld = a.ld, nx1 = a.nx - 1, ny1 = a.ny - 1;
   const long long ps = a.ps;
   const T* __restrict__ F = a.Fin;
-  T vF[NF][3], vR[NR][2], vQ[NQ][2], vJ[DISS ? NF : 1];
-  // The loads stay under their lane conditions here (unlike the plane-strain
-  // tile): the compiler then waits for the F halo before the metric loads,
-  // which slows this launch a little and leaves the second stream's edge and
-  // band kernels, as long as the launch here, room to keep up (C2-sized
-  // antiplane step: 0.366 against 0.414 ms with the loads unconditional).
+  T vF[NF][3], vR[MC ? 1 : NR][2], vQ[MC ? 1 : NQ][2], vJ[DISS ? NF : 1];
+  float fR[MC ? NR : 1][2], fQ[MC ? NQ : 1][2];
+  // every lane loads in every pass, as in the plane-strain tile
 #pragma unroll
   for (int p = 0; p < NF; p++) {
-    const int k = tid + p * NT;
-    if (k < HY * HX) {
-      const int r = k / HX, c = k - r * HX;
-      const int gj = min(max(j0 - H + r, 0), ny1), gi = min(max(i0 - H + c, 0), nx1);
-      const unsigned o = (unsigned)(gj * ld + gi) * (unsigned)sizeof(T);
+    const int k = min(tid + p * NT, HY * HX - 1);
+    const int r = k / HX, c = k - r * HX;
+    const int gj = min(max(j0 - H + r, 0), ny1), gi = min(max(i0 - H + c, 0), nx1);
+    const unsigned o = (unsigned)(gj * ld + gi) * (unsigned)sizeof(T);
 #pragma unroll
-      for (int l = 0; l < 3; l++) vF[p][l] = ld_off(F + l * ps, o);
-      if constexpr (DISS) vJ[p] = ld_off(a.J, o);
-    }
+    for (int l = 0; l < 3; l++) vF[p][l] = ld_off(F + l * ps, o);
+    if constexpr (DISS) vJ[p] = ld_off(a.J, o);
   }
 #pragma unroll
   for (int p = 0; p < NR; p++) {
-    const int k = tid + p * NT;
-    if (k < TY * HX) {
-      const int r = k / HX, c = k - r * HX;
-      const int gj = min(j0 + r, ny1), gi = min(max(i0 - H + c, 0), nx1);
-      const unsigned o = (unsigned)(gj * ld + gi) * (unsigned)sizeof(T);
-      vR[p][0] = ld_off(a.xr, o);
-      vR[p][1] = ld_off(a.yr, o);
+    const int k = min(tid + p * NT, TY * HX - 1);
+    const int r = k / HX, c = k - r * HX;
+    const int gj = min(j0 + r, ny1), gi = min(max(i0 - H + c, 0), nx1);
+    const unsigned o = (unsigned)(gj * ld + gi);
+    if constexpr (MC) {
+      fR[p][0] = ld_off(a.fxr, o * 4u);
+      fR[p][1] = ld_off(a.fyr, o * 4u);
+    } else {
+      vR[p][0] = ld_off(a.xr, o * (unsigned)sizeof(T));
+      vR[p][1] = ld_off(a.yr, o * (unsigned)sizeof(T));
     }
   }
 #pragma unroll
   for (int p = 0; p < NQ; p++) {
-    const int k = tid + p * NT;
-    if (k < HY * TX) {
-      const int r = k / TX, c = k - r * TX;
-      const int gj = min(max(j0 - H + r, 0), ny1), gi = min(i0 + c, nx1);
-      const unsigned o = (unsigned)(gj * ld + gi) * (unsigned)sizeof(T);
-      vQ[p][0] = ld_off(a.xq, o);
-      vQ[p][1] = ld_off(a.yq, o);
+    const int k = min(tid + p * NT, HY * TX - 1);
+    const int r = k / TX, c = k - r * TX;
+    const int gj = min(max(j0 - H + r, 0), ny1), gi = min(i0 + c, nx1);
+    const unsigned o = (unsigned)(gj * ld + gi);
+    if constexpr (MC) {
+      fQ[p][0] = ld_off(a.fxq, o * 4u);
+      fQ[p][1] = ld_off(a.fyq, o * 4u);
+    } else {
+      vQ[p][0] = ld_off(a.xq, o * (unsigned)sizeof(T));
+      vQ[p][1] = ld_off(a.yq, o * (unsigned)sizeof(T));
     }
   }
   const int i = i0 + threadIdx.x, j = j0 + threadIdx.y;
@@ -2359,9 +2364,10 @@ bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   T dfa[3];
   if (!a.a_zero) {
 #pragma unroll
-    for (int l = 0; l < 3; l++) dfa[l] = ld_off(a.DF + l * ps, oc);
+    for (int l = 0; l < 3; l++) dfa[l] = ld_sel<NTS>(a.DF + l * ps, oc);
   }
-  const T Ji = ld_off(a.Ji, oc);
+  T Ji = (T)0;
+  if constexpr (!JI) Ji = ld_off(a.Ji, oc);
   T mrho = (T)0, mG = (T)0;
   if constexpr (HET) {
     mrho = ld_off(a.mrho, oc);
@@ -2382,8 +2388,15 @@ bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
     const int k = tid + p * NT;
     if (k < TY * HX) {
       const int r = k / HX, c = k - r * HX;
-      sR[0][r][c] = vR[p][0];
-      sR[1][r][c] = vR[p][1];
+      if constexpr (MC) {
+        const int gj = min(j0 + r, ny1), gi = min(max(i0 - H + c, 0), nx1);
+        const unsigned o = (unsigned)(gj * ld + gi) * 8u;
+        sR[0][r][c] = metric_of(fR[p][0], B4->mbase[1], a.xr, o);
+        sR[1][r][c] = metric_of(fR[p][1], B4->mbase[3], a.yr, o);
+      } else {
+        sR[0][r][c] = vR[p][0];
+        sR[1][r][c] = vR[p][1];
+      }
     }
   }
 #pragma unroll
@@ -2391,12 +2404,24 @@ bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
     const int k = tid + p * NT;
     if (k < HY * TX) {
       const int r = k / TX, c = k - r * TX;
-      sQ[0][r][c] = vQ[p][0];
-      sQ[1][r][c] = vQ[p][1];
+      if constexpr (MC) {
+        const int gj = min(max(j0 - H + r, 0), ny1), gi = min(i0 + c, nx1);
+        const unsigned o = (unsigned)(gj * ld + gi) * 8u;
+        sQ[0][r][c] = metric_of(fQ[p][0], B4->mbase[0], a.xq, o);
+        sQ[1][r][c] = metric_of(fQ[p][1], B4->mbase[2], a.yq, o);
+      } else {
+        sQ[0][r][c] = vQ[p][0];
+        sQ[1][r][c] = vQ[p][1];
+      }
     }
   }
   __syncthreads();
   if (!valid) return;
+  if constexpr (JI) {
+    const T J = sQ[0][threadIdx.y + H][threadIdx.x] * sR[1][threadIdx.y][threadIdx.x + H] -
+                sR[0][threadIdx.y][threadIdx.x + H] * sQ[1][threadIdx.y + H][threadIdx.x];
+    Ji = (T)1.0 / J;
+  }
   T d[6];
   if (a.a_zero) {
 #pragma unroll
@@ -2436,8 +2461,10 @@ bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
 #pragma unroll
     for (int l = 0; l < 3; l++) st_sel<NTS>(a.Fout + l * ps, oc, acc.f(l, 0, 0) + Bdt * d[l]);
   }
+  if (!a.skip_df) {
 #pragma unroll
-  for (int l = 0; l < 3; l++) st_sel<NTS>(a.DF + l * ps, oc, d[l]);
+    for (int l = 0; l < 3; l++) st_sel<NTS>(a.DF + l * ps, oc, d[l]);
+  }
 }
 
 }  // namespace fdm

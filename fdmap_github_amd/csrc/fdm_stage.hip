@@ -43,12 +43,33 @@ void stage2(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e) {
   stage2_v<T, TX, TY, OP, HET, DISS, false, false>(L, a, e);
 }
 
+namespace {
+
+template <typename T, int OP, bool HET, bool DISS, bool JI, bool MC>
+void stage3_v(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e) {
+  if (L.nt_store)
+    hipLaunchKernelGGL((bulk_interior3<T, 64, 4, true, OP, HET, DISS, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
+                       L.tiles);
+  else
+    hipLaunchKernelGGL((bulk_interior3<T, 64, 4, false, OP, HET, DISS, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
+                       L.tiles);
+}
+
+}  // namespace
+
 template <typename T, int OP, bool HET, bool DISS>
 void stage3(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e) {
-  if (L.nt_store)
-    hipLaunchKernelGGL((bulk_interior3<T, 64, 4, true, OP, HET, DISS>), L.grid, L.block, 0, L.stream, a, e, L.tiles);
-  else
-    hipLaunchKernelGGL((bulk_interior3<T, 64, 4, false, OP, HET, DISS>), L.grid, L.block, 0, L.stream, a, e, L.tiles);
+  if constexpr (std::is_same<T, double>::value) {
+    if (L.mcomp && L.ji_calc) {
+      stage3_v<T, OP, HET, DISS, true, true>(L, a, e);
+      return;
+    }
+    if (L.ji_calc) {
+      stage3_v<T, OP, HET, DISS, true, false>(L, a, e);
+      return;
+    }
+  }
+  stage3_v<T, OP, HET, DISS, false, false>(L, a, e);
 }
 
 namespace {
