@@ -486,8 +486,8 @@ BulkArgs<T> bulk_args(fdm_ctx* c, double A, double Bdt, int do_update, double t,
 // the lean variants serve launches without manufactured solutions or a
 // plastic update
 template <typename T>
-bool full_variant(const fdm_ctx* c, const BulkArgs<T>& a) {
-  return c->any_mms || c->mms_side || a.do_plastic;
+int full_variant(const fdm_ctx* c, const BulkArgs<T>& a) {
+  return c->any_mms || c->mms_side ? 1 : (a.do_plastic ? 2 : 0);
 }
 
 // the band points of the blocks without a layer, in contexts with one
@@ -569,7 +569,7 @@ void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const Edg
   dim3 block(kTileShape[q][0], kTileShape[q][1]);
   if (!grid.x) return;
   EventPair* ep = prof_begin(c, 0, s);
-  const bool full = full_variant(c, a);
+  const int full = full_variant(c, a);
   c->df6_stale = !full && c->mode == 2;
   // (shapes: fdm_create and fdm_tune keep 64 x 4 for antiplane shear, SBP2, a
   // heterogeneous medium and dissipation; SBP6 in a uniform medium runs 64 x
@@ -2389,7 +2389,7 @@ int ens_step_launches(fdm_ensemble* e, int p) {
     const size_t o = ((size_t)p * ns + (s - 1)) * M;
     const BulkArgs<T>* bt = (const BulkArgs<T>*)e->btab + o;
     const EdgeArgs<T>* et = (const EdgeArgs<T>*)e->etab + o;
-    const bool full = e->mms_side || (e->any_plastic && s == ns);
+    const int full = e->mms_side ? 1 : (e->any_plastic && s == ns ? 2 : 0);
     for (int q = 0; q < 3; q++) {
       const dim3 grid(e->nahead[q] + e->ntiles[q]), block(kTileShape[q][0], kTileShape[q][1]);
       if (grid.x)

@@ -472,13 +472,50 @@ __device__ __forceinline__ void point_sources(const BulkArgs<T>& a, const double
   }
 }
 
+// update_fields_plastic (plastic.f90:8-59), full dt, after the last stage: f,
+// d the point's updated fields and rates, gp its gammap, mG and mM its G and M
+// in a heterogeneous medium, which gives each point its G and K (plastic.f90:
+// 37-43).  gammap changes only where the point yields.
+template <typename T, typename BlockRef>
+__device__ __forceinline__ void plastic_update(const BulkArgs<T>& a, BlockRef& B, const long long pc,
+                                               const double gp0, const double mG, const double mM, T (&f)[6],
+                                               T (&d)[6]) {
+  double s[4], Ds[4], s0[6], lam = 0.0, gp = gp0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    s[k] = (double)f[2 + k];
+    Ds[k] = (double)d[2 + k];
+  }
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) s[k] = s[k] + B.Fb[2 + k];
+  }
+#pragma unroll
+  for (int k = 0; k < 6; k++) s0[k] = B.s0[k];
+  const double Gel = a.mG ? mG : B.G;
+  const double Kel = a.mG ? mM - 1.333333333333333 * mG : B.K;
+  plastic_point(Gel, Kel, B.mu, B.beta, B.b, B.h, B.eta, s0, a.dt, s, Ds, lam, gp);
+  a.lambda[pc] = lam;
+  if (lam != 0.0) a.gammap[pc] = gp;
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) s[k] = s[k] - B.Fb[2 + k];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    f[2 + k] = (T)s[k];
+    d[2 + k] = (T)Ds[k];
+  }
+}
+
 // szz overwrite, sources, RK update, plasticity and stores of one point
 // (rates.f90:920-936, source.f90:196-296, fields.f90:1225-1242,
 // plastic.f90:8-59).  Fc: the point's fields at the start of the stage.
-// FULL = false leaves out the manufactured-solution source and plasticity;
+// FULL = 0 leaves out the manufactured-solution source and plasticity, FULL =
+// 2 the manufactured solution alone (FULL = 1: neither);
 // the host selects it for launches that need neither.  NTS stores F and DF
 // non-temporally.
-template <typename T, bool FULL, bool NTS = false>
+template <typename T, int FULL, bool NTS = false>
 __device__ __forceinline__ void finish_point(const BulkArgs<T>& a, const BlockDev& B, const int bi,
                                              const int i, const int j, const long long cc,
                                              T (&d)[6], const T (&Fc)[6]) {
@@ -488,7 +525,7 @@ __device__ __forceinline__ void finish_point(const BulkArgs<T>& a, const BlockDe
   d[5] = (a.mnu ? a.mnu[cc] : (T)B.nu) * (d[2] + d[4]);
   point_sources<T>(a, B.rho, bi, i, j, d);
   // manufactured-solution source (source.f90:256-269)
-  if (FULL && B.mms) {
+  if (FULL == 1 && B.mms) {
     double x = a.X[(long long)j * a.nx + i], y = a.Y[(long long)j * a.nx + i];
 #pragma unroll 1
     for (int l = 0; l < 6; l++) d[l] = d[l] + (T)mms_sin(x, y, a.t, B.id, 6 + l);
@@ -499,36 +536,9 @@ __device__ __forceinline__ void finish_point(const BulkArgs<T>& a, const BlockDe
     T f[6];
 #pragma unroll
     for (int l = 0; l < 6; l++) f[l] = Fc[l] + Bdt * d[l];
-    if (FULL && a.do_plastic && B.plastic) {
-      // update_fields_plastic (plastic.f90:8-59), full dt, after the last stage
-      double s[4], Ds[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        s[k] = (double)f[2 + k];
-        Ds[k] = (double)d[2 + k];
-      }
-      if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) s[k] = s[k] + B.Fb[2 + k];
-      }
-      long long pc = (long long)j * a.nx + i;
-      double lam = a.lambda[pc], gp = a.gammap[pc];
-      // a heterogeneous medium gives each point its G and K (plastic.f90:37-43)
-      const double Gel = a.mG ? (double)a.mG[cc] : B.G;
-      const double Kel = a.mG ? (double)a.mM[cc] - 1.333333333333333 * (double)a.mG[cc] : B.K;
-      plastic_point(Gel, Kel, B.mu, B.beta, B.b, B.h, B.eta, B.s0, a.dt, s, Ds, lam, gp);
-      a.lambda[pc] = lam;
-      a.gammap[pc] = gp;
-      if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) s[k] = s[k] - B.Fb[2 + k];
-      }
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        f[2 + k] = (T)s[k];
-        d[2 + k] = (T)Ds[k];
-      }
-    }
+    if (FULL && a.do_plastic && B.plastic)
+      plastic_update<T>(a, B, (long long)j * a.nx + i, a.gammap[(long long)j * a.nx + i],
+                        a.mG ? (double)a.mG[cc] : 0.0, a.mG ? (double)a.mM[cc] : 0.0, f, d);
 #pragma unroll
     for (int l = 0; l < 6; l++) {
       if constexpr (NTS) __builtin_nontemporal_store(f[l], &a.Fout[l * ps + cc]);
@@ -921,7 +931,7 @@ __device__ __forceinline__ int block_at(const BulkArgs<T>& a, const int i, const
 
 // PML = false leaves the layer out (contexts without one), INNER = true the
 // closures (interior points only).
-template <typename T, bool FULL, bool EXT, int OP = 4, bool PML = EXT, bool INNER = false>
+template <typename T, int FULL, bool EXT, int OP = 4, bool PML = EXT, bool INNER = false>
 __device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i, const int j, const int bi) {
   const BlockDev& B = a.blocks[bi];
   const long long ps = a.ps;
@@ -1075,7 +1085,7 @@ constexpr int kRimRowsMax =
 constexpr int kRimHats = 2 * kRimIface > kRimNodes ? 2 * kRimIface : kRimNodes;
 constexpr int kRimBytes = (kRimRowsMax + 6 * kRimHats) * (int)sizeof(double);
 
-template <typename T, int TX, int TY, bool FULL, bool NTS, bool HET, bool DISS, int OP = 4,
+template <typename T, int TX, int TY, int FULL, bool NTS, bool HET, bool DISS, int OP = 4,
           bool JI = false, bool MC = false>
 __device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 td, char* smem) {
   // H: the operator's interior half-width, the tile's halo; NB: the
@@ -1157,6 +1167,12 @@ __device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 t
     for (int l = 0; l < 5; l++) dfa[l] = ld_sel<NTS>(a.DF + l * ps, oc);
   }
   const T f6 = ld_sel<NTS>(F + 5 * ps, oc);
+  // the lane's gammap, where this launch ends in a plastic update
+  const int pc = min(j, ny1) * a.nx + min(i, nx1);
+  double gp = 0.0;
+  const bool yields = FULL == 2 && a.do_plastic && B4->plastic;
+  if constexpr (FULL == 2)
+    if (yields) gp = a.gammap[pc];
   T Ji = (T)0.0;
   if constexpr (!JI) Ji = ld_off(a.Ji, oc);
   // a heterogeneous medium: the lane's own material (rho, G, M, gamma, nu)
@@ -1254,8 +1270,8 @@ __device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 t
 #pragma unroll
   for (int k = 0; k < 5; k++) Fc[k] = acc.f(k, 0, 0);
   Fc[5] = f6;
-  if constexpr (FULL) {
-    finish_point<T, true>(a, a.blocks[bu], bu, i, j, (long long)j * ld + i, d, Fc);
+  if constexpr (FULL == 1) {
+    finish_point<T, 1>(a, a.blocks[bu], bu, i, j, (long long)j * ld + i, d, Fc);
   } else {
     // rates_szz (rates.f90:920-936), update_fields_interior (fields.f90:1225-1242).
     // DF6 is not stored: no stage reads it (each overwrites it with this
@@ -1267,12 +1283,23 @@ __device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 t
     d[5] = nu * (d[2] + d[4]);
     if (a.do_update) {
       const T Bdt = (T)a.Bdt;
+      T f[6];
 #pragma unroll
-      for (int l = 0; l < 6; l++) st_sel<NTS>(a.Fout + l * ps, oc, Fc[l] + Bdt * d[l]);
+      for (int l = 0; l < 6; l++) f[l] = Fc[l] + Bdt * d[l];
+      if constexpr (FULL == 2) {
+        double mG = 0.0, mM = 0.0;
+        if constexpr (HET) {
+          mG = (double)mat[1];
+          mM = (double)mat[2];
+        }
+        if (yields) plastic_update<T>(a, *B4, pc, gp, mG, mM, f, d);
+      }
+#pragma unroll
+      for (int l = 0; l < 6; l++) st_sel<NTS>(a.Fout + l * ps, oc, f[l]);
     }
     if (!a.skip_df) {
 #pragma unroll
-      for (int l = 0; l < 5; l++) st_sel<NTS>(a.DF + l * ps, oc, d[l]);
+      for (int l = 0; l < (FULL ? 6 : 5); l++) st_sel<NTS>(a.DF + l * ps, oc, d[l]);
     }
   }
 }
@@ -1597,7 +1624,7 @@ __device__ __forceinline__ T band_sum(T d, const BandTerms<T, OP, EXT>& o, const
 // szz, DF(6) = nu (DF(3) + DF(5)), from field 4's rate two lanes up.  FULL:
 // the lane of field 0 gathers the rates and finishes the point.  Every lane
 // runs to the shuffles (idle ones on a clamped point).
-template <typename T, int MODE, bool FULL>
+template <typename T, int MODE, int FULL>
 __device__ __forceinline__ void band_finish(const BulkArgs<T>& a, const BlockDev& B, const BandPt& p,
                                             const long long cc, const int l, const int lane, const bool active,
                                             const T d, const T Fown, const T F6) {
@@ -1614,7 +1641,7 @@ __device__ __forceinline__ void band_finish(const BulkArgs<T>& a, const BlockDev
     if (!active || l != 0) return;
 #pragma unroll
     for (int k = 0; k < 6; k++) Fc[k] = a.Fin[k * ps + cc];
-    finish_point<T, true>(a, B, p.blk, p.i, p.j, cc, dd, Fc);
+    finish_point<T, FULL>(a, B, p.blk, p.i, p.j, cc, dd, Fc);
   } else {
     const T d4 = __shfl(d, (lane + 2) & 63, 64);
     if (!active) return;
@@ -1643,7 +1670,7 @@ struct BandLanes {
 };
 
 // a wave of inner band points
-template <typename T, int MODE, bool FULL, bool EXT, int OP>
+template <typename T, int MODE, int FULL, bool EXT, int OP>
 __device__ __forceinline__ void inner_band_wave(const BulkArgs<T>& a, const int first, const int lane) {
   using L = BandLanes<MODE>;
   const int grp = lane / L::per, l = min(lane - L::per * grp, L::per - 1);
@@ -1687,7 +1714,7 @@ __device__ __forceinline__ const P& memory_args(const void* p) {
 // edge nodes in LDS, a node a lane and a quarter of the rows a wave, so that
 // the node's whole input is in flight at once whatever registers the tiles
 // leave the kernel; then the first wave evaluates the nodes from LDS.
-template <typename T, int MODE, bool FULL, bool EXT, int OP>
+template <typename T, int MODE, int FULL, bool EXT, int OP>
 __device__ __forceinline__ void rim_group(const void* pa, const void* pe, const int wb, double* sN, const int wave,
                                           const int lane) {
   constexpr int NF = MODE == 3 ? 3 : 6;
@@ -1722,7 +1749,7 @@ __device__ __forceinline__ void rim_group(const void* pa, const void* pe, const 
   auto hats = [&](FaultSolved& f) {
     const EdgeArgs<T>& en = memory_args<EdgeArgs<T>>(pe);
     double hm[6], hp[6];
-    edge_node<T, MODE, true, FULL>(en, nd, NodeRows{sN + lane, stride}, hm, hp, f);
+    edge_node<T, MODE, true, FULL == 1>(en, nd, NodeRows{sN + lane, stride}, hm, hp, f);
 #pragma unroll
     for (int k = 0; k < NF; k++) sH[lane][k] = hm[k];
     if (nd.iface >= 0) {
@@ -1805,7 +1832,7 @@ __device__ __forceinline__ void point_generic3(const BulkArgs<T>& a, const int i
 // band.  Dispatched first, their latency overlaps the tiles.  pa, pe: the
 // stage's BulkArgs (also a) and EdgeArgs in memory; wb: this workgroup's
 // index among them.
-template <typename T, int MODE, int TX, int TY, bool FULL, bool EXT, int OP>
+template <typename T, int MODE, int TX, int TY, int FULL, bool EXT, int OP>
 __device__ __forceinline__ void stage_ahead(const BulkArgs<T>& a, const void* pa, const void* pe, int wb,
                                             char* smem) {
   constexpr int NT = TX * TY;
@@ -1853,11 +1880,14 @@ __device__ __forceinline__ void stage_ahead(const BulkArgs<T>& a, const void* pa
 // 32.3 -> 15.4, 2 x 801x401 42.6 -> 26.1, 2 x 1601x801 106 -> 88.8 (FP32-bulk
 // 58.1 -> 47.6).  A heterogeneous medium holds five
 // more values per lane, dissipation the Jacobian's staging: three waves per
-// SIMD keep them in registers.
-template <typename T, int TX, int TY, bool FULL, bool NTS, bool HET, bool DISS, int OP = 4,
+// SIMD keep them in registers, and the plastic update with them (FULL = 2; the
+// last stage of 2 x 3201x1601 points, FP64: 606 us on the variant that also
+// carries manufactured solutions, two waves, normal stores and DF always
+// stored, 398 on its own).
+template <typename T, int TX, int TY, int FULL, bool NTS, bool HET, bool DISS, int OP = 4,
           bool JI = false, bool MC = false>
 __global__ void __launch_bounds__(TX * TY)
-    __attribute__((amdgpu_waves_per_eu(FULL ? 2 : ((HET || DISS || OP == 6) ? 3 : 4))))
+    __attribute__((amdgpu_waves_per_eu(FULL == 1 ? 2 : ((FULL || HET || DISS || OP == 6) ? 3 : 4))))
 bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   constexpr int kTile = tile_bytes<T, TX, TY, DISS, OP, 5>();
   __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];
@@ -1868,7 +1898,7 @@ bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
     return;
   }
   const int4 td = tiles[linear_tile(a.xcd_swizzle, ahead)];
-  if constexpr (!FULL) {
+  if constexpr (FULL != 1) {
     if (td.w) {
       // The few tiles a point source reaches, a lane a point from global
       // memory: in the tile's own path the source's terms took registers that
@@ -1877,7 +1907,7 @@ bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
       const int bu = td.x, i = td.y + threadIdx.x, j = td.z + threadIdx.y;
       const BlockDev& B = a.blocks[bu];
       if (i <= B.px - Sbp<OP>::nbst && j <= B.py - Sbp<OP>::nbst)
-        point_generic<T, false, HET || DISS, OP, false, true>(a, i, j, bu);
+        point_generic<T, FULL, HET || DISS, OP, false, true>(a, i, j, bu);
       return;
     }
   }
@@ -1887,8 +1917,8 @@ bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
 // Batched stage launch: the rim groups, inner band points and tiles of many
 // problems.  ahead[k] = (problem, its workgroup index) of the nahead
 // workgroups ahead of the tiles; tile .w selects the problem's arguments.
-template <typename T, int TX, int TY, bool FULL, bool NTS>
-__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(FULL ? 2 : 4)))
+template <typename T, int TX, int TY, int FULL, bool NTS>
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(FULL == 1 ? 2 : (FULL ? 3 : 4))))
 bulk_interior_batch(const BulkArgs<T>* __restrict__ tab, const EdgeArgs<T>* __restrict__ etab,
                     const int2* __restrict__ ahead, int nahead, const int4* __restrict__ tiles, int swz) {
   constexpr int kTile = tile_bytes<T, TX, TY, false, 4, 5>();
@@ -1962,7 +1992,7 @@ __global__ void __launch_bounds__(256) bulk_layer(BulkArgs<T> a, const int4* __r
   scaled_rates<T>(a, cc, d);
   pml_rates<T, true>(a, B, i, j, cc, d, B.pmlx != 0 && (w & 1), B.pmly != 0 && (w & 2));
   if constexpr (FULL) {
-    finish_point<T, true, NTS>(a, a.blocks[td.x], td.x, i, j, cc, d, Fc);
+    finish_point<T, 1, NTS>(a, a.blocks[td.x], td.x, i, j, cc, d, Fc);
   } else {
     // as in the interior tiles, DF6 is stored only where a source adds to it
     d[5] = (a.mnu ? a.mnu[cc] : (T)B.nu) * (d[2] + d[4]);

@@ -10,15 +10,21 @@ namespace {
 
 template <typename T, int TX, int TY, int OP, bool HET, bool DISS, bool JI, bool MC>
 void stage2_v(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e) {
-  if (L.full)
-    hipLaunchKernelGGL((bulk_interior<T, TX, TY, true, false, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream,
-                       a, e, L.tiles);
+  if (L.full == 1)
+    hipLaunchKernelGGL((bulk_interior<T, TX, TY, 1, false, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
+                       L.tiles);
+  else if (L.full && L.nt_store)
+    hipLaunchKernelGGL((bulk_interior<T, TX, TY, 2, true, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
+                       L.tiles);
+  else if (L.full)
+    hipLaunchKernelGGL((bulk_interior<T, TX, TY, 2, false, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
+                       L.tiles);
   else if (L.nt_store)
-    hipLaunchKernelGGL((bulk_interior<T, TX, TY, false, true, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream,
-                       a, e, L.tiles);
+    hipLaunchKernelGGL((bulk_interior<T, TX, TY, 0, true, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
+                       L.tiles);
   else
-    hipLaunchKernelGGL((bulk_interior<T, TX, TY, false, false, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream,
-                       a, e, L.tiles);
+    hipLaunchKernelGGL((bulk_interior<T, TX, TY, 0, false, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
+                       L.tiles);
 }
 
 }  // namespace
@@ -77,15 +83,21 @@ namespace {
 template <typename T, int TX, int TY>
 void batch_v(const StageLaunch& L, const BulkArgs<T>* bt, const EdgeArgs<T>* et, const int2* ahead, int nahead,
              int swz) {
-  if (L.full)
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, true, false>), L.grid, L.block, 0, L.stream, bt, et, ahead,
-                       nahead, L.tiles, swz);
+  if (L.full == 1)
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 1, false>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
+                       L.tiles, swz);
+  else if (L.full && L.nt_store)
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 2, true>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
+                       L.tiles, swz);
+  else if (L.full)
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 2, false>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
+                       L.tiles, swz);
   else if (L.nt_store)
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, false, true>), L.grid, L.block, 0, L.stream, bt, et, ahead,
-                       nahead, L.tiles, swz);
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 0, true>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
+                       L.tiles, swz);
   else
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, false, false>), L.grid, L.block, 0, L.stream, bt, et, ahead,
-                       nahead, L.tiles, swz);
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 0, false>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
+                       L.tiles, swz);
 }
 
 }  // namespace

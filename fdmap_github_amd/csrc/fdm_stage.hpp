@@ -16,11 +16,12 @@ struct StageLaunch {
   dim3 grid, block;
   const int4* tiles;
   int shape;
-  bool full, nt_store, ji_calc, mcomp;
+  int full;  // FULL of the kernels
+  bool nt_store, ji_calc, mcomp;
 };
 
-// plane strain: FULL (sources, MMS, plasticity), or lean with non-temporal or
-// normal stores; in FP64 with or without Ji formed in the kernel (ji_calc)
+// plane strain: FULL = 1 (manufactured solutions, plasticity), 2 (plasticity)
+// or lean, these with non-temporal or normal stores; in FP64 with or without Ji formed in the kernel (ji_calc)
 // and FP32-delta metrics (mcomp)
 template <typename T, int OP, bool HET, bool DISS, int SHAPE>
 void stage2(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e);
