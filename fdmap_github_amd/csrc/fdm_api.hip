@@ -1900,6 +1900,9 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
 
 int fdm_set_fields(fdm_ctx* c, const double* F, const double* DF) {
   if (!c || !F) return FDM_EINVAL;
+  // the copies below are not ordered after the context's stream, which may
+  // still be stepping
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->df6_stale = false;
   size_t pe = (size_t)c->ps;
   if (c->precision == FDM_FP64) {
