@@ -47,11 +47,6 @@ struct fdm_ctx {
   size_t esz = 8;
   double rkA[FDM_MAX_STAGES], rkB[FDM_MAX_STAGES], rkC[FDM_MAX_STAGES + 1];
   hipStream_t stream = nullptr;
-  // edge and band kernels run on a second stream (default priority) so that
-  // they overlap the interior launches; evI / evB mark the latest interior /
-  // band launch, evJ forks the side stream off the main one
-  hipStream_t side = nullptr;
-  hipEvent_t evI = nullptr, evB = nullptr, evJ = nullptr;
   int device = 0;
   // bulk storage (element type per precision)
   void* F[2] = {nullptr, nullptr};
@@ -141,15 +136,11 @@ struct fdm_ctx {
   // Wy, DWx, DWy, 6 planes each (field precision, plane stride ps)
   bool pml = false, pml_wx = false, pml_wy = false;
   void* W = nullptr;
-  // the points of the layer blocks within four of an edge of their block
-  // (lpts), and the tiles of the others (bulk_layer; hltiles: on the host,
-  // without padding)
-  int2* lpts = nullptr;
-  int nlpts = 0;
+  // the tiles of the layer blocks (bulk_layer; hltiles: on the host, without
+  // padding)
   int4* ltiles = nullptr;
   int nltiles = 0;
   std::vector<int4> hltiles;
-  long long nlayer_inner = 0;  // points of the layer tiles
   int layer_all = 0;           // BulkArgs::layer_all
   // 2: plane strain, 6 fields; 3: antiplane shear, 3 fields
   int mode = 2, nF = 6;
@@ -163,8 +154,6 @@ struct fdm_ctx {
   // interior tiles (block, i0, j0, 0) for the tile shapes 64x4, 64x8, 128x4; band points (i, j)
   int4* tiles[3] = {nullptr, nullptr, nullptr};
   int ntiles[3] = {0, 0, 0};
-  int2* band = nullptr;
-  int nband = 0;
   // host copies of the tile list (ensembles merge them), the band points and
   // the edge tasks
   std::vector<int4> htiles[3];
@@ -176,7 +165,6 @@ struct fdm_ctx {
   long long* nstep_dev = nullptr;
   bool graph_mode = false;
   double g_tinit = 0.0, g_dt = 0.0, g_rkc = 0.0;
-  long long ninterior = 0;
   // adjoint forward passes: fault trajectories ([nstage][3][NI] per step,
   // step n at trace + (n - trace_n0) nstage 3 NI), the slot of the stage
   // being launched, and vx, vy at receivers after every step (step n at
@@ -344,7 +332,6 @@ EventPair* prof_begin(fdm_ctx* c, int kind, hipStream_t s) {
     } else {
       // drain: accumulate and recycle
       (void)hipStreamSynchronize(c->stream);
-      if (c->side) (void)hipStreamSynchronize(c->side);
       for (size_t k = 0; k < c->pool_used; k++) {
         float ms = 0.f;
         (void)hipEventElapsedTime(&ms, c->pool[k].a, c->pool[k].b);
@@ -490,51 +477,6 @@ int full_variant(const fdm_ctx* c, const BulkArgs<T>& a) {
   return c->any_mms || c->mms_side ? 1 : (a.do_plastic ? 2 : 0);
 }
 
-// the band points of the blocks without a layer, in contexts with one
-template <typename T>
-void launch_band(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
-  const int n = c->nband;
-  if (!n) return;
-  EventPair* ep = prof_begin(c, 2, s);
-  dim3 grid((n + 63) / 64), block(64);
-  const bool ext = c->het || c->diss;
-  if (full_variant(c, a) && ext)
-    hipLaunchKernelGGL((bulk_band<T, true, true>), grid, block, 0, s, a, c->band, n);
-  else if (full_variant(c, a))
-    hipLaunchKernelGGL((bulk_band<T, true, false>), grid, block, 0, s, a, c->band, n);
-  else if (ext)
-    hipLaunchKernelGGL((bulk_band<T, false, true>), grid, block, 0, s, a, c->band, n);
-  else
-    hipLaunchKernelGGL((bulk_band<T, false, false>), grid, block, 0, s, a, c->band, n);
-  prof_end(c, ep, 2, s);
-}
-
-// the layer points near block edges, after the band on the same stream (they
-// need this stage's edge values); timed with the band
-template <typename T>
-void launch_layer_edges(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
-  if (!c->nlpts) return;
-  EventPair* ep = prof_begin(c, 2, s);
-  dim3 grid((c->nlpts + 63) / 64), block(64);
-  if (full_variant(c, a)) hipLaunchKernelGGL((bulk_pml<T, true>), grid, block, 0, s, a, c->lpts, c->nlpts);
-  else hipLaunchKernelGGL((bulk_pml<T, false>), grid, block, 0, s, a, c->lpts, c->nlpts);
-  prof_end(c, ep, 2, s);
-}
-
-// the other layer points, which need no edge value: timed with the interior
-template <typename T>
-void launch_layer_tiles(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
-  if (!c->nltiles) return;
-  const bool full = full_variant(c, a);
-  c->df6_stale = !full;
-  EventPair* ep = prof_begin(c, 0, s);
-  dim3 grid(c->nltiles), block(64, 4);
-  if (full) hipLaunchKernelGGL((bulk_layer<T, true, false>), grid, block, 0, s, a, c->ltiles);
-  else if (c->nt_store) hipLaunchKernelGGL((bulk_layer<T, false, true>), grid, block, 0, s, a, c->ltiles);
-  else hipLaunchKernelGGL((bulk_layer<T, false, false>), grid, block, 0, s, a, c->ltiles);
-  prof_end(c, ep, 0, s);
-}
-
 // Inner band points: one lane per (point, field), or one lane per point?
 // Five lanes a point finish sooner (5 us against 12) but hold five times the
 // workgroups.  They pay while the whole launch is resident at once (`others`
@@ -553,13 +495,13 @@ inline int band_wgs(int nib, int nt, int mode, int lanes) {
 }
 
 // One stage: the rim groups, receivers and inner band points ahead of the
-// interior tiles (contexts with a layer: the tiles alone).
+// interior tiles (contexts with a layer: the tiles of the other blocks alone).
 template <typename T>
 void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const EdgeArgs<T>& e) {
   const int q = c->tile_shape;
   BulkArgs<T> a = a0;
   const int nt = kTileShape[q][0] * kTileShape[q][1];
-  if (c->fused) {
+  if (!c->pml) {
     a.nrimwg = c->nrim;
     a.nrecwg = (a.nrec + nt - 1) / nt;
     a.ib_lanes = band_lanes(c->nib, c->nrim + c->ntiles[q], nt, c->mode);
@@ -599,6 +541,31 @@ void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const Edg
   prof_end(c, ep, 0, s);
 }
 
+// contexts with a layer: the rim groups and inner band points of all blocks,
+// ahead of the layer's tiles
+template <typename T>
+void launch_layer(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const EdgeArgs<T>& e) {
+  BulkArgs<T> a = a0;
+  a.nrimwg = c->nrim;
+  a.nibwg = (c->nib + 255) / 256;
+  const int full = full_variant(c, a);
+  c->df6_stale = !full;
+  EventPair* ep = prof_begin(c, 0, s);
+  dim3 grid(a.nrimwg + a.nibwg + c->nltiles), block(64, 4);
+  auto go = [&](auto mix) {
+    constexpr bool MIX = decltype(mix)::value;
+    if (full == 1) hipLaunchKernelGGL((bulk_layer<T, 1, false, MIX>), grid, block, 0, s, a, e, c->ltiles);
+    else if (full && c->nt_store) hipLaunchKernelGGL((bulk_layer<T, 2, true, MIX>), grid, block, 0, s, a, e, c->ltiles);
+    else if (full) hipLaunchKernelGGL((bulk_layer<T, 2, false, MIX>), grid, block, 0, s, a, e, c->ltiles);
+    else if (c->nt_store) hipLaunchKernelGGL((bulk_layer<T, 0, true, MIX>), grid, block, 0, s, a, e, c->ltiles);
+    else hipLaunchKernelGGL((bulk_layer<T, 0, false, MIX>), grid, block, 0, s, a, e, c->ltiles);
+  };
+  const bool mixed = std::any_of(c->hblocks.begin(), c->hblocks.end(), [](const BlockDev& B) { return !(B.pmlx | B.pmly); });
+  if (mixed) go(std::true_type{});
+  else go(std::false_type{});
+  prof_end(c, ep, 0, s);
+}
+
 template <typename T>
 void launch_pointwise(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a) {
   c->df6_stale = false;
@@ -632,23 +599,6 @@ void record_receivers(fdm_ctx* c, hipStream_t s, long long n) {
   hipLaunchKernelGGL(record_receivers_kernel, dim3((c->nrec + 63) / 64), dim3(64), 0, s,
                      (const double*)c->F[c->cur], c->ps, c->rec_cc, c->nrec,
                      c->rec_out + (size_t)(n - c->rec_n0) * c->nrec * 2);
-}
-
-// Fork the side stream off the main one before a sequence of stages, and
-// join it back afterwards, so that work queued on the main stream later (and
-// every synchronisation of it) is ordered after both.
-int fork_side(fdm_ctx* c) {
-  HIPCHK(c, hipEventRecord(c->evJ, c->stream));
-  HIPCHK(c, hipStreamWaitEvent(c->side, c->evJ, 0));
-  HIPCHK(c, hipEventRecord(c->evB, c->side));
-  HIPCHK(c, hipEventRecord(c->evI, c->stream));
-  return FDM_OK;
-}
-
-int join_side(fdm_ctx* c) {
-  HIPCHK(c, hipEventRecord(c->evB, c->side));
-  HIPCHK(c, hipStreamWaitEvent(c->stream, c->evB, 0));
-  return FDM_OK;
 }
 
 // skip_df: the stage is the last of a step that another step of the same
@@ -687,22 +637,7 @@ int run_stage(fdm_ctx* c, int stage, double t0, double dt, int final_step, int s
       record_receivers(c, c->stream, c->cur_n - 1);
     }
     launch_interior<T>(c, c->stream, a, e);
-  } else if (c->bulk_mode == 2) {
-    // A context with a layer.  Interior points need neither this stage's
-    // edge values nor this stage's band: only the band of the previous stage
-    // (halo values, and the buffer this launch overwrites is the one that
-    // band read).  The band needs this stage's edge values and the previous
-    // interior launch.
-    HIPCHK(c, hipStreamWaitEvent(c->stream, c->evB, 0));
-    launch_interior<T>(c, c->stream, a, e);
-    launch_layer_tiles<T>(c, c->stream, a);
-    rc = launch_edges<T>(c, c->side, e);
-    if (rc) return rc;
-    HIPCHK(c, hipStreamWaitEvent(c->side, c->evI, 0));
-    launch_band<T>(c, c->side, a);
-    launch_layer_edges<T>(c, c->side, a);
-    HIPCHK(c, hipEventRecord(c->evB, c->side));
-    HIPCHK(c, hipEventRecord(c->evI, c->stream));
+    if (c->pml) launch_layer<T>(c, c->stream, a, e);
   } else {
     rc = launch_edges<T>(c, c->stream, e);
     if (rc) return rc;
@@ -716,7 +651,7 @@ int run_stage(fdm_ctx* c, int stage, double t0, double dt, int final_step, int s
 
 template <typename T>
 int step_impl(fdm_ctx* c, double t, double dt, long long n_first, int nsteps) {
-  int rc = c->fused ? FDM_OK : fork_side(c);
+  int rc = FDM_OK;
   c->first_n = n_first;
   for (int k = 0; k < nsteps && !rc; k++) {
     long long n = n_first + k;
@@ -728,20 +663,16 @@ int step_impl(fdm_ctx* c, double t, double dt, long long n_first, int nsteps) {
     for (int stage = 1; stage <= c->nstage && !rc; stage++)
       rc = run_stage<T>(c, stage, t0, dt, 0, stage == 1, skip_df);
   }
-  int rj = c->fused ? FDM_OK : join_side(c);
-  if (!rc && !rj && c->rec_out && nsteps > 0) {
+  if (!rc && c->rec_out && nsteps > 0) {
     record_receivers(c, c->stream, n_first + nsteps - 1);
     HIPCHK(c, hipGetLastError());
   }
-  return rc ? rc : rj;
+  return rc;
 }
 
 template <typename T>
 int stage1_impl(fdm_ctx* c, double t0, double dt) {
-  int rc = c->fused ? FDM_OK : fork_side(c);
-  if (!rc) rc = run_stage<T>(c, 1, t0, dt, 1, 1);
-  int rj = c->fused ? FDM_OK : join_side(c);
-  return rc ? rc : rj;
+  return run_stage<T>(c, 1, t0, dt, 1, 1);
 }
 
 // whether a point source's footprint holds point (i, j) of block b
@@ -897,7 +828,6 @@ int layer_tiles(fdm_ctx* c, const fdm_problem* P) {
     if (!layer_block(B)) continue;
     const int ia = B.mx + 4, ib = B.px - 4, ja = B.my + 4, jb = B.py - 4;
     if (ia > ib || ja > jb) continue;
-    c->nlayer_inner += (long long)(ib - ia + 1) * (jb - ja + 1);
     // a direction may be left out where its profile (pml_rates) is zero at
     // every point, if zeros then stay zeros: finite factors, and a first
     // stage that starts its rates afresh
@@ -992,7 +922,7 @@ int build_stage_lists(fdm_ctx* c) {
   }
   int rc;
   if ((rc = dupload(c, &c->nodes, nodes.data(), std::max<size_t>(1, nodes.size()) * sizeof(EdgeNode)))) return rc;
-  c->fused = c->bulk_mode == 2 && !c->pml;
+  c->fused = c->bulk_mode == 2;
   if (!c->fused) return FDM_OK;
 
   auto band_pt = [&](int2 p) {
@@ -1112,7 +1042,6 @@ const char* fdm_last_error(const fdm_ctx* c) { return c ? c->err.c_str() : g_cre
 void fdm_destroy(fdm_ctx* c) {
   if (!c) return;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->side) (void)hipStreamSynchronize(c->side);
   if (c->copy) {
     (void)hipStreamSynchronize(c->copy);
     (void)hipStreamDestroy(c->copy);
@@ -1128,10 +1057,6 @@ void fdm_destroy(fdm_ctx* c) {
     (void)hipEventDestroy(ep.b);
   }
   for (void* p : c->allocs) (void)hipFree(p);
-  if (c->evI) (void)hipEventDestroy(c->evI);
-  if (c->evB) (void)hipEventDestroy(c->evB);
-  if (c->evJ) (void)hipEventDestroy(c->evJ);
-  if (c->side) (void)hipStreamDestroy(c->side);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -1247,16 +1172,6 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     delete c;
     return set_err(nullptr, FDM_EDEVICE, "fdm_create: hipStreamCreate failed");
   }
-  if (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
-      // the stage marks order work on this device only: no system-scope
-      // fence (an event recorded with one costs about 3 us of GPU time per
-      // stage on the stream that records it)
-      hipEventCreateWithFlags(&c->evI, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess ||
-      hipEventCreateWithFlags(&c->evB, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess ||
-      hipEventCreateWithFlags(&c->evJ, hipEventDisableTiming) != hipSuccess) {
-    fdm_destroy(c);
-    return set_err(nullptr, FDM_EDEVICE, "fdm_create: stream/event creation failed");
-  }
   auto fail = [&](int rc) {
     g_create_error = c->err.empty() ? g_create_error : c->err;
     fdm_destroy(c);
@@ -1350,7 +1265,6 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
       if (layer_block(B)) continue;
       const int ia = B.mx + nbst, ib = B.px - nbst, ja = B.my + nbst, jb = B.py - nbst;
       if (ia > ib || ja > jb) continue;
-      c->ninterior += (long long)(ib - ia + 1) * (jb - ja + 1);
       // .w: a point source's five-point footprint reaches the tile
       auto reached = [&](int i0, int j0, int tx, int ty) {
         for (int k = 0; k < P->source.nplace; k++) {
@@ -1365,27 +1279,19 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
           for (int i0 = ia; i0 <= ib; i0 += tx) tl[q].push_back(make_int4(b, i0, j0, reached(i0, j0, tx, ty)));
       }
     }
-    std::vector<int2> band, lpts;
+    std::vector<int2> band;
     for (int j = 0; j < P->ny; j++)
       for (int i = 0; i < P->nx; i++) {
         const fdm_block& B = P->blocks[block_of(c, i, j)];
         const bool edge = i - B.mx < nbst || B.px - i < nbst || j - B.my < nbst || B.py - j < nbst;
-        if (c->mode == 2 && layer_block(B)) {
-          if (edge) lpts.push_back(make_int2(i, j));
-        } else if (edge) {
-          band.push_back(make_int2(i, j));
-        }
+        if (edge) band.push_back(make_int2(i, j));
       }
-    c->nlpts = (int)lpts.size();
-    if (c->nlpts && (rc = dupload(c, &c->lpts, lpts.data(), lpts.size() * sizeof(int2)))) return fail(rc);
     if (c->mode == 2 && (rc = layer_tiles(c, P))) return fail(rc);
     for (int q = 0; q < 3; q++) {
       c->ntiles[q] = (int)tl[q].size();
       if (c->ntiles[q] && (rc = dupload(c, &c->tiles[q], tl[q].data(), tl[q].size() * sizeof(int4))))
         return fail(rc);
     }
-    c->nband = (int)band.size();
-    if (c->nband && (rc = dupload(c, &c->band, band.data(), band.size() * sizeof(int2)))) return fail(rc);
     for (int q = 0; q < 3; q++) c->htiles[q] = std::move(tl[q]);
     c->hband = std::move(band);
   }
@@ -2252,10 +2158,7 @@ int fdm_profile_read(fdm_ctx* c, fdm_profile_t* out) {
   out->edge_launches = c->kind_n[1];
   out->band_ms = c->kind_ms[2];
   out->band_launches = c->kind_n[2];
-  // the points of one stage launch (all of them), in contexts with a layer
-  // the tiles' and the inner layer's
-  out->bulk_points = c->fused || c->bulk_mode != 2 ? (int64_t)c->nx * c->ny
-                                                   : (int64_t)c->ninterior + c->nlayer_inner;
+  out->bulk_points = (int64_t)c->nx * c->ny;
   return FDM_OK;
 }
 

@@ -696,6 +696,10 @@ __device__ __forceinline__ void closure_rates(const BulkArgs<T>& a, const BlockD
   }
 }
 
+// Loads of a batch stay ahead of it, and their uses behind: without it the
+// compiler walks the terms one by one, a memory latency each.
+__device__ __forceinline__ void load_fence() { asm volatile("" ::: "memory"); }
+
 // Derivative terms of a PML block's boundary forms (rates.f90:2194-2218
 // and the like): v the fields at a one-sided neighbour or a central
 // difference, D its coefficient; the auxiliary rate dw takes sigma times
@@ -774,7 +778,7 @@ __device__ __forceinline__ void pml_rates(const BulkArgs<T>& a, BlockRef& B, con
   }
   const T sx = (T)sxd, sy = (T)syd, kap = (T)B.pml[2];
   const T rho = (T)B.rho, G = (T)B.G, M = (T)B.M, gamma = (T)B.gamma;
-  T* __restrict__ W = a.W;
+  T* W = a.W;
   const T A = (T)a.A;
   T dwx[6], dwy[6];
 #pragma unroll
@@ -889,18 +893,21 @@ __device__ __forceinline__ void pml_rates(const BulkArgs<T>& a, BlockRef& B, con
     }
   }
   const T Bdt = (T)a.Bdt;
-  // W + Bdt*DW from the values loaded above (this lane's own point)
+  // W + Bdt*DW from the values loaded above (this lane's own point), near the
+  // edges read again: 24 registers that the closures need
+  if constexpr (!INNER) load_fence();
+  auto w_of = [&](const T (&w)[6], int l, int dir) { return INNER ? w[l] : W[(6 * dir + l) * ps + cc]; };
   if (onx) {
 #pragma unroll
     for (int l = 0; l < 6; l++) {
-      if (a.do_update) __builtin_nontemporal_store(wx[l] + Bdt * dwx[l], &W[l * ps + cc]);
+      if (a.do_update) __builtin_nontemporal_store(w_of(wx, l, 0) + Bdt * dwx[l], &W[l * ps + cc]);
       __builtin_nontemporal_store(dwx[l], &W[(12 + l) * ps + cc]);
     }
   }
   if (ony) {
 #pragma unroll
     for (int l = 0; l < 6; l++) {
-      if (a.do_update) __builtin_nontemporal_store(wy[l] + Bdt * dwy[l], &W[(6 + l) * ps + cc]);
+      if (a.do_update) __builtin_nontemporal_store(w_of(wy, l, 1) + Bdt * dwy[l], &W[(6 + l) * ps + cc]);
       __builtin_nontemporal_store(dwy[l], &W[(18 + l) * ps + cc]);
     }
   }
@@ -1367,10 +1374,6 @@ struct BandTerms {
   bool corner;
 };
 
-// Loads of a batch stay ahead of it, and their uses behind: without it the
-// compiler walks the terms one by one, a memory latency each.
-__device__ __forceinline__ void load_fence() { asm volatile("" ::: "memory"); }
-
 // the products of field l at a neighbour, p1 = (y metric) F(UA), p2 = (x
 // metric) F(UB): plane strain multiplies one of them by gamma (Fld),
 // antiplane shear has both for vz, the first alone for sxz and the second
@@ -1710,6 +1713,28 @@ __device__ __forceinline__ const P& memory_args(const void* p) {
   return *(const P*)(ConstP*)u;
 }
 
+// the values of a group's edge nodes into LDS, a node a lane and a quarter of
+// the rows a wave
+template <typename T, int NF>
+__device__ __forceinline__ void stage_nodes(const EdgeArgs<T>& e, const EdgeNode& nd, const bool active, double* s,
+                                            const int stride, const int wave) {
+  if (!active) return;
+  const bool itf = nd.iface >= 0;
+  if (wave == 0) {
+    stage_rows<T, kRowFm, NF>(e, nd, s, stride);
+    if (itf) stage_rows<T, kRowFp, NF>(e, nd, s, stride);
+  } else if (wave == 1) {
+    stage_rows<T, kRowF0m, NF>(e, nd, s, stride);
+    if (itf) stage_rows<T, kRowF0p, NF>(e, nd, s, stride);
+  } else if (wave == 2) {
+    stage_rows<T, kRowN, 5>(e, nd, s, stride);
+    if (itf) stage_rows<T, kRowRs, 7>(e, nd, s, stride);
+  } else if (wave == 3 && itf) {
+    stage_rows<T, kRowMp, 3>(e, nd, s, stride);
+    stage_rows<T, kRowS0, 3 + kNodeStRows>(e, nd, s, stride);
+  }
+}
+
 // A rim group (see above).  First all four waves stage the values of its
 // edge nodes in LDS, a node a lane and a quarter of the rows a wave, so that
 // the node's whole input is in flight at once whatever registers the tiles
@@ -1728,23 +1753,7 @@ __device__ __forceinline__ void rim_group(const void* pa, const void* pe, const 
   const int first = max(wave - 1, 0) * L::wave;
   const int grp = lane / L::per, l = min(lane - L::per * grp, L::per - 1);
   const RimPt rp = e.rimpts[wb * kRimPts + max(min(first + min(grp, L::wave - 1), g.y - 1), 0)];
-  if (lane < g.x) {
-    double* s = sN + lane;
-    const bool itf = nd.iface >= 0;
-    if (wave == 0) {
-      stage_rows<T, kRowFm, NF>(e, nd, s, stride);
-      if (itf) stage_rows<T, kRowFp, NF>(e, nd, s, stride);
-    } else if (wave == 1) {
-      stage_rows<T, kRowF0m, NF>(e, nd, s, stride);
-      if (itf) stage_rows<T, kRowF0p, NF>(e, nd, s, stride);
-    } else if (wave == 2) {
-      stage_rows<T, kRowN, 5>(e, nd, s, stride);
-      if (itf) stage_rows<T, kRowRs, 7>(e, nd, s, stride);
-    } else if (wave == 3 && itf) {
-      stage_rows<T, kRowMp, 3>(e, nd, s, stride);
-      stage_rows<T, kRowS0, 3 + kNodeStRows>(e, nd, s, stride);
-    }
-  }
+  stage_nodes<T, NF>(e, nd, lane < g.x, sN + lane, stride, wave);
   __syncthreads();
   auto hats = [&](FaultSolved& f) {
     const EdgeArgs<T>& en = memory_args<EdgeArgs<T>>(pe);
@@ -1933,34 +1942,60 @@ bulk_interior_batch(const BulkArgs<T>* __restrict__ tab, const EdgeArgs<T>* __re
 }
 
 
-// Band kernel: the points within the closure depth of their block's edge
-// (one-sided closures, SAT), one lane each, from a list of (i, j).
-template <typename T, bool FULL, bool EXT, int OP = 4>
-__global__ void __launch_bounds__(64) bulk_band(BulkArgs<T> a, const int2* __restrict__ pts, int npts) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= npts) return;
-  const int2 p = pts[k];
-  point_generic<T, FULL, EXT, OP>(a, p.x, p.y, block_at(a, p.x, p.y));
+// A point near a block edge in a context with a layer.  MIX: some block has no
+// layer (the plain closures' registers would be the kernel's most).
+template <typename T, int FULL, bool MIX>
+__device__ __forceinline__ void layer_edge_point(const BulkArgs<T>& a, const BandPt& p) {
+  if constexpr (MIX) {
+    point_generic<T, FULL, true, 4, true>(a, p.i, p.j, p.blk);
+  } else {
+    const BlockDev& B = a.blocks[p.blk];
+    const long long cc = (long long)p.j * a.ld + p.i;
+    T d[6];
+    scaled_rates<T>(a, cc, d);
+    pml_rates<T>(a, B, p.i, p.j, cc, d, B.pmlx != 0, B.pmly != 0);
+    T Fc[6];
+#pragma unroll
+    for (int l = 0; l < 6; l++) Fc[l] = a.Fin[l * a.ps + cc];
+    finish_point<T, FULL>(a, B, p.blk, p.i, p.j, cc, d, Fc);
+  }
 }
 
-// The points of the perfectly matched layer blocks within four points of an
-// edge of their block, one lane each.
-template <typename T, bool FULL>
-__global__ void __launch_bounds__(256) bulk_pml(BulkArgs<T> a, const int2* __restrict__ pts, int npts) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= npts) return;
-  const int2 p = pts[k];
-  const int i = p.x, j = p.y;
-  const int bi = a.blk[a.rowb[j] * a.nbx + a.colb[i]];
-  const BlockDev& B = a.blocks[bi];
-  const long long cc = (long long)j * a.ld + i;
-  T d[6];
-  scaled_rates<T>(a, cc, d);
-  pml_rates<T>(a, B, i, j, cc, d, B.pmlx != 0, B.pmly != 0);
-  T Fc[6];
+// A rim group of a context with a layer: the nodes as in rim_group, their hats
+// to the side arrays, and after the barrier the group's points from there, a
+// lane each (the layer's closures keep twelve auxiliary values a point, so its
+// points are not split by field).
+template <typename T, int FULL, bool MIX>
+__device__ __forceinline__ void layer_rim_group(const void* pa, const void* pe, const int wb, double* sN,
+                                                const int wave, const int lane) {
+  const EdgeArgs<T>& e = memory_args<EdgeArgs<T>>(pe);
+  const int4 g = e.rim[wb];
+  const int stride = g.z ? kRimIface : kRimNodes;
+  const EdgeNode nd = e.rimnodes[wb * kRimNodes + lane];
+  stage_nodes<T, 6>(e, nd, lane < g.x, sN + lane, stride, wave);
+  __syncthreads();
+  FaultSolved f;
+  const bool mine = lane < g.x && wave == (g.z && nd.iface < 0 ? 1 : 0);
+  if (mine) {
+    const EdgeArgs<T>& en = memory_args<EdgeArgs<T>>(pe);
+    double hm[6], hp[6];
+    edge_node<T, 2, true, FULL == 1>(en, nd, NodeRows{sN + lane, stride}, hm, hp, f);
 #pragma unroll
-  for (int l = 0; l < 6; l++) Fc[l] = a.Fin[l * a.ps + cc];
-  finish_point<T, FULL>(a, B, bi, i, j, cc, d, Fc);
+    for (int k = 0; k < 6; k++) en.sd.Fhat[k * en.sd.NS + nd.som] = hm[k];
+    if (nd.iface >= 0) {
+#pragma unroll
+      for (int k = 0; k < 6; k++) en.sd.Fhat[k * en.sd.NS + nd.sop] = hp[k];
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    if (mine && nd.iface >= 0)
+      edge_finish<T>(memory_args<EdgeArgs<T>>(pe), nd, NodeRows{sN + lane, stride}, f);
+    return;
+  }
+  const int k = (wave - 1) * 64 + lane;
+  if (k >= g.y) return;
+  layer_edge_point<T, FULL, MIX>(memory_args<BulkArgs<T>>(pa), e.rimpts[wb * kRimPts + k].p);
 }
 
 // The other points of the layer blocks: 64 x 4 tiles (block, i0, j0, w),
@@ -1976,9 +2011,32 @@ __global__ void __launch_bounds__(256) bulk_pml(BulkArgs<T> a, const int2* __res
 // tiles on the main stream: 184 -> 93 us a stage.
 // NTS: F and DF stored non-temporally (working set beyond the last-level
 // cache).
-template <typename T, bool FULL, bool NTS>
-__global__ void __launch_bounds__(256) bulk_layer(BulkArgs<T> a, const int4* __restrict__ tiles) {
-  const int4 td = tiles[blockIdx.x];
+//
+// Ahead of the tiles, as in the other stage launches, the rim groups and the
+// inner band points, of layer blocks and others: with an edge, a band and a layer
+// kernel on a second stream instead, that stream set the pace (93 us a stage of
+// the grid above, 80 now).  Three waves per SIMD hold the tiles; the points near
+// edges spill 148 bytes a lane.
+template <typename T, int FULL, bool NTS, bool MIX>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+bulk_layer(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
+  __shared__ __attribute__((aligned(16))) char smem[kRimBytes];
+  const int ahead = a.nrimwg + a.nibwg;
+  if ((int)blockIdx.x < ahead) {
+    const int tid = threadIdx.y * 64 + threadIdx.x;
+    int wb = blockIdx.x;
+    if (wb < a.nrimwg) {
+      const char* args = (const char*)__builtin_amdgcn_kernarg_segment_ptr();
+      layer_rim_group<T, FULL, MIX>(args, args + edge_args_at<T>(), wb, reinterpret_cast<double*>(smem),
+                               __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
+      return;
+    }
+    const int k = (wb - a.nrimwg) * 256 + tid;
+    if (k >= a.nib) return;
+    layer_edge_point<T, FULL, MIX>(a, a.ibpts[k]);
+    return;
+  }
+  const int4 td = tiles[blockIdx.x - ahead];
   if (td.x < 0) return;
   ConstBlockDev& B = *((ConstBlockDev*)a.blocks + td.x);
   const int i = td.y + threadIdx.x, j = td.z + threadIdx.y;
@@ -1992,7 +2050,7 @@ __global__ void __launch_bounds__(256) bulk_layer(BulkArgs<T> a, const int4* __r
   scaled_rates<T>(a, cc, d);
   pml_rates<T, true>(a, B, i, j, cc, d, B.pmlx != 0 && (w & 1), B.pmly != 0 && (w & 2));
   if constexpr (FULL) {
-    finish_point<T, 1, NTS>(a, a.blocks[td.x], td.x, i, j, cc, d, Fc);
+    finish_point<T, FULL, NTS>(a, a.blocks[td.x], td.x, i, j, cc, d, Fc);
   } else {
     // as in the interior tiles, DF6 is stored only where a source adds to it
     d[5] = (a.mnu ? a.mnu[cc] : (T)B.nu) * (d[2] + d[4]);

@@ -238,10 +238,9 @@ typedef struct fdm_profile_t {
                             where the stage launch evaluates them)         */
   int64_t edge_launches;
   int64_t bulk_points;   /* grid points updated per stage by those launches */
-  double band_ms;        /* summed duration of the launches that update the
-                            points within four of a block edge, PML blocks'
-                            included (0 when the bulk launch covers every
-                            point)                                         */
+  double band_ms;        /* summed duration of launches that update the
+                            points near block edges alone (0: the bulk
+                            launches cover every point)                    */
   int64_t band_launches;
 } fdm_profile_t;
 
