@@ -35,7 +35,7 @@ HBM_PEAK_GBS = 8000.0
 # DF(6) + F(6), read 5 metric arrays; the first stage does not read DF
 # (A1 = 0).  FP64: 232 B (184 B at stage 1); FP32-bulk: half.
 BYTES_STAGE = {"fp64": (184.0, 232.0), "fp32": (92.0, 116.0)}
-# what the interior kernel itself must move, per point and stage: DF6 is
+# what the interior tiles themselves must move, per point and stage: DF6 is
 # neither read nor stored (no stage needs it); Ji is not read where the
 # kernel forms it from the metrics (ji); the metrics take 4 FP32 deltas
 # instead of 4 FP64 values where that encoding is exact (mc); the last
@@ -44,7 +44,7 @@ BYTES_STAGE = {"fp64": (184.0, 232.0), "fp32": (92.0, 116.0)}
 
 
 def kernel_min_bytes(prec, ns, ji=False, mc=False):
-    """average bytes per point of one interior launch over a step's stages"""
+    """average bytes per point of the interior tiles over a step's stages"""
     e = 8.0 if prec == "fp64" else 4.0
     read = 6 * e + (16.0 if mc else 4 * e) + (0.0 if ji else e)
     tot = 0.0
@@ -260,7 +260,7 @@ def run_c2_variant(args, tmp, het, cdiss):
                    "dt": r64["r"]["hp"].dt},
         "roofline": {
             "bound": "hbm",
-            "kernel": f"bulk_interior<double,64,4,false,true,{str(bool(het)).lower()},"
+            "kernel": f"bulk_interior<double,64,4,0,true,{str(bool(het)).lower()},"
                       f"{str(bool(cdiss)).lower()},4,{str(r64['r']['ji']).lower()},"
                       f"{str(r64['r']['mc']).lower()}>",
             "kernel_points": r64["kpts"], "achieved": r64["achieved"], "peak": HBM_PEAK_GBS,
@@ -319,7 +319,7 @@ def run_c2_sbp6(args, tmp):
         "roofline": {
             "bound": "hbm",
             # SBP6 in a uniform medium runs 64 x 8 tiles
-            "kernel": f"bulk_interior<double,64,8,false,true,false,false,6,{str(r64['r']['ji']).lower()},"
+            "kernel": f"bulk_interior<double,64,8,0,true,false,false,6,{str(r64['r']['ji']).lower()},"
                       f"{str(r64['r']['mc']).lower()}>",
             "kernel_points": r64["kpts"], "achieved": r64["achieved"], "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": r64["achieved"] / HBM_PEAK_GBS,
@@ -346,15 +346,14 @@ def run_c2_sbp6(args, tmp):
 
 def run_c2_pml(args, tmp):
     """C2 with a graded perfectly matched layer in both blocks (pmlx and
-    pmly, n = 2, from 80 % of the half-widths outwards): every point is a
-    layer point, evaluated by the band kernel's layer path.  Per point per
-    stage the layer kernel reads F (48 B), Wx, Wy (96 B), the coordinates
-    (16 B) and, after stage 1, DF (40 B) and DWx, DWy (96 B); it writes F,
-    DF (96 B), W and its rates (192 B): 448 B at stage 1 and 584 B after, in
-    FP64 (the field planes halve in FP32, the coordinates stay FP64).  The
-    dominant launch is the one over the points four or more from every
-    block edge (bulk_pml<T, FULL, true>), which the profile counts with the
-    interior launches."""
+    pmly, n = 2, from 80 % of the half-widths outwards).  Per point per stage
+    the layer kernel reads F (48 B), the coordinates (16 B) and, after stage 1,
+    DF (40 B), and writes F and DF (96 B): 160 B at stage 1 and 200 B after, in
+    FP64 (the field planes halve in FP32, the coordinates stay FP64).  A point
+    that a direction damps also reads that direction's auxiliary fields (48
+    B) and, after stage 1, their rates (48 B), and writes both (96 B): 144
+    and 192 B more.  Elsewhere they are zero and stay zero.  The launch
+    (bulk_layer) covers the whole stage."""
     from fdmap_github_amd import inputs
 
     nx, ny = args.nx, args.ny
@@ -370,9 +369,14 @@ def run_c2_pml(args, tmp):
     for prec in ("fp64",) if args.no_fp32 else ("fp64", "fp32"):
         r = run_device(inpath, prec, args.steps, args.warmup, args.prof_steps)
         ns, prof = r["nstage"], r["prof"]
-        b1, b2 = (448.0, 584.0) if prec == "fp64" else (232.0, 300.0)
+        xg, yg = (np.ctypeslib.as_array(getattr(r["hp"].ptr.contents, k),
+                                        shape=(r["hp"].ny, r["hp"].nx)) for k in ("x", "y"))
+        damped = (float(np.mean((xg < layer["mx"]) | (xg > layer["px"])))
+                  + float(np.mean((yg < layer["my"]) | (yg > layer["py"]))))
+        b1, b2 = (160.0, 200.0) if prec == "fp64" else (88.0, 108.0)
+        e = 1.0 if prec == "fp64" else 0.5
+        b1, b2 = b1 + 144.0 * e * damped, b2 + 192.0 * e * damped
         kpts = prof["bulk_points"]
-        assert kpts == 2 * (nx - 8) * (ny - 8)
         bytes_launch = kpts * (b1 + (ns - 1) * b2) / ns
         avg_ms = prof["bulk_ms"] / max(1, prof["bulk_launches"])
         res[prec] = dict(r=r, ups=r["npts"] * args.steps / r["el"], avg_ms=avg_ms, kpts=kpts,
@@ -387,7 +391,7 @@ def run_c2_pml(args, tmp):
                                f"(n 2) in both blocks, 2 blocks x ({nx}x{ny}), RFL slip law, LSRK(5,4) CFL 0.5",
                    "grid_points": r64["r"]["npts"], "fault_nodes": nx, "dt": r64["r"]["hp"].dt},
         "roofline": {
-            "bound": "hbm", "kernel": "bulk_pml<double,false,true> (layer points four or more from the block edges)",
+            "bound": "hbm", "kernel": "bulk_layer<double,0,true,false> (a whole stage of a problem with a layer)",
             "kernel_points": r64["kpts"], "achieved": r64["achieved"], "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": r64["achieved"] / HBM_PEAK_GBS,
             "traffic": measured_traffic("bulk_pml_c2pml_fp64"),
@@ -444,7 +448,7 @@ def run_m3(args, tmp):
                                "vertical RAL fault, free surface, LSRK(5,4) CFL 0.5",
                    "grid_points": r64["r"]["npts"], "fault_nodes": r64["r"]["hp"].ny},
         "roofline": {
-            "bound": "hbm", "kernel": "bulk_interior3<double,64,4,NT>",
+            "bound": "hbm", "kernel": "bulk_interior3<double,64,4,NT,4>",
             "kernel_points": r64["kpts"], "achieved": r64["achieved"], "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": r64["achieved"] / HBM_PEAK_GBS,
             "traffic": measured_traffic("bulk_interior3_m3_fp64"),
@@ -749,8 +753,8 @@ def main():
     prof = r64["prof"]
     ns = r64["nstage"]
     b1, b2 = BYTES_STAGE["fp64"]
-    # the dominant kernel updates the block interiors; its launches cover
-    # prof["bulk_points"] points each
+    # one launch a stage: edge nodes, inner band and interior tiles; it
+    # covers prof["bulk_points"] points
     kpts = prof["bulk_points"]
     bytes_launch = kpts * (b1 + (ns - 1) * b2) / ns
     avg_ms = prof["bulk_ms"] / max(1, prof["bulk_launches"])
@@ -777,10 +781,11 @@ def main():
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": f"bulk_interior<double,64,4,false,true,false,false,4,"
+            "kernel": f"bulk_interior<double,64,4,0,true,false,false,4,"
                       f"{str(r64['ji']).lower()},{str(r64['mc']).lower()}> (SBP4 interior rates + "
-                      "RK update, 64x4 LDS tiles over the block interiors, non-temporal stores "
-                      "since the 23 field, rate and metric planes exceed 256 MB; JI: Ji formed "
+                      "RK update, a whole stage: edge nodes and the points near edges ahead of "
+                      "64x4 LDS tiles over the block interiors; non-temporal stores since "
+                      "the 23 field, rate and metric planes exceed 256 MB; JI: Ji formed "
                       "from the metrics, MC: metrics read as FP32 deltas)",
             "kernel_points": kpts,
             "achieved": achieved,

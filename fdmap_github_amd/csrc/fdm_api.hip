@@ -89,7 +89,7 @@ struct fdm_ctx {
   // edge tasks
   int ntasks = 0;
   EdgeNode* nodes = nullptr;
-  // the stage launch (every context without a layer, with the tile kernels):
+  // the stage launch (every context with the tile kernels):
   // rim groups, their nodes and points, and the inner band points
   bool fused = false;
   int nrim = 0, nib = 0;
@@ -129,7 +129,7 @@ struct fdm_ctx {
   // artificial dissipation in some block: the Jacobian plane
   bool diss = false;
   void* Jp = nullptr;
-  // kinematic forcing on some interface: the edge kernels carrying it
+  // kinematic forcing on some interface: the edge nodes carrying it
   bool any_force = false;
   // perfectly matched layer: some block has it in effect (pml); Wx / Wy
   // exist when some block sets pmlx / pmly (pml_wx, pml_wy); W holds Wx,
@@ -269,7 +269,6 @@ void pack_plane(std::vector<T>& out, const double* in, int nx, int ny, int ld) {
     for (int i = 0; i < nx; i++) out[(size_t)j * ld + i] = (T)in[(size_t)j * nx + i];
 }
 
-// source time function (source.f90:212-223), evaluated on the host
 // f(k, nt) for k = 0..nt-1 on nt threads, one for every MiB of the work up to
 // 8.  A copy of fields on one thread is bound by that thread and, into fresh
 // memory, by its page faults (a snapshot of 2 x 3201x1601 points read in 10 ms
@@ -291,6 +290,7 @@ void parallel_parts(size_t bytes, const Fn& f) {
   for (auto& t : th) t.join();
 }
 
+// source time function (source.f90:212-223), evaluated on the host
 double stf_amplitude(const fdm_source& s, double t) {
   const double pi = 3.14159265358979323846264338327950288419716939937510;
   double tc = s.t_center, td = s.t_duration;
@@ -813,7 +813,7 @@ int check_fail(fdm_ctx* c) {
 
 namespace {
 
-// A block's layer in effect: all of its points go to the layer lists.
+// A block's layer in effect: all of its points go to the layer's launch.
 bool layer_block(const fdm_block& B) { return (B.pmlx || B.pmly) && !(B.Cdiss > 0.0); }
 
 // Tiles of the layer blocks' points four or more from every edge of their
@@ -878,14 +878,13 @@ bool layer_needs(const fdm_ctx* c, int dir, const double* W) {
   return false;
 }
 
-// Work lists of the edges: the tasks resolved into EdgeNode records, and for
-// contexts without a layer the rim groups and inner band points of the stage
-// launch (see the band section of fdm_bulk.hpp).  A hat and the points it
-// enters belong to one group: tasks and points are joined where a task
-// writes a side node of the point (a corner joins its two or more tasks),
-// and whole joined sets are packed, interface nodes first (the fault solve
-// is the longest chain), until a group's first wave has no lane left for a
-// node or its other waves none for a point.
+// Work lists of the edges: the tasks resolved into EdgeNode records, and the
+// rim groups and inner band points of the stage launch (see the band section
+// of fdm_bulk.hpp).  A hat and the points it enters belong to one group: tasks
+// and points are joined where a task writes a side node of the point (a corner
+// joins its two or more tasks), and whole joined sets are packed, interface
+// nodes first (the fault solve is the longest chain), until a group's first
+// wave has no lane left for a node or its other waves none for a point.
 int build_stage_lists(fdm_ctx* c) {
   std::vector<EdgeNode> nodes(c->htasks.size());
   // (block, side, node) -> edge point (i, j)
@@ -1257,8 +1256,8 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
   {
     // interior tiles: each block's rectangle [mx+nbst, px-nbst] x [my+nbst, py-nbst]
     // covered from its corner, x fastest; band: every other point, row-major.
-    // A block with a perfectly matched layer in effect has no tiles and no
-    // band: all of its points go to the layer list.
+    // A block with a perfectly matched layer in effect has tiles of its own
+    // (layer_tiles).
     std::vector<int4> tl[3];
     for (int b = 0; b < c->nb; b++) {
       const fdm_block& B = P->blocks[b];

@@ -89,7 +89,7 @@ struct BulkArgs {
   // ib_lanes, else one lane per point
   const BandPt* ibpts;
   int nib, nibwg, ib_lanes;
-  // rim groups: the first nrimwg workgroups of the stage launch (fdm_rim.hpp)
+  // rim groups: the first nrimwg workgroups of the stage launch
   int nrimwg;
   // receivers: vx, vy of Fin at the nrec points rcc into rout (FP64
   // plane-strain contexts), by nrecwg workgroups ahead of the inner band

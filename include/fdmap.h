@@ -229,10 +229,8 @@ typedef struct fdm_problem {
 
 /* Kernel timing gathered with HIP events on the context's stream. */
 typedef struct fdm_profile_t {
-  double bulk_ms;        /* summed duration of the bulk (stencil+RK) launches:
-                            whole stages, or in a problem with a PML the
-                            interior tiles and the layer points four or more
-                            from every block edge                          */
+  double bulk_ms;        /* summed duration of the bulk (stencil+RK) launches,
+                            each a whole stage                             */
   int64_t bulk_launches;
   double edge_ms;        /* summed duration of edge/interface launches (0
                             where the stage launch evaluates them)         */
