@@ -318,8 +318,7 @@ def run_c2_sbp6(args, tmp):
                    "grid_points": r64["r"]["npts"], "fault_nodes": nx, "dt": r64["r"]["hp"].dt},
         "roofline": {
             "bound": "hbm",
-            # SBP6 in a uniform medium runs 64 x 8 tiles
-            "kernel": f"bulk_interior<double,64,8,0,true,false,false,6,{str(r64['r']['ji']).lower()},"
+            "kernel": f"bulk_interior<double,64,4,0,true,false,false,6,{str(r64['r']['ji']).lower()},"
                       f"{str(r64['r']['mc']).lower()}>",
             "kernel_points": r64["kpts"], "achieved": r64["achieved"], "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": r64["achieved"] / HBM_PEAK_GBS,

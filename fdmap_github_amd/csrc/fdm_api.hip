@@ -1598,10 +1598,15 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
   // gamma, nu (5)
   c->het = P->mat_rho && P->mat_cs && P->mat_cp;
   if (c->het || c->diss || c->mode == 3 || c->sbp != 4) {
-    // SBP6 in a uniform medium: 64 x 8 unless FDM_TILE asks for 64 x 4
+    // SBP6 in a uniform medium: 64 x 4 unless FDM_TILE asks for 64 x 8.  The
+    // taller tile stages fewer halo rows, but its eight waves hold the
+    // workgroups ahead of the tiles to two a CU and their closures to four
+    // waves' registers (ms a step, FP64 / FP32-bulk, 64 x 8 and 64 x 4: 2 x
+    // 401x201 0.085 / 0.069 and 0.088 / 0.080, 2 x 801x401 0.181 / 0.119 and
+    // 0.164 / 0.113, 2 x 1601x801 0.540 / 0.294 and 0.538 / 0.295).
     const bool t8 = c->sbp == 6 && !c->het && !c->diss && c->mode == 2;
     const char* e = getenv("FDM_TILE");
-    c->tile_shape = (t8 && !(e && !strcmp(e, "64x4"))) ? 1 : 0;
+    c->tile_shape = t8 && e && !strcmp(e, "64x8") ? 1 : 0;
   }
   if (c->diss && !P->J) {
     set_err(c, FDM_EINVAL, "fdm_create: artificial dissipation needs the Jacobian J");

@@ -1892,11 +1892,15 @@ __device__ __forceinline__ void stage_ahead(const BulkArgs<T>& a, const void* pa
 // SIMD keep them in registers, and the plastic update with them (FULL = 2; the
 // last stage of 2 x 3201x1601 points, FP64: 606 us on the variant that also
 // carries manufactured solutions, two waves, normal stores and DF always
-// stored, 398 on its own).
+// stored, 398 on its own).  SBP6's closures take 198 registers ahead of the
+// tiles.  In FP64 the 64 x 4 tile's LDS leaves three waves anyway; the other
+// shapes spill them there at four waves (at three, 64 x 8 leaves one workgroup
+// a CU: 2 x 1601x801 FP64 0.669 ms a step against 0.540, FP32-bulk 0.374
+// against 0.294; 64 x 4 FP32-bulk 0.317 against 0.295).
 template <typename T, int TX, int TY, int FULL, bool NTS, bool HET, bool DISS, int OP = 4,
           bool JI = false, bool MC = false>
 __global__ void __launch_bounds__(TX * TY)
-    __attribute__((amdgpu_waves_per_eu(FULL == 1 ? 2 : ((FULL || HET || DISS || OP == 6) ? 3 : 4))))
+    __attribute__((amdgpu_waves_per_eu(FULL == 1 ? 2 : ((FULL || HET || DISS || (OP == 6 && TX * TY == 256 && sizeof(T) == 8)) ? 3 : 4))))
 bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   constexpr int kTile = tile_bytes<T, TX, TY, DISS, OP, 5>();
   __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];
