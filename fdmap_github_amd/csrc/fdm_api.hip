@@ -188,12 +188,15 @@ struct fdm_ctx {
   // equals 1/(xq yr - xr yq) everywhere; FDM_JI_CALC = 0 turns it off)
   bool ji_calc = false;
   // output streaming: a copy stream and the snapshot slots (device staging,
-  // pinned host copy, the events that end each plane's host copy)
+  // pinned host copy, the events that end each plane's host copy, and in
+  // FP32-bulk the background [block][field] that the planes deviate from:
+  // fdm_set_fields may change the context's own before the slot is read)
   hipStream_t copy = nullptr;
   struct Snapshot {
     void* dev = nullptr;
     void* host = nullptr;
     hipEvent_t staged = nullptr, done[6] = {};
+    std::vector<double> Fb;
     uint32_t mask = 0;
     bool busy = false;
   } snap[FDM_SNAPSHOT_SLOTS];
@@ -1916,6 +1919,10 @@ int fdm_snapshot(fdm_ctx* c, uint32_t field_mask, int32_t* slot) {
     HIPCHK(c, hipEventCreateWithFlags(&sn.staged, hipEventDisableTiming));
     for (int l = 0; l < c->nF; l++) HIPCHK(c, hipEventCreateWithFlags(&sn.done[l], hipEventDisableTiming));
   }
+  if (c->precision != FDM_FP64) {
+    sn.Fb.resize((size_t)c->nb * 6);
+    for (int b = 0; b < c->nb; b++) std::copy(c->hblocks[b].Fb, c->hblocks[b].Fb + 6, &sn.Fb[(size_t)b * 6]);
+  }
   // the selected planes of the current fields, packed, then to the host on
   // the copy stream while the main stream goes on
   int q = 0;
@@ -1963,7 +1970,7 @@ int fdm_snapshot_read(fdm_ctx* c, int32_t slot, double* out) {
         for (int j = j0; j < j1; j++)
           for (int i = 0; i < c->nx; i++)
             dst[(size_t)j * c->nx + i] =
-                (double)h[(size_t)j * c->ld + i] + c->hblocks[block_of(c, i, j)].Fb[field[q]];
+                (double)h[(size_t)j * c->ld + i] + sn.Fb[(size_t)block_of(c, i, j) * 6 + field[q]];
       }
     }
   });
