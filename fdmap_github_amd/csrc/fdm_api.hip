@@ -151,6 +151,7 @@ struct fdm_ctx {
   // bulk kernel: 0 per-point, 2 interior tiles (kTileShape[tile_shape]) + band points
   int bulk_mode = 2;
   int tile_shape = 0;  // index into kTileShape
+  int band_lanes = -1;  // FDM_BAND_LANES (band_lanes): 0, 1, or by rule
   // interior tiles (block, i0, j0, 0) for the tile shapes 64x4, 64x8, 128x4; band points (i, j)
   int4* tiles[3] = {nullptr, nullptr, nullptr};
   int ntiles[3] = {0, 0, 0};
@@ -486,9 +487,13 @@ int full_variant(const fdm_ctx* c, const BulkArgs<T>& a) {
 // its other workgroups); beyond that, every workgroup ahead of the tiles
 // holds a tile's place: 2 x 801x401 FP64 26.0 against 28.0 us a stage, 2 x
 // 1601x801 99.7 against 96.5 (FP32-bulk 50.6 against 47.6).
-// FDM_BAND_LANES = 0|1 overrides.
-inline int band_lanes(int nib, int others, int nt, int mode) {
-  if (const char* e = getenv("FDM_BAND_LANES")) return atoi(e) != 0;
+// forced: 0 or 1 where FDM_BAND_LANES was set at the creation, else -1.
+inline int band_lanes_env() {
+  const char* e = getenv("FDM_BAND_LANES");
+  return e ? atoi(e) != 0 : -1;
+}
+inline int band_lanes(int nib, int others, int nt, int mode, int forced) {
+  if (forced >= 0) return forced;
   const int per = (mode == 3 ? BandLanes<3>::wave : BandLanes<2>::wave) * (nt / 64);
   return (nib + per - 1) / per + others <= 3 * 1024 * 256 / nt;
 }
@@ -507,7 +512,7 @@ void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const Edg
   if (!c->pml) {
     a.nrimwg = c->nrim;
     a.nrecwg = (a.nrec + nt - 1) / nt;
-    a.ib_lanes = band_lanes(c->nib, c->nrim + c->ntiles[q], nt, c->mode);
+    a.ib_lanes = band_lanes(c->nib, c->nrim + c->ntiles[q], nt, c->mode, c->band_lanes);
     a.nibwg = band_wgs(c->nib, nt, c->mode, a.ib_lanes);
   }
   dim3 grid(a.nrimwg + a.nrecwg + a.nibwg + c->ntiles[q]);
@@ -1169,6 +1174,7 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     }
   }
   if (const char* e = getenv("FDM_XCD_SWIZZLE")) c->xcd_swizzle = atoi(e) != 0;
+  c->band_lanes = band_lanes_env();
   (void)hipGetDevice(&c->device);
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     delete c;
@@ -2349,7 +2355,7 @@ int ens_lists(fdm_ensemble* e) {
     nib += c->nib;
     others += c->nrim + c->ntiles[c->tile_shape];
   }
-  e->ib_lanes = band_lanes(nib, others, 256, 2);
+  e->ib_lanes = band_lanes(nib, others, 256, 2, band_lanes_env());
   for (int k = 0; k < M; k++)
     for (int w = 0; w < e->m[k]->nrim; w++) ah[e->m[k]->tile_shape].push_back(make_int2(k, w));
   for (int k = 0; k < M; k++) {
