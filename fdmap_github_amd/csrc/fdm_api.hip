@@ -16,7 +16,6 @@
 #include <string>
 #include <thread>
 #include <type_traits>
-#include <unordered_map>
 #include <vector>
 
 #include "fdm_stage.hpp"
@@ -265,14 +264,6 @@ int dupload(fdm_ctx* c, P** p, const void* host, size_t bytes) {
 
 int side_len(const fdm_block& b, int s) { return s < 2 ? (b.py - b.my + 1) : (b.px - b.mx + 1); }
 
-// copy a [ny][nx] double plane into a padded [ny][ld] plane of type T
-template <typename T>
-void pack_plane(std::vector<T>& out, const double* in, int nx, int ny, int ld) {
-  out.assign((size_t)ld * ny, (T)0);
-  for (int j = 0; j < ny; j++)
-    for (int i = 0; i < nx; i++) out[(size_t)j * ld + i] = (T)in[(size_t)j * nx + i];
-}
-
 // f(k, nt) for k = 0..nt-1 on nt threads, one for every MiB of the work up to
 // 8.  A copy of fields on one thread is bound by that thread and, into fresh
 // memory, by its page faults (a snapshot of 2 x 3201x1601 points read in 10 ms
@@ -292,6 +283,28 @@ void parallel_parts(size_t bytes, const Fn& f) {
   }
   f(0, nt);
   for (auto& t : th) t.join();
+}
+
+// n planes [ny][nx] of doubles into padded device planes of type T, through one
+// buffer (fresh pages cost a plane's copy as much again)
+template <typename T>
+int upload_planes(fdm_ctx* c, int n, const double* const* in, void* const* out) {
+  const size_t ne = (size_t)c->ld * c->ny;
+  std::unique_ptr<T[]> h(new (std::nothrow) T[ne]);
+  if (!h) return set_err(c, FDM_ENOMEM, "fdm_create: out of host memory");
+  for (int q = 0; q < n; q++) {
+    parallel_parts(ne * sizeof(T), [&](int k, int nt) {
+      const int j1 = (int)((long long)c->ny * (k + 1) / nt);
+      for (int j = (int)((long long)c->ny * k / nt); j < j1; j++) {
+        T* d = &h[(size_t)j * c->ld];
+        const double* f = in[q] + (size_t)j * c->nx;
+        for (int i = 0; i < c->nx; i++) d[i] = (T)f[i];
+        std::fill(d + c->nx, d + c->ld, (T)0);
+      }
+    });
+    HIPCHK(c, hipMemcpy(out[q], h.get(), ne * sizeof(T), hipMemcpyHostToDevice));
+  }
+  return FDM_OK;
 }
 
 // source time function (source.f90:212-223), evaluated on the host
@@ -902,19 +915,13 @@ int build_stage_lists(fdm_ctx* c) {
                  : make_int2(B.mx + k, s == FDM_SIDE_B ? B.my : B.py);
   };
   auto cc = [&](int2 p) { return (unsigned)((long long)p.y * c->ld + p.x); };
-  struct Writes {
-    int n, blk[2], side[2], k[2];
-  };
-  std::vector<Writes> wr(c->htasks.size());
   for (size_t t = 0; t < c->htasks.size(); t++) {
     const int2 T = c->htasks[t];
     EdgeNode& N = nodes[t];
-    Writes& W = wr[t];
     if (T.x >= 0) {
       const int b = T.x >> 2, s = T.x & 3;
       const BlockDev& B = c->hblocks[b];
       N = EdgeNode{-1, -1, cc(at(b, s, T.y)), 0u, B.side_off[s] + T.y, B.side_bc[s], b, B.id};
-      W = Writes{1, {b, 0}, {s, 0}, {T.y, 0}};
     } else {
       const IfaceDev& I = c->hifaces[-T.x - 1];
       const BlockDev& Bm = c->hblocks[I.bm];
@@ -924,7 +931,6 @@ int build_stage_lists(fdm_ctx* c) {
       const int km = g - (x ? Bm.my : Bm.mx), kp = g - (x ? Bp.my : Bp.mx);
       N = EdgeNode{-T.x - 1, I.node_off + T.y, cc(at(I.bm, sm, km)), cc(at(I.bp, sp, kp)),
                    Bm.side_off[sm] + km, Bp.side_off[sp] + kp, I.bm, I.bp};
-      W = Writes{2, {I.bm, I.bp}, {sm, sp}, {km, kp}};
     }
   }
   int rc;
@@ -941,7 +947,8 @@ int build_stage_lists(fdm_ctx* c) {
   // edge points, their side nodes, and the set each belongs to
   std::vector<BandPt> ib;
   std::vector<RimPt> ep;
-  std::unordered_map<long long, int> id;
+  std::vector<int> pt_at(c->NS, -1);  // side node -> edge point
+  ib.reserve(c->hband.size());
   for (const int2& p : c->hband) {
     const BandPt b = band_pt(p);
     const BlockDev& B = c->hblocks[b.blk];
@@ -954,7 +961,7 @@ int build_stage_lists(fdm_ctx* c) {
       ib.push_back(b);
       continue;
     }
-    id[(long long)p.y * c->nx + p.x] = (int)ep.size();
+    for (int k = 0; k < n; k++) pt_at[so[k]] = (int)ep.size();
     ep.push_back(RimPt{b, so[0], -1, n > 1 ? so[1] : -1, -1});
   }
   const int nt = (int)nodes.size(), np = (int)ep.size();
@@ -965,15 +972,29 @@ int build_stage_lists(fdm_ctx* c) {
     return k;
   };
   std::vector<std::array<int, 2>> pt_of(nt, {-1, -1});
-  for (int t = 0; t < nt; t++)
-    for (int w = 0; w < wr[t].n; w++) {
-      const int2 p = at(wr[t].blk[w], wr[t].side[w], wr[t].k[w]);
-      pt_of[t][w] = id.at((long long)p.y * c->nx + p.x);
+  for (int t = 0; t < nt; t++) {
+    const EdgeNode& N = nodes[t];
+    for (int w = 0; w < (N.iface < 0 ? 1 : 2); w++) {
+      pt_of[t][w] = pt_at[w ? N.sop : N.som];
       par[root(t)] = root(nt + pt_of[t][w]);
     }
-  std::vector<std::vector<int>> mt(nt + np), mp(nt + np);
-  for (int t = 0; t < nt; t++) mt[root(t)].push_back(t);
-  for (int k = 0; k < np; k++) mp[root(nt + k)].push_back(k);
+  }
+  // members of each set, in order: the tasks or points of set r from
+  // start[r] to start[r + 1]
+  struct Members {
+    std::vector<int> start, of;
+    const int* begin(int r) const { return of.data() + start[r]; }
+    int size(int r) const { return start[r + 1] - start[r]; }
+  };
+  auto members = [&](int first, int n) {
+    Members M{std::vector<int>(nt + np + 1, 0), std::vector<int>(n)};
+    for (int k = 0; k < n; k++) M.start[root(first + k) + 1]++;
+    for (int r = 0; r < nt + np; r++) M.start[r + 1] += M.start[r];
+    std::vector<int> at(M.start);
+    for (int k = 0; k < n; k++) M.of[at[root(first + k)]++] = k;
+    return M;
+  };
+  const Members mt = members(0, nt), mp = members(nt, np);
   std::vector<int> order;
   std::vector<char> seen(nt + np, 0);
   auto visit = [&](int r) {
@@ -991,9 +1012,6 @@ int build_stage_lists(fdm_ctx* c) {
   std::vector<RimPt> rp;
   std::vector<int> gt, gp;
   bool gi = false;
-  auto has_iface = [&](const std::vector<int>& v) {
-    return std::any_of(v.begin(), v.end(), [&](int t) { return nodes[t].iface >= 0; });
-  };
   auto flush = [&]() {
     if (gt.empty() && gp.empty()) return;
     const int stride = gi ? kRimIface : kRimNodes;
@@ -1001,7 +1019,7 @@ int build_stage_lists(fdm_ctx* c) {
     for (size_t q = 0; q < gt.size(); q++) {
       const int t = gt[q];
       rn.push_back(nodes[t]);
-      for (int w = 0; w < wr[t].n; w++) {
+      for (int w = 0; w < (nodes[t].iface < 0 ? 1 : 2); w++) {
         RimPt& P = ep[pt_of[t][w]];
         const int so = w ? nodes[t].sop : nodes[t].som;
         if (P.soA == so) P.slotA = (int)q + w * stride;
@@ -1017,18 +1035,20 @@ int build_stage_lists(fdm_ctx* c) {
     gi = false;
   };
   for (int r : order) {
-    const bool ri = has_iface(mt[r]);
-    if (mt[r].size() > (size_t)(ri ? kRimIface : kRimNodes) || mp[r].size() > (size_t)maxp) {
+    const int *t = mt.begin(r), *k = mp.begin(r);
+    const size_t st = mt.size(r), sk = mp.size(r);
+    const bool ri = std::any_of(t, t + st, [&](int q) { return nodes[q].iface >= 0; });
+    if (st > (size_t)(ri ? kRimIface : kRimNodes) || sk > (size_t)maxp) {
       // dozens of interfaces over the same nodes: the per-point kernels
       c->fused = false;
       c->bulk_mode = 0;
       return FDM_OK;
     }
     const size_t most = gi || ri ? kRimIface : kRimNodes;
-    if (gt.size() + mt[r].size() > most || gp.size() + mp[r].size() > (size_t)maxp) flush();
+    if (gt.size() + st > most || gp.size() + sk > (size_t)maxp) flush();
     gi = gi || ri;
-    gt.insert(gt.end(), mt[r].begin(), mt[r].end());
-    gp.insert(gp.end(), mp[r].begin(), mp[r].end());
+    gt.insert(gt.end(), t, t + st);
+    gp.insert(gp.end(), k, k + sk);
   }
   flush();
   c->nrim = (int)groups.size();
@@ -1289,10 +1309,14 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     }
     std::vector<int2> band;
     for (int j = 0; j < P->ny; j++)
-      for (int i = 0; i < P->nx; i++) {
-        const fdm_block& B = P->blocks[block_of(c, i, j)];
-        const bool edge = i - B.mx < nbst || B.px - i < nbst || j - B.my < nbst || B.py - j < nbst;
-        if (edge) band.push_back(make_int2(i, j));
+      for (int bx = 0; bx < c->nbx; bx++) {
+        const fdm_block& B = P->blocks[blk[(size_t)rowb[j] * c->nbx + bx]];
+        const bool row = j - B.my < nbst || B.py - j < nbst;
+        for (int i = B.mx; i <= B.px; i++) {
+          // between the strips at its sides
+          if (!row && i == B.mx + nbst) i = std::max(i, B.px - nbst + 1);
+          band.push_back(make_int2(i, j));
+        }
       }
     if (c->mode == 2 && (rc = layer_tiles(c, P))) return fail(rc);
     for (int q = 0; q < 3; q++) {
@@ -1631,6 +1655,9 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
   HIPCHK(c, hipMemset(arena, 0, nplanes * pbytes + slack));
   char* ab = (char*)arena + (size_t)c->coff * c->esz;
   c->nt_store = nt_store_choice((double)nplanes * (double)pbytes);
+  auto upload = [&](int n, const double* const* in, void* const* out) {
+    return c->precision == FDM_FP64 ? upload_planes<double>(c, n, in, out) : upload_planes<float>(c, n, in, out);
+  };
   if (c->het) {
     // init_medium (material.f90:254-262), in FP64, then the field precision
     const size_t np = (size_t)c->nx * c->ny;
@@ -1645,47 +1672,23 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
       m[4][q] = 0.5 * (m[2][q] - 2.0 * m[1][q]) / (m[2][q] - m[1][q]);
     }
     c->hnu = m[4];
+    const double* mp[5];
     for (int k = 0; k < 5; k++) {
       c->mat[k] = ab + (size_t)(pmat + k) * pbytes;
-      if (c->precision == FDM_FP64) {
-        std::vector<double> h;
-        pack_plane(h, m[k].data(), c->nx, c->ny, c->ld);
-        HIPCHK(c, hipMemcpy(c->mat[k], h.data(), h.size() * 8, hipMemcpyHostToDevice));
-      } else {
-        std::vector<float> h;
-        pack_plane(h, m[k].data(), c->nx, c->ny, c->ld);
-        HIPCHK(c, hipMemcpy(c->mat[k], h.data(), h.size() * 4, hipMemcpyHostToDevice));
-      }
+      mp[k] = m[k].data();
     }
+    if ((rc = upload(5, mp, c->mat))) return fail(rc);
   }
   if (c->diss) {
     c->Jp = ab + (size_t)pJ * pbytes;
-    if (c->precision == FDM_FP64) {
-      std::vector<double> h;
-      pack_plane(h, P->J, c->nx, c->ny, c->ld);
-      HIPCHK(c, hipMemcpy(c->Jp, h.data(), h.size() * 8, hipMemcpyHostToDevice));
-    } else {
-      std::vector<float> h;
-      pack_plane(h, P->J, c->nx, c->ny, c->ld);
-      HIPCHK(c, hipMemcpy(c->Jp, h.data(), h.size() * 4, hipMemcpyHostToDevice));
-    }
+    if ((rc = upload(1, &P->J, &c->Jp))) return fail(rc);
   }
   c->F[0] = ab;
   c->F[1] = ab + (size_t)nF * pbytes;
   c->DF = ab + (size_t)(2 * nF) * pbytes;
   for (int q = 0; q < 5; q++) c->met[q] = ab + (size_t)(pmet + q) * pbytes;
   const double* mets[5] = {P->xq, P->xr, P->yq, P->yr, P->Ji};
-  for (int q = 0; q < 5; q++) {
-    if (c->precision == FDM_FP64) {
-      std::vector<double> h;
-      pack_plane(h, mets[q], c->nx, c->ny, c->ld);
-      HIPCHK(c, hipMemcpy(c->met[q], h.data(), h.size() * 8, hipMemcpyHostToDevice));
-    } else {
-      std::vector<float> h;
-      pack_plane(h, mets[q], c->nx, c->ny, c->ld);
-      HIPCHK(c, hipMemcpy(c->met[q], h.data(), h.size() * 4, hipMemcpyHostToDevice));
-    }
-  }
+  if ((rc = upload(5, mets, c->met))) return fail(rc);
   {
     // In FP64 the interior kernel may form Ji itself when the given Ji is
     // 1/(xq yr - xr yq) to the bit (grid.f90:531-534) at every point: the
@@ -1725,24 +1728,33 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
       for (int q = 0; q < 4; q++) D.mbase[q] = mets[q][(size_t)j0 * c->nx + i0];
     }
     const float qnan = std::numeric_limits<float>::quiet_NaN();
-    std::vector<float> h[4];
+    const size_t ps = (size_t)c->ps;
+    std::unique_ptr<float[]> h(new (std::nothrow) float[4 * ps]);
+    if (!h) {
+      set_err(c, FDM_ENOMEM, "fdm_create: out of host memory");
+      return fail(FDM_ENOMEM);
+    }
     std::atomic<long long> escapes{0};
-    for (int q = 0; q < 4; q++) h[q].assign((size_t)c->ps, 0.0f);
     parallel_parts((size_t)c->nx * c->ny * 32, [&](int part, int nt) {
       const int j1 = (int)((long long)c->ny * (part + 1) / nt);
       long long n = 0;
       for (int j = (int)((long long)c->ny * part / nt); j < j1; j++)
-        for (int i = 0; i < c->nx; i++) {
-          const BlockDev& D = c->hblocks[block_of(c, i, j)];
-          for (int q = 0; q < 4; q++) {
-            const double m = mets[q][(size_t)j * c->nx + i];
-            const double d = m - D.mbase[q];
-            const float f = (float)d;
-            const double back = D.mbase[q] + (double)f;
-            const bool ok = std::isfinite(d) && (double)f == d && std::memcmp(&back, &m, sizeof(double)) == 0;
-            h[q][(size_t)j * c->ld + i] = ok ? f : qnan;
-            n += ok ? 0 : 1;
+        for (int q = 0; q < 4; q++) {
+          const double* m = mets[q] + (size_t)j * c->nx;
+          float* f = &h[q * ps + (size_t)j * c->ld];
+          for (int bx = 0; bx < c->nbx; bx++) {
+            const BlockDev& D = c->hblocks[c->hblk[(size_t)c->hrowb[j] * c->nbx + bx]];
+            const double base = D.mbase[q];
+            for (int i = D.mx; i <= D.px; i++) {
+              const double d = m[i] - base;
+              const float fi = (float)d;
+              const double back = base + (double)fi;
+              const bool ok = std::isfinite(d) && (double)fi == d && std::memcmp(&back, &m[i], sizeof(double)) == 0;
+              f[i] = ok ? fi : qnan;
+              n += ok ? 0 : 1;
+            }
           }
+          std::fill(f + c->nx, j + 1 < c->ny ? f + c->ld : &h[0] + (q + 1) * ps, 0.0f);
         }
       escapes += n;
     });
@@ -1754,10 +1766,8 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
       const size_t fbytes = (size_t)c->ps * 4;
       if ((rc = dalloc(c, &mb, 4 * fbytes + (size_t)c->coff * 4 + 256))) return fail(rc);
       char* fb = (char*)mb + (size_t)c->coff * 4;
-      for (int q = 0; q < 4; q++) {
-        c->mfp[q] = (float*)(fb + q * fbytes);
-        HIPCHK(c, hipMemcpy(c->mfp[q], h[q].data(), fbytes, hipMemcpyHostToDevice));
-      }
+      for (int q = 0; q < 4; q++) c->mfp[q] = (float*)(fb + q * fbytes);
+      HIPCHK(c, hipMemcpy(fb, h.get(), 4 * fbytes, hipMemcpyHostToDevice));
       HIPCHK(c, hipMemcpy(c->blocks, c->hblocks.data(), c->hblocks.size() * sizeof(BlockDev),
                           hipMemcpyHostToDevice));
       c->mcomp = true;
