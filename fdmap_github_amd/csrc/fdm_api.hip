@@ -1841,8 +1841,10 @@ int fdm_set_fields(fdm_ctx* c, const double* F, const double* DF) {
     for (int which = 0; which < 2; which++) {
       const double* src = which ? DF : F;
       // row r = l ny + j, its padding and (after a plane's last row) the
-      // plane's tail zero
-      parallel_parts(n * 8, [&](int k, int nt) {
+      // plane's tail zero.  On several threads from 24 MiB: below, their start
+      // and their page faults cost more (18 MiB 2.00 ms against 1.91 on one, 8
+      // MiB 1.07 against 0.82; 32 MiB 3.2 to 4.5 against 4.1 to 7.2)
+      parallel_parts(n * 8 < (24u << 20) ? 0 : n * 8, [&](int k, int nt) {
         const int nr = c->nF * c->ny, r1 = (int)((long long)nr * (k + 1) / nt);
         for (int r = (int)((long long)nr * k / nt); r < r1; r++) {
           const int l = r / c->ny, j = r - l * c->ny;
