@@ -697,31 +697,37 @@ int stage1_impl(fdm_ctx* c, double t0, double dt) {
   return run_stage<T>(c, 1, t0, dt, 1, 1);
 }
 
-// whether a point source's footprint holds point (i, j) of block b
-bool source_at(const fdm_ctx* c, int b, int i, int j) {
-  for (int p = 0; p < c->src.nplace; p++) {
-    const fdm_source_place& S = c->src.place[p];
-    if (S.block == b && std::abs(i - S.i0) <= 2 && std::abs(j - S.j0) <= 2) return true;
-  }
-  return false;
-}
-
 // DF6 = nu (DF3 + DF5) at the interior points of every block, in the
 // precision of the bulk fields: the value the lean interior kernel computes
-// and does not store (rates.f90:920-936)
+// and does not store (rates.f90:920-936), but for the points that a source
+// reaches, which their tiles store
 template <typename T>
 void restore_df6(const fdm_ctx* c, T* h) {
   const size_t pe = (size_t)c->ps;
-  for (int b = 0; b < c->nb; b++) {
-    const BlockDev& B = c->hblocks[b];
-    for (int j = B.my + c->nbst; j <= B.py - c->nbst; j++)
-      for (int i = B.mx + c->nbst; i <= B.px - c->nbst; i++) {
-        const size_t k = (size_t)j * c->ld + i;
-        if (source_at(c, b, i, j)) continue;  // stored by its tile
-        const T nu = c->het ? (T)c->hnu[(size_t)j * c->nx + i] : (T)B.nu;
-        h[5 * pe + k] = nu * (h[2 * pe + k] + h[4 * pe + k]);
+  std::vector<std::pair<size_t, T>> stored;
+  for (int p = 0; p < c->src.nplace; p++) {
+    const fdm_source_place& S = c->src.place[p];
+    const BlockDev& B = c->hblocks[S.block];
+    for (int j = std::max(S.j0 - 2, B.my); j <= std::min(S.j0 + 2, B.py); j++)
+      for (int i = std::max(S.i0 - 2, B.mx); i <= std::min(S.i0 + 2, B.px); i++) {
+        const size_t k = 5 * pe + (size_t)j * c->ld + i;
+        stored.push_back({k, h[k]});
       }
   }
+  for (int b = 0; b < c->nb; b++) {
+    const BlockDev& B = c->hblocks[b];
+    const int ja = B.my + c->nbst, n = B.py - c->nbst + 1 - ja;
+    if (n <= 0) continue;
+    parallel_parts((size_t)n * (B.px - B.mx) * 3 * sizeof(T), [&](int part, int nt) {
+      for (int j = ja + (int)((long long)n * part / nt); j < ja + (int)((long long)n * (part + 1) / nt); j++)
+        for (int i = B.mx + c->nbst; i <= B.px - c->nbst; i++) {
+          const size_t k = (size_t)j * c->ld + i;
+          const T nu = c->het ? (T)c->hnu[(size_t)j * c->nx + i] : (T)B.nu;
+          h[5 * pe + k] = nu * (h[2 * pe + k] + h[4 * pe + k]);
+        }
+    });
+  }
+  for (const auto& s : stored) h[s.first] = s.second;
 }
 
 // one step of a member context inside a graph capture: advance the device
