@@ -110,9 +110,9 @@ struct fdm_ctx {
   bool prof = false;
   std::vector<EventPair> pool;
   size_t pool_used = 0;
-  // kinds: 0 interior (or per-point) bulk, 1 edge, 2 band
-  double kind_ms[3] = {0.0, 0.0, 0.0};
-  long long kind_n[3] = {0, 0, 0};
+  // kinds: 0 stage (or per-point bulk), 1 edge
+  double kind_ms[2] = {0.0, 0.0};
+  long long kind_n[2] = {0, 0};
   std::vector<int> pair_kind;
   std::string err;
   std::vector<void*> allocs;
@@ -532,7 +532,6 @@ void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const Edg
   dim3 grid(a.nrimwg + a.nrecwg + a.nibwg + c->ntiles[q]);
   dim3 block(kTileShape[q][0], kTileShape[q][1]);
   if (!grid.x) return;
-  EventPair* ep = prof_begin(c, 0, s);
   const int full = full_variant(c, a);
   c->df6_stale = !full && c->mode == 2;
   // (shapes: fdm_create and fdm_tune keep 64 x 4 for antiplane shear, SBP2, a
@@ -560,7 +559,6 @@ void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const Edg
   else if (q == 0) stage2<T, 4, false, false, 0>(L, a, e);
   else if (q == 1) stage2<T, 4, false, false, 1>(L, a, e);
   else stage2<T, 4, false, false, 2>(L, a, e);
-  prof_end(c, ep, 0, s);
 }
 
 // contexts with a layer: the rim groups and inner band points of all blocks,
@@ -572,7 +570,6 @@ void launch_layer(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const EdgeAr
   a.nibwg = (c->nib + 255) / 256;
   const int full = full_variant(c, a);
   c->df6_stale = !full;
-  EventPair* ep = prof_begin(c, 0, s);
   dim3 grid(a.nrimwg + a.nibwg + c->nltiles), block(64, 4);
   auto go = [&](auto mix) {
     constexpr bool MIX = decltype(mix)::value;
@@ -585,7 +582,6 @@ void launch_layer(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const EdgeAr
   const bool mixed = std::any_of(c->hblocks.begin(), c->hblocks.end(), [](const BlockDev& B) { return !(B.pmlx | B.pmly); });
   if (mixed) go(std::true_type{});
   else go(std::false_type{});
-  prof_end(c, ep, 0, s);
 }
 
 template <typename T>
@@ -658,8 +654,12 @@ int run_stage(fdm_ctx* c, int stage, double t0, double dt, int final_step, int s
     } else if (rec_now) {
       record_receivers(c, c->stream, c->cur_n - 1);
     }
+    // one pair of events for the stage, also where it takes two launches (a
+    // layer in some of the blocks)
+    EventPair* ep = prof_begin(c, 0, c->stream);
     launch_interior<T>(c, c->stream, a, e);
     if (c->pml) launch_layer<T>(c, c->stream, a, e);
+    prof_end(c, ep, 0, c->stream);
   } else {
     rc = launch_edges<T>(c, c->stream, e);
     if (rc) return rc;
@@ -2177,7 +2177,7 @@ int fdm_profile_enable(fdm_ctx* c, int32_t enable) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->prof = enable != 0;
   c->pool_used = 0;
-  for (int k = 0; k < 3; k++) {
+  for (int k = 0; k < 2; k++) {
     c->kind_ms[k] = 0.0;
     c->kind_n[k] = 0;
   }
@@ -2197,8 +2197,8 @@ int fdm_profile_read(fdm_ctx* c, fdm_profile_t* out) {
   out->bulk_launches = c->kind_n[0];
   out->edge_ms = c->kind_ms[1];
   out->edge_launches = c->kind_n[1];
-  out->band_ms = c->kind_ms[2];
-  out->band_launches = c->kind_n[2];
+  out->band_ms = 0.0;
+  out->band_launches = 0;
   out->bulk_points = (int64_t)c->nx * c->ny;
   return FDM_OK;
 }

@@ -229,17 +229,17 @@ typedef struct fdm_problem {
 
 /* Kernel timing gathered with HIP events on the context's stream. */
 typedef struct fdm_profile_t {
-  double bulk_ms;        /* summed duration of the bulk (stencil+RK) launches,
-                            each a whole stage                             */
-  int64_t bulk_launches;
+  double bulk_ms;        /* summed duration of the bulk (stencil+RK) work     */
+  int64_t bulk_launches; /* the stages in bulk_ms: a launch each, or two,
+                            counted together, where some of the blocks have a
+                            perfectly matched layer                        */
   double edge_ms;        /* summed duration of edge/interface launches (0
                             where the stage launch evaluates them)         */
   int64_t edge_launches;
-  int64_t bulk_points;   /* grid points updated per stage by those launches */
-  double band_ms;        /* summed duration of launches that update the
-                            points near block edges alone (0: the bulk
-                            launches cover every point)                    */
-  int64_t band_launches;
+  int64_t bulk_points;   /* grid points updated per stage: all of them       */
+  double band_ms;        /* 0: no launch updates the points near block edges
+                            alone                                          */
+  int64_t band_launches; /* 0                                                */
 } fdm_profile_t;
 
 typedef struct fdm_ctx fdm_ctx;
