@@ -161,10 +161,6 @@ struct fdm_ctx {
   // the latest interior launch was a lean one, which leaves DF6 unwritten at
   // interior points
   bool df6_stale = false;
-  // graph capture (ensembles): stage times come from the device step counter
-  long long* nstep_dev = nullptr;
-  bool graph_mode = false;
-  double g_tinit = 0.0, g_dt = 0.0, g_rkc = 0.0;
   // adjoint forward passes: fault trajectories ([nstage][3][NI] per step,
   // step n at trace + (n - trace_n0) nstage 3 NI), the slot of the stage
   // being launched, and vx, vy at receivers after every step (step n at
@@ -388,10 +384,8 @@ EdgeArgs<T> edge_args(fdm_ctx* c, double t, double Bdt, double A, int do_scale, 
   a.fi = IfacesDev{c->ifaces, c->inhat, c->irs, c->isw, c->iS0b, c->iN0b, c->ildS, c->ildN,
                    c->iout, c->iknx, c->ist, c->ist1, c->NI};
   a.t = t;
-  a.nstep = c->graph_mode ? c->nstep_dev : nullptr;
-  a.t_init = c->g_tinit;
-  a.dt = c->g_dt;
-  a.rkc = c->g_rkc;
+  a.nstep = nullptr;  // ensembles set these four
+  a.t_init = a.dt = a.rkc = 0.0;
   a.Bdt = Bdt;
   a.A = A;
   a.Bload = Bload;
@@ -400,7 +394,6 @@ EdgeArgs<T> edge_args(fdm_ctx* c, double t, double Bdt, double A, int do_scale, 
   a.snapshot = snapshot;
   a.fail = c->fail;
   a.trace = c->trace_cur;
-  a.mode = c->mode;
   return a;
 }
 
@@ -471,7 +464,6 @@ BulkArgs<T> bulk_args(fdm_ctx* c, double A, double Bdt, int do_update, double t,
   a.mnu = (const T*)c->mat[4];
   a.J = (const T*)c->Jp;
   a.W = (T*)c->W;
-  a.ji_calc = c->ji_calc ? 1 : 0;
   a.skip_df = 0;
   a.fxq = c->mfp[0];
   a.fxr = c->mfp[1];
@@ -536,7 +528,7 @@ void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const Edg
   c->df6_stale = !full && c->mode == 2;
   // (shapes: fdm_create and fdm_tune keep 64 x 4 for antiplane shear, SBP2, a
   // heterogeneous medium and dissipation; SBP6 in a uniform medium runs 64 x
-  // 8 by default or 64 x 4)
+  // 4 by default or 64 x 8)
   const StageLaunch L{s, grid, block, c->tiles[q], q, full, c->nt_store, c->ji_calc, c->mcomp};
   if (c->mode == 3) {
     if (c->sbp == 2 && c->het) stage3<T, 2, true, false>(L, a, e);
@@ -630,7 +622,6 @@ int run_stage(fdm_ctx* c, int stage, double t0, double dt, int final_step, int s
   double t = t0 + c->rkC[stage - 1] * dt;  // D%t during this stage (time_step.f90:137)
   double Bload = c->ld_T.empty() ? 1.0 : load_ramp(t, c->ld_T[0]);
   double srcA = c->src.nplace ? stf_amplitude(c->src, t) : 0.0;
-  c->g_rkc = c->rkC[stage - 1];
   int last = (stage == c->nstage);
   BulkArgs<T> a =
       bulk_args<T>(c, A, Bdt, final_step ? 0 : 1, t, srcA, (!final_step && last) ? 1 : 0, dt);

@@ -69,13 +69,8 @@ struct BulkArgs {
   // PML auxiliary fields: Wx (planes 0-5), Wy (6-11), DWx (12-17), DWy
   // (18-23), plane stride ps (null without a layer)
   T* W;
-  // ji_calc: the context's Ji equals 1/(xq yr - xr yq) bit for bit at every
-  // point, so the interior tiles may form it from the staged metrics instead
-  // of reading the Ji plane (the host then launches their JI variant);
-  // skip_df leaves DF1..5 unstored (the last stage of a step that another
-  // step of the same call follows: the next stage scales DF by A = 0 and
-  // never reads it)
-  int ji_calc;
+  // leaves DF1..5 unstored (the last stage of a step that another step of the
+  // same call follows: the next stage scales DF by A = 0 and never reads it)
   int skip_df;
   // FP32 deltas of xq, xr, yq, yr from their block's mbase (FP64 contexts
   // whose metrics allow it; read by the interior tiles' MC variant only)
@@ -123,7 +118,7 @@ __device__ __forceinline__ void tile_of(int swz, int& tx, int& ty) {
 // workgroups dispatched to XCD x (ids congruent to x mod 8) take a
 // contiguous range of the tile list.
 __device__ __forceinline__ int linear_tile(int swz, int off = 0) {
-  // off: workgroups ahead of the tiles (the interior launch's inner band)
+  // off: workgroups ahead of the tiles
   const int bid = blockIdx.x - off;
   if (!swz) return bid;
   const int nwg = gridDim.x - off;
@@ -1069,9 +1064,9 @@ typedef const __attribute__((address_space(4))) BlockDev ConstBlockDev;
 // xq/yq with the r halo go to LDS; the lane's own DF, F6 and Ji stay in
 // registers.  Halo indices are clamped into the grid; a clamped value never
 // reaches an active lane.  tiles[k] = (block, i0, j0, a point source reaches it).
-// JI: form Ji from the staged metrics (a context with ji_calc set) rather
-// than read it; a compile-time switch, so that neither path holds the other's
-// registers.  MC: read xq, xr, yq, yr as FP32 deltas from their block's base
+// JI: form Ji from the staged metrics (a context whose Ji equals 1/(xq yr - xr
+// yq) bit for bit at every point) rather than read it; a compile-time switch,
+// so that neither path holds the other's registers.  MC: read xq, xr, yq, yr as FP32 deltas from their block's base
 // (FP64 only; the values staged in LDS are the FP64 metrics to the bit).
 // LDS bytes of an interior tile with NF staged fields, and of a launch whose
 // rim workgroups use the same buffer for their hats

@@ -132,8 +132,6 @@ struct EdgeArgs {
   // when set, [3][NI]: slip velocity, state variable at the start of the
   // stage and normal stress of every frictional node (adjoint trajectories)
   double* trace;
-  // 2: plane strain; 3: antiplane shear (fields vz, sxz, syz)
-  int mode;
 };
 
 template <typename T>
@@ -546,8 +544,7 @@ __device__ __forceinline__ void edge_finish(const EdgeArgs<T>& a, const EdgeNode
   if (I.coupling != FDM_COUPLING_LOCKED) fault_update<T>(a, I, nd.q, src, f, stage_time(a));
 }
 
-// the hats to the side arrays, where the band kernels of a launch of their
-// own read them
+// the hats to the side arrays, where the per-point kernels read them
 template <typename T, int MODE, bool FORCE>
 __device__ __forceinline__ void edge_store(const EdgeArgs<T>& a, const EdgeNode& nd) {
   constexpr int NF = MODE == 3 ? 3 : 6;

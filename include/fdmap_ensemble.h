@@ -19,18 +19,19 @@ extern "C" {
 /* launch knobs of one context */
 #define FDM_TUNE_TILE 0    /* interior tile shape: 0 = 64x4, 1 = 64x8, 2 = 128x4
                               (SBP4 in a uniform medium without dissipation;
-                              SBP6 there: 0 or 1, default 1; else 0 only) */
+                              SBP6 there: 0 or 1; else 0 only); default 0 */
 #define FDM_TUNE_SWIZZLE 1 /* XCD-contiguous tile order: 0 or 1 */
 #define FDM_TUNE_NT_STORE 2 /* non-temporal stores of the interior kernel: 0 or 1
                                (default: 1 when the 23 field, rate and metric
                                planes exceed 256 MB) */
 #define FDM_TUNE_METRIC_F32 3 /* interior tiles read the metrics as FP32 deltas
-                                 from a per-block base (FP64 plane-strain
-                                 contexts, 64x4 and 64x8 tiles): 0 or 1.  fdm_create turns it
+                                 from a per-block base (FP64 contexts, 64x4
+                                 and 64x8 tiles): 0 or 1.  fdm_create turns it
                                  on where the encoding is exact for all but
                                  1/64 of the metric values (those are read
-                                 from the FP64 planes); value 1 fails where
-                                 it did not. */
+                                 from the FP64 planes) and, in antiplane shear,
+                                 Ji equals 1/(xq yr - xr yq) to the bit; value
+                                 1 fails where it did not. */
 
 /* Set a launch knob of ctx.  Results do not depend on it.  Set knobs
    before putting ctx into an ensemble (its graphs keep the shapes they were
@@ -40,9 +41,8 @@ int fdm_tune(fdm_ctx* ctx, int32_t knob, int32_t value);
 typedef struct fdm_ensemble fdm_ensemble;
 
 /* Group n contexts (each an independent problem with its own storage) so
-   that they advance together: every RK stage of all members is one interior
-   launch per tile shape in use, one edge launch and one band launch over
-   the members' merged work lists, and every step is one hipGraph launch,
+   that they advance together: every RK stage of all members is one launch
+   per tile shape in use over the members' merged work lists, and every step is one hipGraph launch,
    captured on first use.  Members must have no point source, no
    manufactured solution and no load ramp, use the tile kernels, and share
    the precision, RK order and device; at each step they must share the
