@@ -529,7 +529,7 @@ void launch_interior(fdm_ctx* c, hipStream_t s, const BulkArgs<T>& a0, const Edg
   // (shapes: fdm_create and fdm_tune keep 64 x 4 for antiplane shear, SBP2, a
   // heterogeneous medium and dissipation; SBP6 in a uniform medium runs 64 x
   // 4 by default or 64 x 8)
-  const StageLaunch L{s, grid, block, c->tiles[q], q, full, c->nt_store, c->ji_calc, c->mcomp};
+  const StageLaunch L{s, grid, block, c->tiles[q], q, full, c->nt_store, c->ji_calc, c->mcomp, grid.x > kManyWgs};
   if (c->mode == 3) {
     if (c->sbp == 2 && c->het) stage3<T, 2, true, false>(L, a, e);
     else if (c->sbp == 2) stage3<T, 2, false, false>(L, a, e);
@@ -2331,7 +2331,7 @@ int ens_step_launches(fdm_ensemble* e, int p) {
     for (int q = 0; q < 3; q++) {
       const dim3 grid(e->nahead[q] + e->ntiles[q]), block(kTileShape[q][0], kTileShape[q][1]);
       if (grid.x)
-        stage_batch<T>(StageLaunch{e->master, grid, block, e->tiles[q], q, full, e->nt_store, false, false}, bt, et,
+        stage_batch<T>(StageLaunch{e->master, grid, block, e->tiles[q], q, full, e->nt_store, false, false, false}, bt, et,
                        e->ahead[q], e->nahead[q], e->swz);
     }
   }

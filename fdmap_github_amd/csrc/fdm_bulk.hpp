@@ -1882,20 +1882,23 @@ __device__ __forceinline__ void stage_ahead(const BulkArgs<T>& a, const void* pa
 // on two streams joined by events twice a stage, us a stage: 151^2 with a
 // point source 25.8 -> 10.4, 401^2 28.5 -> 13.5, 2 x 333x167 with a fault
 // 32.3 -> 15.4, 2 x 801x401 42.6 -> 26.1, 2 x 1601x801 106 -> 88.8 (FP32-bulk
-// 58.1 -> 47.6).  A heterogeneous medium holds five
-// more values per lane, dissipation the Jacobian's staging: three waves per
-// SIMD keep them in registers, and the plastic update with them (FULL = 2; the
-// last stage of 2 x 3201x1601 points, FP64: 606 us on the variant that also
-// carries manufactured solutions, two waves, normal stores and DF always
-// stored, 398 on its own).  SBP6's closures take 198 registers ahead of the
-// tiles.  In FP64 the 64 x 4 tile's LDS leaves three waves anyway; the other
-// shapes spill them there at four waves (at three, 64 x 8 leaves one workgroup
-// a CU: 2 x 1601x801 FP64 0.669 ms a step against 0.540, FP32-bulk 0.374
-// against 0.294; 64 x 4 FP32-bulk 0.317 against 0.295).
+// 58.1 -> 47.6).
+//
+// Waves per SIMD: the points ahead of the tiles take the most registers, and
+// what a cap spills is mostly theirs (scratch bytes a lane, FULL = 0: FP64 SBP4
+// 100, a medium or dissipation 100, SBP6 108 and 392 at 64 x 8; FP32 28, SBP6 80,
+// a medium or dissipation none at three waves and 52 at four).  Three where the
+// tile holds more (a medium's five values, the Jacobian's staging, the plastic
+// update: the last stage of 2 x 3201x1601 points, FP64, 398 us, 606 on the
+// variant that also carries manufactured solutions, two waves, normal stores
+// and DF always stored), MANY: four there (kManyWgs); three for SBP6's FP64 64
+// x 4 tile, whose LDS leaves three anyway; else four.  SBP6's 64 x 8 tile at
+// three leaves one workgroup a CU: 2 x 1601x801 FP64 0.669 ms a step against
+// 0.540, FP32-bulk 0.374 against 0.294; 64 x 4 FP32-bulk 0.317 against 0.295.
 template <typename T, int TX, int TY, int FULL, bool NTS, bool HET, bool DISS, int OP = 4,
-          bool JI = false, bool MC = false>
-__global__ void __launch_bounds__(TX * TY)
-    __attribute__((amdgpu_waves_per_eu(FULL == 1 ? 2 : ((FULL || HET || DISS || (OP == 6 && TX * TY == 256 && sizeof(T) == 8)) ? 3 : 4))))
+          bool JI = false, bool MC = false, bool MANY = false>
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(
+    FULL == 1 ? 2 : (!MANY && (FULL || HET || DISS || (OP == 6 && TX * TY == 256 && sizeof(T) == 8)) ? 3 : 4))))
 bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   constexpr int kTile = tile_bytes<T, TX, TY, DISS, OP, 5>();
   __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];

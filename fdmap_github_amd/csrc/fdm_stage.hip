@@ -10,6 +10,17 @@ namespace {
 
 template <typename T, int TX, int TY, int OP, bool HET, bool DISS, bool JI, bool MC>
 void stage2_v(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e) {
+  if constexpr (std::is_same<T, float>::value && (HET || DISS)) {
+    if (!L.full && L.many) {
+      if (L.nt_store)
+        hipLaunchKernelGGL((bulk_interior<T, TX, TY, 0, true, HET, DISS, OP, JI, MC, true>), L.grid, L.block, 0,
+                           L.stream, a, e, L.tiles);
+      else
+        hipLaunchKernelGGL((bulk_interior<T, TX, TY, 0, false, HET, DISS, OP, JI, MC, true>), L.grid, L.block, 0,
+                           L.stream, a, e, L.tiles);
+      return;
+    }
+  }
   if (L.full == 1)
     hipLaunchKernelGGL((bulk_interior<T, TX, TY, 1, false, HET, DISS, OP, JI, MC>), L.grid, L.block, 0, L.stream, a, e,
                        L.tiles);

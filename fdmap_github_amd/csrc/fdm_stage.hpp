@@ -11,6 +11,16 @@ namespace fdm {
 // interior tile shapes (columns x rows) selectable with FDM_TILE
 constexpr int kTileShape[3][2] = {{64, 4}, {64, 8}, {128, 4}};
 
+// From this many workgroups on (of 256 threads: six rounds of those that four
+// waves per SIMD hold) the FP32 variants for a medium or dissipation run four
+// waves instead of three: a longer launch gains more from the tiles' waves than
+// it loses by what the points ahead of them spill.  ms a step at three and at
+// four: 2 x 401x201 (730 workgroups) 0.066 and 0.070 with dissipation, 0.063 and
+// 0.070 in a medium, 2 x 1201x601 (5913) 0.190 and 0.195, 0.177 and 0.178; 2 x
+// 1301x651 (7015) 0.208 and 0.198, 0.200 and 0.194, 2 x 2201x1101 0.640 and
+// 0.580 (0.590 in three launches a stage), 0.640 and 0.608.
+constexpr unsigned kManyWgs = 6 * 1024;
+
 struct StageLaunch {
   hipStream_t stream;
   dim3 grid, block;
@@ -18,6 +28,7 @@ struct StageLaunch {
   int shape;
   int full;  // FULL of the kernels
   bool nt_store, ji_calc, mcomp;
+  bool many;  // more than kManyWgs workgroups
 };
 
 // plane strain: FULL = 1 (manufactured solutions, plasticity), 2 (plasticity)
