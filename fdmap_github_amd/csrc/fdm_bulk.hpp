@@ -2378,10 +2378,13 @@ __global__ void __launch_bounds__(256) bulk_kernel3(BulkArgs<T> a) {
 // halo of F; a block without it keeps the plain expression.  JI, MC: as in the
 // plane-strain tile.  2 x 701x1401 points, FP64 SBP6, us a stage: 52.0 with
 // Ji and the metrics read as FP64, DF stored every stage and the loads under
-// their lane conditions, 49.5 now.
+// their lane conditions, 49.5 with all three mended.  Four waves per SIMD, in FP64
+// with dissipation three (150 registers); in FP32 dissipation takes 130, and at
+// three waves 2 x 2201x1101 took 0.456 ms a step against 0.393, 2 x 801x401 0.078
+// against 0.073.
 template <typename T, int TX, int TY, bool NTS, int OP = 4, bool HET = false, bool DISS = false, bool JI = false,
           bool MC = false>
-__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(DISS ? 3 : 4)))
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(DISS && sizeof(T) == 8 ? 3 : 4)))
 bulk_interior3(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
   static_assert(!DISS || OP == 4, "artificial dissipation is built for SBP4 only");
   constexpr int H = Sbp<OP>::half, NB = Sbp<OP>::nbst;
