@@ -2226,15 +2226,19 @@ int fdm_tune(fdm_ctx* c, int32_t knob, int32_t value) {
 
 // An ensemble steps many contexts with batched launches: every RK stage is
 // one launch per tile shape in use over the merged work lists of all
-// members.  The per-member kernel arguments of each
+// members, or, where many workgroups would go ahead of the tiles
+// (ens_ahead_most), that of the tiles beside one of the edge nodes and one of the points near
+// edges on a second stream.  The per-member kernel arguments of each
 // (buffer parity, stage) sit in device tables; stage times come from one
 // device step counter.  A step is captured once per starting buffer parity
 // as a hipGraph (FDM_ENSEMBLE_GRAPH=0 launches the same kernels directly).
 struct fdm_ensemble {
   std::vector<fdm_ctx*> m;
   int precision = FDM_FP64, nstage = 0, flip = 0, swz = 1, ib_lanes = 0;
-  bool any_plastic = false, mms_side = false, use_graph = true, nt_store = false;
-  hipStream_t master = nullptr;
+  bool any_plastic = false, mms_side = false, use_graph = true, nt_store = false, split = false;
+  hipStream_t master = nullptr, side = nullptr;
+  // split: the fork, the latest tiles and the latest band
+  hipEvent_t evJ = nullptr, evI = nullptr, evB = nullptr;
   hipEvent_t done = nullptr;
   std::vector<hipEvent_t> pre;  // each member's earlier work, before a step
   // merged lists per tile shape in use: tiles (block, i0, j0, member), and
@@ -2244,6 +2248,10 @@ struct fdm_ensemble {
   int ntiles[3] = {0, 0, 0};
   int2* ahead[3] = {nullptr, nullptr, nullptr};
   int nahead[3] = {0, 0, 0};
+  // split: a wave each of the edge nodes and the points near edges
+  int2* ewaves = nullptr;
+  int4* band = nullptr;
+  int newaves = 0, nbwaves = 0;
   void* btab = nullptr;  // BulkArgs<T>[2][nstage][members]
   void* etab = nullptr;  // EdgeArgs<T>[2][nstage][members]
   long long* nstep = nullptr;
@@ -2319,22 +2327,40 @@ int ens_tables(fdm_ensemble* e) {
 }
 
 // One RK step of every member from buffer parity p: a stage launch per tile
-// shape in use, then the step counter.
+// shape in use, then the step counter.  Split: tiles need only the previous
+// stage's band (halo values, and the buffer that they overwrite is the one that
+// band read); the edge nodes need the previous band (same stream), the band
+// also the previous tiles.
 template <typename T>
 int ens_step_launches(fdm_ensemble* e, int p) {
   const size_t M = e->m.size(), ns = e->nstage;
+  if (e->split) {
+    ENSCHK(e, hipEventRecord(e->evJ, e->master));
+    ENSCHK(e, hipStreamWaitEvent(e->side, e->evJ, 0));
+    ENSCHK(e, hipEventRecord(e->evB, e->side));
+    ENSCHK(e, hipEventRecord(e->evI, e->master));
+  }
   for (size_t s = 1; s <= ns; s++) {
     const size_t o = ((size_t)p * ns + (s - 1)) * M;
     const BulkArgs<T>* bt = (const BulkArgs<T>*)e->btab + o;
     const EdgeArgs<T>* et = (const EdgeArgs<T>*)e->etab + o;
     const int full = e->mms_side ? 1 : (e->any_plastic && s == ns ? 2 : 0);
+    if (e->split) ENSCHK(e, hipStreamWaitEvent(e->master, e->evB, 0));
     for (int q = 0; q < 3; q++) {
       const dim3 grid(e->nahead[q] + e->ntiles[q]), block(kTileShape[q][0], kTileShape[q][1]);
       if (grid.x)
         stage_batch<T>(StageLaunch{e->master, grid, block, e->tiles[q], q, full, e->nt_store, false, false, false}, bt, et,
                        e->ahead[q], e->nahead[q], e->swz);
     }
+    if (!e->split) continue;
+    hipLaunchKernelGGL((edge_kernel_batch<T>), dim3(e->newaves), dim3(64), 0, e->side, et, e->ewaves);
+    ENSCHK(e, hipStreamWaitEvent(e->side, e->evI, 0));
+    if (full) hipLaunchKernelGGL((bulk_band_batch<T, 2>), dim3(e->nbwaves), dim3(64), 0, e->side, bt, e->band);
+    else hipLaunchKernelGGL((bulk_band_batch<T, 0>), dim3(e->nbwaves), dim3(64), 0, e->side, bt, e->band);
+    ENSCHK(e, hipEventRecord(e->evB, e->side));
+    ENSCHK(e, hipEventRecord(e->evI, e->master));
   }
+  if (e->split) ENSCHK(e, hipStreamWaitEvent(e->master, e->evB, 0));
   hipLaunchKernelGGL(step_counter_kernel, dim3(1), dim3(64), 0, e->master, e->nstep);
   ENSCHK(e, hipGetLastError());
   return FDM_OK;
@@ -2360,6 +2386,16 @@ int ens_capture(fdm_ensemble* e, int p) {
   return FDM_OK;
 }
 
+// The most workgroups ahead of the tiles of one stage launch, by precision.
+// They are bound by latency and hold the tiles' places meanwhile, and a launch of
+// many problems has them in proportion.  ms a step with all in one launch and
+// split, members of 2 x 401x201: FP64 10 (960 workgroups ahead) 0.51 and 0.54, 12
+// (1152) 0.60 and 0.61, 14 (1344) 0.71 and 0.70, 48 (4608) 2.54 and 2.12; FP32-bulk
+// 18 (1728) 0.54 and 0.55, 24 (2304) 0.70 and 0.70, 28 (2688) 0.83 and 0.81, 48 1.49
+// and 1.31.  Sixteen of 401..2001 x 201..1001 points: 6.35 and 5.67, 3.38 and 3.13.
+// FDM_ENSEMBLE_SPLIT = 0|1 overrides.
+inline size_t ens_ahead_most(int precision) { return precision == FDM_FP64 ? 1280 : 2048; }
+
 // merged work lists of all members
 int ens_lists(fdm_ensemble* e) {
   const int M = (int)e->m.size();
@@ -2379,14 +2415,32 @@ int ens_lists(fdm_ensemble* e) {
     for (int w = 0; w < band_wgs(c->nib, nt, 2, e->ib_lanes); w++) ah[q].push_back(make_int2(k, c->nrim + w));
     for (const int4& t : c->htiles[q]) tl[q].push_back(make_int4(t.x, t.y, t.z, k));
   }
+  e->split = ah[0].size() + ah[1].size() + ah[2].size() > ens_ahead_most(e->precision);
+  if (const char* v = getenv("FDM_ENSEMBLE_SPLIT")) e->split = atoi(v) != 0;
   for (int q = 0; q < 3; q++) {
     e->ntiles[q] = (int)tl[q].size();
     if (e->ntiles[q] && ens_upload(e, &e->tiles[q], tl[q].data(), tl[q].size() * sizeof(int4)))
       return FDM_EDEVICE;
-    e->nahead[q] = (int)ah[q].size();
+    e->nahead[q] = e->split ? 0 : (int)ah[q].size();
     if (e->nahead[q] && ens_upload(e, &e->ahead[q], ah[q].data(), ah[q].size() * sizeof(int2)))
       return FDM_EDEVICE;
   }
+  if (!e->split) return FDM_OK;
+  std::vector<int2> ew;
+  std::vector<int4> band;
+  for (int k = 0; k < M; k++) {
+    const fdm_ctx* c = e->m[k];
+    for (int n = 0; n < c->ntasks; n += 64) ew.push_back(make_int2(k, n));
+    for (const int2& p : c->hband) band.push_back(make_int4(p.x, p.y, block_of(c, p.x, p.y), k));
+    while (band.size() % 64) band.push_back(make_int4(0, 0, -1, k));
+  }
+  e->newaves = (int)ew.size();
+  e->nbwaves = (int)(band.size() / 64);
+  if (ens_upload(e, &e->ewaves, ew.data(), ew.size() * sizeof(int2)) ||
+      ens_upload(e, &e->band, band.data(), band.size() * sizeof(int4)))
+    return FDM_EDEVICE;
+  ENSCHK(e, hipStreamCreateWithFlags(&e->side, hipStreamNonBlocking));
+  for (hipEvent_t* ev : {&e->evJ, &e->evI, &e->evB}) ENSCHK(e, hipEventCreateWithFlags(ev, hipEventDisableTiming));
   return FDM_OK;
 }
 
@@ -2399,12 +2453,15 @@ const char* fdm_ensemble_last_error(const fdm_ensemble* e) { return e ? e->err.c
 void fdm_ensemble_destroy(fdm_ensemble* e) {
   if (!e) return;
   if (e->master) (void)hipStreamSynchronize(e->master);
+  if (e->side) (void)hipStreamSynchronize(e->side);
   for (int q = 0; q < 2; q++)
     if (e->exec[q]) (void)hipGraphExecDestroy(e->exec[q]);
   for (hipEvent_t ev : e->pre)
     if (ev) (void)hipEventDestroy(ev);
-  if (e->done) (void)hipEventDestroy(e->done);
+  for (hipEvent_t ev : {e->evJ, e->evI, e->evB, e->done})
+    if (ev) (void)hipEventDestroy(ev);
   for (void* p : e->allocs) (void)hipFree(p);
+  if (e->side) (void)hipStreamDestroy(e->side);
   if (e->master) (void)hipStreamDestroy(e->master);
   delete e;
 }

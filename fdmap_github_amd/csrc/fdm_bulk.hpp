@@ -1087,8 +1087,10 @@ constexpr int kRimRowsMax =
 constexpr int kRimHats = 2 * kRimIface > kRimNodes ? 2 * kRimIface : kRimNodes;
 constexpr int kRimBytes = (kRimRowsMax + 6 * kRimHats) * (int)sizeof(double);
 
+// OWN: LDS arrays of its own, where the kernel holds nothing but tiles (FP64:
+// 126 registers, against 128 and two in scratch out of a shared buffer).
 template <typename T, int TX, int TY, int FULL, bool NTS, bool HET, bool DISS, int OP = 4,
-          bool JI = false, bool MC = false>
+          bool JI = false, bool MC = false, bool OWN = false>
 __device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 td, char* smem) {
   // H: the operator's interior half-width, the tile's halo; NB: the
   // closure's depth, how far the interior rectangle stays from block edges
@@ -1099,11 +1101,23 @@ __device__ __forceinline__ void interior_tile(const BulkArgs<T>& a, const int4 t
   constexpr int NF = (HY * HX + NT - 1) / NT;  // staging passes, F1..F5
   constexpr int NR = (TY * HX + NT - 1) / NT;  // xr, yr
   constexpr int NQ = (HY * TX + NT - 1) / NT;  // xq, yq
-  T (*sF)[HY][HX] = reinterpret_cast<T (*)[HY][HX]>(smem);
-  T (*sR)[TY][HX] = reinterpret_cast<T (*)[TY][HX]>(smem + 5 * HY * HX * sizeof(T));
-  T (*sQ)[HY][TX] = reinterpret_cast<T (*)[HY][TX]>(smem + (5 * HY + 2 * TY) * HX * sizeof(T));
+  T (*sF)[HY][HX];
+  T (*sR)[TY][HX];
+  T (*sQ)[HY][TX];
   // the Jacobian with the same halo as F, for artificial dissipation
-  T (*sJ)[HX] = reinterpret_cast<T (*)[HX]>(smem + ((5 * HY + 2 * TY) * HX + 2 * HY * TX) * sizeof(T));
+  T (*sJ)[HX] = nullptr;
+  if constexpr (OWN) {
+    static_assert(!DISS, "arrays of its own");
+    __shared__ T oF[5][HY][HX], oR[2][TY][HX], oQ[2][HY][TX];
+    sF = oF;
+    sR = oR;
+    sQ = oQ;
+  } else {
+    sF = reinterpret_cast<T (*)[HY][HX]>(smem);
+    sR = reinterpret_cast<T (*)[TY][HX]>(smem + 5 * HY * HX * sizeof(T));
+    sQ = reinterpret_cast<T (*)[HY][TX]>(smem + (5 * HY + 2 * TY) * HX * sizeof(T));
+    sJ = reinterpret_cast<T (*)[HX]>(smem + ((5 * HY + 2 * TY) * HX + 2 * HY * TX) * sizeof(T));
+  }
   const int bu = td.x, i0 = td.y, j0 = td.z;
   ConstBlockDev* B4 = (ConstBlockDev*)a.blocks + bu;
   const int tid = threadIdx.y * TX + threadIdx.x;
@@ -1928,21 +1942,50 @@ bulk_interior(BulkArgs<T> a, EdgeArgs<T> e, const int4* __restrict__ tiles) {
 // Batched stage launch: the rim groups, inner band points and tiles of many
 // problems.  ahead[k] = (problem, its workgroup index) of the nahead
 // workgroups ahead of the tiles; tile .w selects the problem's arguments.
-template <typename T, int TX, int TY, int FULL, bool NTS>
+// AHEAD = false: the tiles alone, beside edge_kernel_batch and
+// bulk_band_batch (whose registers the tiles then do without: FP64 126, no
+// scratch, against 132 bytes a lane).
+template <typename T, int TX, int TY, int FULL, bool NTS, bool AHEAD>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(FULL == 1 ? 2 : (FULL ? 3 : 4))))
 bulk_interior_batch(const BulkArgs<T>* __restrict__ tab, const EdgeArgs<T>* __restrict__ etab,
                     const int2* __restrict__ ahead, int nahead, const int4* __restrict__ tiles, int swz) {
-  constexpr int kTile = tile_bytes<T, TX, TY, false, 4, 5>();
-  __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];
-  if ((int)blockIdx.x < nahead) {
-    const int2 w = ahead[blockIdx.x];
-    stage_ahead<T, 2, TX, TY, FULL, false, 4>(tab[w.x], tab + w.x, etab + w.x, w.y, smem);
-    return;
+  if constexpr (AHEAD) {
+    constexpr int kTile = tile_bytes<T, TX, TY, false, 4, 5>();
+    __shared__ __attribute__((aligned(16))) char smem[kTile > kRimBytes ? kTile : kRimBytes];
+    if ((int)blockIdx.x < nahead) {
+      const int2 w = ahead[blockIdx.x];
+      stage_ahead<T, 2, TX, TY, FULL, false, 4>(tab[w.x], tab + w.x, etab + w.x, w.y, smem);
+      return;
+    }
+    const int4 td = tiles[linear_tile(swz, nahead)];
+    interior_tile<T, TX, TY, FULL, NTS, false, false>(tab[td.w], td, smem);
+  } else {
+    const int4 td = tiles[linear_tile(swz)];
+    interior_tile<T, TX, TY, FULL, NTS, false, false, 4, false, false, true>(tab[td.w], td, nullptr);
   }
-  const int4 td = tiles[linear_tile(swz, nahead)];
-  interior_tile<T, TX, TY, FULL, NTS, false, false>(tab[td.w], td, smem);
 }
 
+// The edge nodes and the points near edges of many problems in launches of
+// their own, a lane each, a wave for one problem: waves[w] = (problem, its
+// first node), and pts[k] = (i, j, block, problem), padded to whole waves with
+// block < 0.  Sixty-four points a wave, where a rim group spreads 36 over
+// three: longer for one, but half the wave time of all.
+template <typename T>
+__global__ void __launch_bounds__(64)
+edge_kernel_batch(const EdgeArgs<T>* __restrict__ etab, const int2* __restrict__ waves) {
+  const int2 w = waves[blockIdx.x];
+  const EdgeArgs<T>& e = etab[w.x];
+  const int k = w.y + (int)threadIdx.x;
+  if (k < e.ntasks) edge_store<T, 2, true>(e, e.nodes[k]);
+}
+
+template <typename T, int FULL>
+__global__ void __launch_bounds__(64)
+bulk_band_batch(const BulkArgs<T>* __restrict__ tab, const int4* __restrict__ pts) {
+  const int4 p = pts[blockIdx.x * 64 + threadIdx.x];
+  const int m = __builtin_amdgcn_readfirstlane(p.w);
+  if (p.z >= 0) point_generic<T, FULL, false, 4, false>(tab[m], p.x, p.y, p.z);
+}
 
 // A point near a block edge in a context with a layer.  MIX: some block has no
 // layer (the plain closures' registers would be the kernel's most).

@@ -91,24 +91,32 @@ void stage3(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e) {
 
 namespace {
 
-template <typename T, int TX, int TY>
+template <typename T, int TX, int TY, bool AHEAD>
 void batch_v(const StageLaunch& L, const BulkArgs<T>* bt, const EdgeArgs<T>* et, const int2* ahead, int nahead,
              int swz) {
   if (L.full == 1)
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 1, false>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
-                       L.tiles, swz);
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 1, false, AHEAD>), L.grid, L.block, 0, L.stream, bt, et, ahead,
+                       nahead, L.tiles, swz);
   else if (L.full && L.nt_store)
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 2, true>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
-                       L.tiles, swz);
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 2, true, AHEAD>), L.grid, L.block, 0, L.stream, bt, et, ahead,
+                       nahead, L.tiles, swz);
   else if (L.full)
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 2, false>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
-                       L.tiles, swz);
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 2, false, AHEAD>), L.grid, L.block, 0, L.stream, bt, et, ahead,
+                       nahead, L.tiles, swz);
   else if (L.nt_store)
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 0, true>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
-                       L.tiles, swz);
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 0, true, AHEAD>), L.grid, L.block, 0, L.stream, bt, et, ahead,
+                       nahead, L.tiles, swz);
   else
-    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 0, false>), L.grid, L.block, 0, L.stream, bt, et, ahead, nahead,
-                       L.tiles, swz);
+    hipLaunchKernelGGL((bulk_interior_batch<T, TX, TY, 0, false, AHEAD>), L.grid, L.block, 0, L.stream, bt, et, ahead,
+                       nahead, L.tiles, swz);
+}
+
+template <typename T, bool AHEAD>
+void batch_s(const StageLaunch& L, const BulkArgs<T>* bt, const EdgeArgs<T>* et, const int2* ahead, int nahead,
+             int swz) {
+  if (L.shape == 0) batch_v<T, 64, 4, AHEAD>(L, bt, et, ahead, nahead, swz);
+  else if (L.shape == 1) batch_v<T, 64, 8, AHEAD>(L, bt, et, ahead, nahead, swz);
+  else batch_v<T, 128, 4, AHEAD>(L, bt, et, ahead, nahead, swz);
 }
 
 }  // namespace
@@ -116,9 +124,8 @@ void batch_v(const StageLaunch& L, const BulkArgs<T>* bt, const EdgeArgs<T>* et,
 template <typename T>
 void stage_batch(const StageLaunch& L, const BulkArgs<T>* bt, const EdgeArgs<T>* et, const int2* ahead, int nahead,
                  int swz) {
-  if (L.shape == 0) batch_v<T, 64, 4>(L, bt, et, ahead, nahead, swz);
-  else if (L.shape == 1) batch_v<T, 64, 8>(L, bt, et, ahead, nahead, swz);
-  else batch_v<T, 128, 4>(L, bt, et, ahead, nahead, swz);
+  if (nahead) batch_s<T, true>(L, bt, et, ahead, nahead, swz);
+  else batch_s<T, false>(L, bt, et, ahead, nahead, swz);
 }
 
 #define STAGE2(T, OP, HET, DISS, SHAPE) \

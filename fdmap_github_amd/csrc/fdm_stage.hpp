@@ -41,7 +41,8 @@ void stage2(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e);
 template <typename T, int OP, bool HET, bool DISS>
 void stage3(const StageLaunch& L, const BulkArgs<T>& a, const EdgeArgs<T>& e);
 
-// an ensemble's stage, for the members with tile shape L.shape
+// an ensemble's stage, for the members with tile shape L.shape; without
+// workgroups ahead the tiles alone
 template <typename T>
 void stage_batch(const StageLaunch& L, const BulkArgs<T>* bt, const EdgeArgs<T>* et, const int2* ahead, int nahead,
                  int swz);
