@@ -585,15 +585,20 @@ __device__ __forceinline__ void diss_central(T (&d)[6], const T* __restrict__ F,
 // dissipation term, and strips add the diagonal between their two loops
 // (rates_dissipation_boundary_mode2).  The stencil loops are unrolled so
 // that all of a point's loads are in flight together: the band is a thin
-// set of points, latency-bound.  EXT = false leaves out the heterogeneous
-// medium and dissipation code (launches of problems with neither).
-template <typename T, bool EXT, int OP = 4>
+// set of points, latency-bound.  STAGE: in a stage launch SBP6's nine in FP64
+// take turns of three; all at once took 198 registers, 30 of them in scratch (2
+// x 801x401 0.171 ms a step against 0.150, 2 x 1601x801 0.558 against 0.552; the
+// per-point kernel has them, and took 0.378 against 0.368 in turns).  EXT = false
+// leaves out the heterogeneous medium and dissipation code (launches of
+// problems with neither).
+template <typename T, bool EXT, int OP = 4, bool STAGE = false>
 __device__ __forceinline__ void closure_rates(const BulkArgs<T>& a, const BlockDev& B, const int i,
                                               const int j, const long long cc, T (&d)[6]) {
   const long long ps = a.ps;
   const int ld = a.ld;
   const T* __restrict__ F = a.Fin;
   constexpr int NB = Sbp<OP>::nbst, NS = Sbp<OP>::nbnd, HW = Sbp<OP>::half;
+  constexpr int kUnroll = STAGE && OP == 6 && sizeof(T) == 8 ? 3 : NS;
   const int dl = i - B.mx, dr = B.px - i, db = j - B.my, dtp = B.py - j;
   // SAT penalties, sides in the order L, R, B, T
   if (dl == 0 || dr == 0 || db == 0 || dtp == 0) {
@@ -626,7 +631,7 @@ __device__ __forceinline__ void closure_rates(const BulkArgs<T>& a, const BlockD
   const long long colm = (long long)B.my * ld + i, colp = (long long)B.py * ld + i;
   if (qone) {
     // one-sided q: L or R strip, or q part of a corner
-#pragma unroll
+#pragma unroll kUnroll
     for (int s = 0; s < NS; s++) {
       long long kq = (dl < NB) ? row + B.mx + s : row + B.px - s;
       T Dq = (dl < NB) ? (T)sbp_dl<OP>(dl, s) : (T)(-sbp_dl<OP>(dr, s));
@@ -665,7 +670,7 @@ __device__ __forceinline__ void closure_rates(const BulkArgs<T>& a, const BlockD
     }
   } else {
     // B or T strip: one-sided r, then central q
-#pragma unroll
+#pragma unroll kUnroll
     for (int s = 0; s < NS; s++) {
       long long kr = (db < NB) ? colm + (long long)s * ld : colp - (long long)s * ld;
       T Dr = (db < NB) ? (T)sbp_dl<OP>(db, s) : (T)(-sbp_dl<OP>(dtp, s));
@@ -931,8 +936,8 @@ __device__ __forceinline__ int block_at(const BulkArgs<T>& a, const int i, const
   return a.blk[a.rowb[j] * a.nbx + a.colb[i]];
 }
 
-// PML = false leaves the layer out (contexts without one), INNER = true the
-// closures (interior points only).
+// PML = false leaves the layer out (stage launches without one), INNER = true
+// the closures (interior points only).
 template <typename T, int FULL, bool EXT, int OP = 4, bool PML = EXT, bool INNER = false>
 __device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i, const int j, const int bi) {
   const BlockDev& B = a.blocks[bi];
@@ -972,7 +977,7 @@ __device__ __forceinline__ void point_generic(const BulkArgs<T>& a, const int i,
           d, acc, (T)B.gamma, BlockCoef<T, const BlockDev&>{B}, a.Ji[cc]);
     }
   } else if constexpr (!INNER) {
-    closure_rates<T, EXT, OP>(a, B, i, j, cc, d);
+    closure_rates<T, EXT, OP, !PML>(a, B, i, j, cc, d);
   }
   T Fc[6];
 #pragma unroll
@@ -1900,7 +1905,7 @@ __device__ __forceinline__ void stage_ahead(const BulkArgs<T>& a, const void* pa
 //
 // Waves per SIMD: the points ahead of the tiles take the most registers, and
 // what a cap spills is mostly theirs (scratch bytes a lane, FULL = 0: FP64 SBP4
-// 100, a medium or dissipation 100, SBP6 108 and 392 at 64 x 8; FP32 28, SBP6 80,
+// 100, a medium or dissipation 100, SBP6 none and 296 at 64 x 8; FP32 28, SBP6 80,
 // a medium or dissipation none at three waves and 52 at four).  Three where the
 // tile holds more (a medium's five values, the Jacobian's staging, the plastic
 // update: the last stage of 2 x 3201x1601 points, FP64, 398 us, 606 on the
