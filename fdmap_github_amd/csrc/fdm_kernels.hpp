@@ -106,8 +106,10 @@ struct EdgeNode {
 // (their staged values take the same LDS), and the stride of its points
 constexpr int kRimNodes = 64, kRimIface = 24, kRimPts = 64;
 
+// On whole lines of the scalar cache in a stage kernel's argument segment: 8
+// bytes off them, a stage of 401^2 points took 13.9 us against 13.7.
 template <typename T>
-struct EdgeArgs {
+struct alignas(64) EdgeArgs {
   const T* F;
   int ld;
   long long ps;
