@@ -262,7 +262,7 @@ def run_c2_variant(args, tmp, het, cdiss):
             "bound": "hbm",
             "kernel": f"bulk_interior<double,64,4,0,true,{str(bool(het)).lower()},"
                       f"{str(bool(cdiss)).lower()},4,{str(r64['r']['ji']).lower()},"
-                      f"{str(r64['r']['mc']).lower()}>",
+                      f"{str(r64['r']['mc']).lower()},false>",
             "kernel_points": r64["kpts"], "achieved": r64["achieved"], "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": r64["achieved"] / HBM_PEAK_GBS,
             "traffic": measured_traffic(f"bulk_interior_{name}_fp64"),
@@ -319,7 +319,7 @@ def run_c2_sbp6(args, tmp):
         "roofline": {
             "bound": "hbm",
             "kernel": f"bulk_interior<double,64,4,0,true,false,false,6,{str(r64['r']['ji']).lower()},"
-                      f"{str(r64['r']['mc']).lower()}>",
+                      f"{str(r64['r']['mc']).lower()},false>",
             "kernel_points": r64["kpts"], "achieved": r64["achieved"], "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": r64["achieved"] / HBM_PEAK_GBS,
             "traffic": measured_traffic("bulk_interior_c2sbp6_fp64"),
@@ -473,7 +473,7 @@ def run_c4(args, tmp):
     """Ensemble: scenarios with block sizes uniform in 401..2001 x 201..1001,
     lognormal fault shear prestress (mean 70 MPa, log sd 0.1, correlation
     length 1 km), uniform a in [0.008, 0.012]; FP32 fields, FP64 friction;
-    tile shapes from the autotuner; every RK stage of all scenarios is one
+    tile shapes from the autotuner; every RK stage of all scenarios is a
     batched launch per kernel kind, and a step is one hipGraph launch."""
     import collections
 
@@ -781,7 +781,7 @@ def main():
         "roofline": {
             "bound": "hbm",
             "kernel": f"bulk_interior<double,64,4,0,true,false,false,4,"
-                      f"{str(r64['ji']).lower()},{str(r64['mc']).lower()}> (SBP4 interior rates + "
+                      f"{str(r64['ji']).lower()},{str(r64['mc']).lower()},false> (SBP4 interior rates + "
                       "RK update, a whole stage: edge nodes and the points near edges ahead of "
                       "64x4 LDS tiles over the block interiors; non-temporal stores since "
                       "the 23 field, rate and metric planes exceed 256 MB; JI: Ji formed "

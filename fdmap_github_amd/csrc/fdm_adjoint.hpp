@@ -763,7 +763,7 @@ __device__ __forceinline__ void adj_rim_group(const AdjBulkArgs& a, const AdjEdg
 // a block edge (128 a workgroup), then the interior tiles, under which the
 // latency of the first two passes.  Against an edge, a band and an interior
 // kernel on two streams joined by events twice a stage, 2 x 801x401 points:
-// 43 -> 33 us a stage, 29.5 of them the kernel.  Three waves per SIMD hold the
+// 43 us a stage, 29 now, 27 of them the kernel.  Three waves per SIMD hold the
 // edge node's and the pair's registers; four spill them.
 struct AdjLists {
   const int4* rim;

@@ -489,10 +489,14 @@ int full_variant(const fdm_ctx* c, const BulkArgs<T>& a) {
 
 // Inner band points: one lane per (point, field), or one lane per point?
 // Five lanes a point finish sooner (5 us against 12) but hold five times the
-// workgroups.  They pay while the whole launch is resident at once (`others`
-// its other workgroups); beyond that, every workgroup ahead of the tiles
-// holds a tile's place: 2 x 801x401 FP64 26.0 against 28.0 us a stage, 2 x
-// 1601x801 99.7 against 96.5 (FP32-bulk 50.6 against 47.6).
+// workgroups, and every workgroup ahead of the tiles holds a tile's place.  Up
+// to 3072 workgroups of 256 threads in the whole launch (`others`: those
+// besides) field lanes are the faster at every operator and precision measured;
+// beyond, it depends.  us a stage, a lane a point / field lanes: 2 x 801x401 (3007
+// workgroups) FP64 29.5 / 26.3, FP32-bulk 21.2 / 18.3, SBP6 (3180) 33.9 / 32.8;
+// 2 x 901x451 (3595) SBP4 34.8 / 31.1, SBP6 (3830) 36.9 / 39.1; 2 x 961x493 35.0 /
+// 35.0; 2 x 1001x501 (4509) 35.2 / 37.3, FP32-bulk 24.3 / 24.7, SBP6 40.2 / 45.0; 2
+// x 1251x626 62.4 / 64.1, FP32-bulk 31.8 / 34.0.
 // forced: 0 or 1 where FDM_BAND_LANES was set at the creation, else -1.
 inline int band_lanes_env() {
   const char* e = getenv("FDM_BAND_LANES");
@@ -1632,9 +1636,11 @@ int fdm_create(const fdm_problem* P, fdm_ctx** out) {
     // SBP6 in a uniform medium: 64 x 4 unless FDM_TILE asks for 64 x 8.  The
     // taller tile stages fewer halo rows, but its eight waves hold the
     // workgroups ahead of the tiles to two a CU and their closures to four
-    // waves' registers (ms a step, FP64 / FP32-bulk, 64 x 8 and 64 x 4: 2 x
-    // 401x201 0.085 / 0.069 and 0.088 / 0.080, 2 x 801x401 0.181 / 0.119 and
-    // 0.164 / 0.113, 2 x 1601x801 0.540 / 0.294 and 0.538 / 0.295).
+    // waves' registers.  It is the faster below 2 x 601x301 or so, where a step
+    // is short, and behind by more above, so that one default serves all sizes
+    // (ms a step, 64 x 4 / 64 x 8: 2 x 401x201 FP64 0.088 / 0.085, FP32-bulk
+    // 0.081 / 0.071; 2 x 801x401 0.150 / 0.176, 0.121 / 0.136; 2 x 1601x801 0.547 /
+    // 0.540, 0.299 / 0.318; 2 x 2201x1101 1.02 / 1.02, 0.60 / 0.65).
     const bool t8 = c->sbp == 6 && !c->het && !c->diss && c->mode == 2;
     const char* e = getenv("FDM_TILE");
     c->tile_shape = t8 && e && !strcmp(e, "64x8") ? 1 : 0;

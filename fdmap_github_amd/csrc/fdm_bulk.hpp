@@ -2424,9 +2424,8 @@ __global__ void __launch_bounds__(256) bulk_kernel3(BulkArgs<T> a) {
 // barrier.  HET: a heterogeneous medium, the lane's own rho and G.  DISS:
 // artificial dissipation in some block (SBP4), the Jacobian staged with the
 // halo of F; a block without it keeps the plain expression.  JI, MC: as in the
-// plane-strain tile.  2 x 701x1401 points, FP64 SBP6, us a stage: 52.0 with
-// Ji and the metrics read as FP64, DF stored every stage and the loads under
-// their lane conditions, 49.5 with all three mended.  Four waves per SIMD, in FP64
+// plane-strain tile: 2 x 701x1401 points, FP64 SBP6, 300 steps and the
+// read-back 69.9 ms without them, 65.3 with.  Four waves per SIMD, in FP64
 // with dissipation three (150 registers); in FP32 dissipation takes 130, and at
 // three waves 2 x 2201x1101 took 0.456 ms a step against 0.393, 2 x 801x401 0.078
 // against 0.073.
