@@ -42,11 +42,12 @@ typedef struct fdm_ensemble fdm_ensemble;
 
 /* Group n contexts (each an independent problem with its own storage) so
    that they advance together: every RK stage of all members is one launch
-   per tile shape in use over the members' merged work lists, and every step is one hipGraph launch,
-   captured on first use.  Members must have no point source, no
-   manufactured solution and no load ramp, use the tile kernels, and share
-   the precision, RK order and device; at each step they must share the
-   current buffer parity.  The contexts stay owned by the caller and must
+   per tile shape in use over the members' merged work lists, in a large
+   ensemble beside two for the points near edges, and every step is one
+   hipGraph launch, captured on first use.  Members must have no point
+   source, no manufactured solution and no load ramp, use the tile kernels,
+   and share the precision, RK order and device; at each step they must share
+   the current buffer parity.  The contexts stay owned by the caller and must
    outlive the ensemble. */
 int fdm_ensemble_create(fdm_ctx* const* members, int32_t n, fdm_ensemble** out);
 
